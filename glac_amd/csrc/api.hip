@@ -44,7 +44,7 @@ struct glacx_ctx {
     long long t_launches[GLACX_K_COUNT] = {};
     double t_ms[GLACX_K_COUNT] = {};
     // learned proposal
-    float *samples = nullptr;        // column-major (A, U) pairs
+    float *samples = nullptr;        // (A, U) pairs in float4 planes
     size_t samples_cap = 0, samples_n = 0;
     float *params = nullptr;         // FP32 master parameters, then Adam m, v, gradient
     float *adam_m = nullptr, *adam_v = nullptr, *grad = nullptr;
@@ -893,29 +893,23 @@ int glacx_train(glacx_ctx *c, int steps, int batch, int draws, double lr, double
     if (!c->samples || c->samples_n == 0) return fail(c, GLACX_E_STATE, "train: no samples");
     if (steps < 0 || batch < 1 || draws < 1 || !(lr > 0.0)) return fail(c, GLACX_E_ARG, "train: bad arguments");
     int rc;
-    const int nblk = (batch + kBlock - 1) / kBlock;
-    if ((rc = ensure(c, &c->inter, &c->inter_len, (size_t)kTrainInterCols * batch))) return rc;
-    if ((rc = ensure(c, &c->partials, &c->partials_len, (size_t)nblk * steps))) return rc;
+    // per-block losses of one step, then each step's loss
+    const size_t groups = (size_t)train_groups(batch);
+    if ((rc = ensure(c, &c->inter, &c->inter_len, train_inter_floats(batch)))) return rc;
+    if ((rc = ensure(c, &c->partials, &c->partials_len, groups + steps))) return rc;
+    double *losses = c->partials + groups;
     for (int i = 0; i < steps; i++) {
         hipEvent_t e0 = nullptr;
         if ((rc = timed_begin(c, &e0))) return rc;
         c->adam_t++;
         launch_train_step(c->samples, c->samples_cap, c->samples_n, batch, draws, seed, (uint64_t)c->adam_t, beta,
-                          c->params, c->mean_std, nullptr, c->inter, c->partials + (size_t)i * nblk, c->grad,
-                          c->adam_m, c->adam_v, (float)lr, (int)c->adam_t, c->params_bf16, c->stream);
+                          c->params, c->mean_std, nullptr, c->inter, c->partials, losses + i, c->grad, c->adam_m,
+                          c->adam_v, (float)lr, (int)c->adam_t, c->params_bf16, c->stream);
         CHECK_LAUNCH(c);
         if ((rc = timed_end(c, GLACX_K_TRAIN, e0))) return rc;
     }
-    if (loss && steps > 0) {
-        std::vector<double> h((size_t)nblk * steps);
-        HIP_TRY(c, hipMemcpyAsync(h.data(), c->partials, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
-        for (int i = 0; i < steps; i++) {
-            double s = 0.0;
-            for (int b = 0; b < nblk; b++) s += h[(size_t)i * nblk + b];
-            loss[i] = s;
-        }
-    }
+    if (loss && steps > 0)
+        HIP_TRY(c, hipMemcpyAsync(loss, losses, sizeof(double) * steps, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     return GLACX_OK;
 }
@@ -926,10 +920,10 @@ int glacx_train_grad(glacx_ctx *c, const float *samples, int n, const float *z, 
     CTX_CHECK(c);
     if (!c->proposal_ready) return fail(c, GLACX_E_STATE, "train_grad: set parameters first");
     if (!samples || !z || n < 1 || draws < 1) return fail(c, GLACX_E_ARG, "train_grad: bad arguments");
-    // column-major copy of the host samples, then the draws
+    // the host samples as the device holds them (nine float4 planes), then the draws
     std::vector<float> cols((size_t)36 * n);
     for (int s = 0; s < n; s++)
-        for (int k = 0; k < 36; k++) cols[(size_t)k * n + s] = samples[(size_t)s * 36 + k];
+        for (int k = 0; k < 36; k++) cols[((size_t)(k >> 2) * n + s) * 4 + (k & 3)] = samples[(size_t)s * 36 + k];
     float *dsmp = nullptr, *dz = nullptr;
     HIP_TRY(c, hipMalloc((void **)&dsmp, cols.size() * sizeof(float)));
     const size_t nz = (size_t)n * draws * 8;
@@ -939,10 +933,10 @@ int glacx_train_grad(glacx_ctx *c, const float *samples, int n, const float *z, 
         return fail(c, GLACX_E_HIP, "train_grad: hipMalloc failed");
     }
     int rc = GLACX_OK;
-    const int nblk = (n + kBlock - 1) / kBlock;
+    const size_t groups = (size_t)train_groups(n);
     do {
-        if ((rc = ensure(c, &c->inter, &c->inter_len, (size_t)kTrainInterCols * n))) break;
-        if ((rc = ensure(c, &c->partials, &c->partials_len, (size_t)nblk))) break;
+        if ((rc = ensure(c, &c->inter, &c->inter_len, train_inter_floats(n)))) break;
+        if ((rc = ensure(c, &c->partials, &c->partials_len, groups + 1))) break;
         if (hipMemcpyAsync(dsmp, cols.data(), cols.size() * sizeof(float), hipMemcpyHostToDevice, c->stream) !=
                 hipSuccess ||
             hipMemcpyAsync(dz, z, nz * sizeof(float), hipMemcpyHostToDevice, c->stream) != hipSuccess) {
@@ -950,13 +944,13 @@ int glacx_train_grad(glacx_ctx *c, const float *samples, int n, const float *z, 
             break;
         }
         launch_train_step(dsmp, (size_t)n, (size_t)n, n, draws, 0, 0, beta, c->params, c->mean_std, dz, c->inter,
-                          c->partials, c->grad, c->adam_m, c->adam_v, 0.f, 0, c->params_bf16, c->stream);
+                          c->partials, c->partials + groups, c->grad, c->adam_m, c->adam_v, 0.f, 0, c->params_bf16, c->stream);
         if (hipGetLastError() != hipSuccess) {
             rc = fail(c, GLACX_E_HIP, "train_grad: launch failed");
             break;
         }
-        std::vector<double> h(nblk);
-        if (hipMemcpyAsync(h.data(), c->partials, nblk * sizeof(double), hipMemcpyDeviceToHost, c->stream) !=
+        double step_loss = 0.0;
+        if (hipMemcpyAsync(&step_loss, c->partials + groups, sizeof step_loss, hipMemcpyDeviceToHost, c->stream) !=
                 hipSuccess ||
             (grad && hipMemcpyAsync(grad, c->grad, sizeof(float) * kProposalParams, hipMemcpyDeviceToHost,
                                     c->stream) != hipSuccess) ||
@@ -964,9 +958,7 @@ int glacx_train_grad(glacx_ctx *c, const float *samples, int n, const float *z, 
             rc = fail(c, GLACX_E_HIP, "train_grad: readback failed");
             break;
         }
-        double s = 0.0;
-        for (double v : h) s += v;
-        if (loss) *loss = s;
+        if (loss) *loss = step_loss;
     } while (0);
     (void)hipStreamSynchronize(c->stream);
     (void)hipFree(dsmp);

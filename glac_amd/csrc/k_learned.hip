@@ -9,36 +9,52 @@
 // The second-order dS only shapes the proposal; the sampler uses the exact
 // exponential and exact dS.
 //
-// A training step is three kernels: train_kernel (one thread per sample:
-// forward, loss, per-sample back-propagation to the layer inputs, written as
-// columns), grad_kernel (one thread per parameter: the batch sum of the
-// outer products, in a fixed order) and adam_kernel.
+// A training step is two kernels: train_kernel (one wavefront per 16 samples:
+// forward, loss and back-propagation to the layer inputs, the layers on the
+// matrix cores) and update_kernel (the batch sums of the outer products on the
+// FP64 matrix cores, then Adam).  Both keep every sum in the order of a plain
+// loop: a training run amplifies a last-bit change of a gradient to per cent
+// within 200 steps.
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "learned.hpp"
 #include "proposal.hpp"
 
 namespace glacx {
 
-// Samples hold 36 columns per sample: A (18 reals) then U (18 reals).
-// Per-sample columns kept for the gradient: x, h1, h2, do, da2, da1.
+// Samples hold 36 reals: A (18) then U (18), as nine float4 planes (reals
+// 4q..4q+3 of sample s at plane q): collection writes and the moments read
+// them coalesced, and a training step's random samples touch nine cache lines
+// each instead of 36.
+//
+// Per-sample columns kept for the gradient: x, h1, h2, do, da2, da1 and a
+// column of ones (the input of the biases).
 constexpr int kColX = 0, kColH1 = kColX + kMlpIn, kColH2 = kColH1 + kMlpH1, kColDo = kColH2 + kMlpH2,
-              kColDa2 = kColDo + kMlpOut, kColDa1 = kColDa2 + kMlpH2;
-static_assert(kColDa1 + kMlpH1 == kTrainInterCols, "intermediate column count");
+              kColDa2 = kColDo + kMlpOut, kColDa1 = kColDa2 + kMlpH2, kColOne = kColDa1 + kMlpH1, kCols = kColOne + 1;
 
-template <class T> __device__ __forceinline__ M3<float> to_float(const M3<T> &m) { return convert<float>(m); }
-
-__device__ __forceinline__ M3<float> read_matrix(const float *__restrict__ s, size_t cap, int col0, size_t i)
+// reals [0, 18) (A) or [0, 36) (A and U) of sample i
+template <int N> __device__ __forceinline__ void read_sample(const float4 *__restrict__ smp, size_t cap, size_t i,
+                                                             float v[4 * N])
+{
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        const float4 t = smp[(size_t)q * cap + i];
+        v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
+    }
+}
+__device__ __forceinline__ M3<float> matrix_of(const float *v)
 {
     M3<float> m;
 #pragma unroll
-    for (int k = 0; k < 9; k++) m.e[k / 3][k % 3] = {s[(size_t)(col0 + 2 * k) * cap + i], s[(size_t)(col0 + 2 * k + 1) * cap + i]};
+    for (int k = 0; k < 9; k++) m.e[k / 3][k % 3] = {v[2 * k], v[2 * k + 1]};
     return m;
 }
 
 // ---- sample collection -----------------------------------------------------
 template <class T, int R>
 __global__ __launch_bounds__(kBlock) void collect_kernel(const typename vec2<T>::type *__restrict__ f, Geom g, int mu,
-                                                         int parity, int stride, float *__restrict__ out, size_t cap,
+                                                         int parity, int stride, float4 *__restrict__ out, size_t cap,
                                                          size_t base)
 {
     const int h = (blockIdx.x * kBlock + threadIdx.x) * stride;
@@ -49,30 +65,40 @@ __global__ __launch_bounds__(kBlock) void collect_kernel(const typename vec2<T>:
     const Site x = site_of(g, idx);
     const M3<T> a = staple<T, R>(f, g, x, mu);
     const M3<T> u = load_link<T, R>(f, g, mu, idx);
+    float v[36];
 #pragma unroll
     for (int k = 0; k < 9; k++) {
-        out[(size_t)(2 * k) * cap + s] = float(a.e[k / 3][k % 3].r);
-        out[(size_t)(2 * k + 1) * cap + s] = float(a.e[k / 3][k % 3].i);
-        out[(size_t)(18 + 2 * k) * cap + s] = float(u.e[k / 3][k % 3].r);
-        out[(size_t)(18 + 2 * k + 1) * cap + s] = float(u.e[k / 3][k % 3].i);
+        v[2 * k] = float(a.e[k / 3][k % 3].r);
+        v[2 * k + 1] = float(a.e[k / 3][k % 3].i);
+        v[18 + 2 * k] = float(u.e[k / 3][k % 3].r);
+        v[18 + 2 * k + 1] = float(u.e[k / 3][k % 3].i);
     }
+#pragma unroll
+    for (int q = 0; q < 9; q++)
+        out[(size_t)q * cap + s] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
 }
 
 // ---- feature standardisation ---------------------------------------------------
-__global__ __launch_bounds__(kBlock) void feature_moments_kernel(const float *__restrict__ smp, size_t cap, size_t n,
+// Sums of the six features and their squares: at most kMomentBlocks blocks
+// stride over the samples, so that the second kernel's sum stays short
+// whatever the sample count (one thread summing a partial per 256 samples took
+// 646 us for 262 144 samples, beside the first kernel's 12 us; now 4.7 us).
+constexpr int kMomentBlocks = 1024;
+
+__global__ __launch_bounds__(kBlock) void feature_moments_kernel(const float4 *__restrict__ smp, size_t cap, size_t n,
                                                                  double beta, double *__restrict__ partials)
 {
-    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
     double acc[12];
 #pragma unroll
     for (int k = 0; k < 12; k++) acc[k] = 0.0;
-    if (i < n) {
-        float fe[6];
-        staple_features(read_matrix(smp, cap, 0, i), beta, fe);
+    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
+        float fe[6], v[20];
+        read_sample<5>(smp, cap, i, v);
+        staple_features(matrix_of(v), beta, fe);
 #pragma unroll
         for (int k = 0; k < 6; k++) {
-            acc[k] = fe[k];
-            acc[6 + k] = (double)fe[k] * fe[k];
+            acc[k] += fe[k];
+            acc[6 + k] += (double)fe[k] * fe[k];
         }
     }
     block_sum<12>(acc);
@@ -80,209 +106,283 @@ __global__ __launch_bounds__(kBlock) void feature_moments_kernel(const float *__
         for (int k = 0; k < 12; k++) partials[(size_t)blockIdx.x * 12 + k] = acc[k];
 }
 
-__global__ void feature_moments_finish(const double *__restrict__ partials, int nblk, size_t n,
-                                       float *__restrict__ mean_std)
+// One block: thread (group, k) sums every kMomentGroups-th partial of moment
+// k, then one thread per feature adds the groups, both in a fixed order.
+constexpr int kMomentGroups = kBlock / 12;
+
+__global__ __launch_bounds__(kBlock) void feature_moments_finish(const double *__restrict__ partials, int nblk,
+                                                                 size_t n, float *__restrict__ mean_std)
 {
-    if (threadIdx.x != 0) return;
-    for (int k = 0; k < 6; k++) {
-        double s = 0.0, s2 = 0.0;
-        for (int b = 0; b < nblk; b++) {
-            s += partials[(size_t)b * 12 + k];
-            s2 += partials[(size_t)b * 12 + 6 + k];
-        }
-        const double m = s / (double)n;
-        const double var = s2 / (double)n - m * m;
-        mean_std[k] = (float)m;
-        mean_std[6 + k] = (float)(var > 1e-12 ? sqrt(var) : 1.0);
+    __shared__ double sums[kMomentGroups][12];
+    const int group = threadIdx.x / 12, m = threadIdx.x - 12 * group;
+    if (group < kMomentGroups) {
+        double s = 0.0;
+#pragma unroll 8
+        for (int b = group; b < nblk; b += kMomentGroups) s += partials[(size_t)b * 12 + m];
+        sums[group][m] = s;
     }
+    __syncthreads();
+    const int k = threadIdx.x;
+    if (k >= 6) return;
+    double s = 0.0, s2 = 0.0;
+    for (int b = 0; b < kMomentGroups; b++) {
+        s += sums[b][k];
+        s2 += sums[b][6 + k];
+    }
+    const double mean = s / (double)n;
+    const double var = s2 / (double)n - mean * mean;
+    mean_std[k] = (float)mean;
+    mean_std[6 + k] = (float)(var > 1e-12 ? sqrt(var) : 1.0);
 }
 
 // ---- training step -------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void train_kernel(const float *__restrict__ smp, size_t cap, size_t n_samples,
-                                                       int batch, int draws, uint64_t seed, uint64_t step,
-                                                       double beta, const float *__restrict__ params,
-                                                       const float *__restrict__ mean_std,
-                                                       const float *__restrict__ zin, float *__restrict__ inter,
-                                                       double *__restrict__ loss_partials)
+// One wavefront (a block of its own) trains on 16 samples.  Lane l works for
+// sample l % 16 and, in slot l / 16, on every fourth draw and a quarter of the
+// Cholesky factor's entries; the network's layers are FP32 matrix products
+// [units x inputs] [inputs x 16 samples] on v_mfma_f32_16x16x4 (weights as the
+// A operand), whose columns pass through LDS from layer to layer.  The matrix
+// instruction adds its four products one after the other with one rounding
+// each (checked on random and denormal operands), so a layer rounds exactly as
+// a loop of fused multiply-adds over its inputs.
+//
+// What bounds it: latency.  The default batch of 4096 is 256 wavefronts, one
+// per CU, each a chain sample -> features -> layers -> draws -> backward.
+// One thread per sample with all layers in its registers (64 wavefronts) took
+// 39 us a step at batch 4096 with 4 draws, 16 us now; four wavefronts per
+// 64 samples with the weights in scalar registers 55 us (they spill).
+constexpr int kTrainSites = 16;
+constexpr int kColStride = 20;  // words per column in LDS: a tile's results go to 64 different banks
+
+struct TrainLds {
+    float col[kCols][kColStride];     // the gradient's columns
+    float dz[4][16][kTrainSites];     // per slot: d loss / d w (8) and z (8) of its draw
+};
+
+// Row and column of the Cholesky factor behind output e (eight diagonal
+// entries, then the rows below them): the two indices packed as 16 a + b.
+__device__ constexpr unsigned char kCholIndex[kMlpOut] = {
+    0x00, 0x11, 0x22, 0x33, 0x44, 0x55, 0x66, 0x77, 0x10, 0x20, 0x21, 0x30, 0x31, 0x32, 0x40, 0x41, 0x42, 0x43,
+    0x50, 0x51, 0x52, 0x53, 0x54, 0x60, 0x61, 0x62, 0x63, 0x64, 0x65, 0x70, 0x71, 0x72, 0x73, 0x74, 0x75, 0x76};
+
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c)
 {
-    __shared__ float P[kNParam];
-    for (int k = threadIdx.x; k < kNParam; k += kBlock) P[k] = params[k];
-    __syncthreads();
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    double lacc[1] = {0.0};
-    if (i < batch) {
-        size_t s;
-        if (zin) {
-            s = (size_t)i;
-        } else {
-            uint32_t c[4] = {(uint32_t)i, (uint32_t)(step >> 32), (uint32_t)step, 0x7E57u};
-            philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
-            s = (size_t)((((uint64_t)c[0] << 32) | c[1]) % n_samples);
-        }
-        const M3<float> A = read_matrix(smp, cap, 0, s);
-        const M3<float> U = read_matrix(smp, cap, 18, s);
-        float fe[6];
-        staple_features(A, beta, fe);
-        // forward; the layer inputs go straight to their columns and only the
-        // signs of the pre-activations are kept for the backward pass
-        float *col = inter + i;
-        float x[kMlpIn], h1[kMlpH1], o[kMlpOut];
-        uint32_t pos1 = 0u, pos2 = 0u;
-#pragma unroll
-        for (int k = 0; k < kMlpIn; k++) {
-            x[k] = (fe[k] - mean_std[k]) / mean_std[6 + k];
-            col[(size_t)(kColX + k) * batch] = x[k];
-        }
-#pragma unroll
-        for (int r = 0; r < kMlpH1; r++) {
-            float v = P[kOffB1 + r];
-#pragma unroll
-            for (int k = 0; k < kMlpIn; k++) v = fmaf(P[kOffW1 + r * kMlpIn + k], x[k], v);
-            pos1 |= (v > 0.f ? 1u : 0u) << r;
-            h1[r] = lrelu(v);
-            col[(size_t)(kColH1 + r) * batch] = h1[r];
-        }
-        {
-            float h2[kMlpH2];
-#pragma unroll
-            for (int r = 0; r < kMlpH2; r++) {
-                float v = P[kOffB2 + r];
-#pragma unroll
-                for (int k = 0; k < kMlpH1; k++) v = fmaf(P[kOffW2 + r * kMlpH1 + k], h1[k], v);
-                pos2 |= (v > 0.f ? 1u : 0u) << r;
-                h2[r] = lrelu(v);
-                col[(size_t)(kColH2 + r) * batch] = h2[r];
-            }
-#pragma unroll
-            for (int r = 0; r < kMlpOut; r++) {
-                float v = P[kOffB3 + r];
-#pragma unroll
-                for (int k = 0; k < kMlpH2; k++) v = fmaf(P[kOffW3 + r * kMlpH2 + k], h2[k], v);
-                o[r] = v;
-            }
-        }
-        float L[36];
-        cholesky_from_output(o, L);
-        const M3<float> W = mul(U, A);
-        float gW[8];
-        project_algebra(W, gW);
-        float dL[36];
-#pragma unroll
-        for (int k = 0; k < 36; k++) dL[k] = 0.f;
-        const float bf = (float)(beta / 3.0);
-        const float norm = 1.0f / ((float)batch * (float)draws);
-        Stream rs(seed, (uint32_t)i, 0u, STREAM_TRAIN, step);
-        double loss = 0.0;
-#pragma unroll 1
-        for (int k = 0; k < draws; k++) {
-            float z[8], w[8];
-            if (zin) {
-#pragma unroll
-                for (int a = 0; a < 8; a++) z[a] = zin[((size_t)i * draws + k) * 8 + a];
-            } else {
-#pragma unroll
-                for (int a = 0; a < 8; a += 2) sym_draw_pair(rs, z[a], z[a + 1]);
-            }
-            float w2 = 0.f;
-#pragma unroll
-            for (int a = 0; a < 8; a++) {
-                float v = 0.f;
-#pragma unroll
-                for (int b = 0; b <= a; b++) v = fmaf(L[a * (a + 1) / 2 + b], z[b], v);
-                w[a] = v;
-                w2 = fmaf(v, v, w2);
-            }
-            const M3<float> Y = expand(algebra_from_omega<float>(w));
-            const M3<float> YW = mul(Y, W);
-            M3<float> Q = mul(W, Y);  // Q = YW + WY
-            add_to(Q, YW);
-            const float lin = retrace(YW);
-            const float quad = retrace_mul(Y, YW);
-            const float dS = -bf * (lin + 0.5f * quad);
-            const float alpha = dS > 0.f ? __expf(-dS) : 1.f;
-            loss -= (double)(alpha * w2) * norm;
-            float gQ[8];
-            project_algebra(Q, gQ);
-            float dw[8];
-#pragma unroll
-            for (int a = 0; a < 8; a++) {
-                const float ddS = -bf * (gW[a] + 0.5f * gQ[a]);
-                const float dalpha = dS > 0.f ? -alpha * ddS : 0.f;
-                dw[a] = -(2.f * alpha * w[a] + w2 * dalpha) * norm;
-            }
-#pragma unroll
-            for (int a = 0; a < 8; a++)
-#pragma unroll
-                for (int b = 0; b <= a; b++) dL[a * (a + 1) / 2 + b] = fmaf(dw[a], z[b], dL[a * (a + 1) / 2 + b]);
-        }
-        lacc[0] = loss;
-        // d loss / d o
-        float dout[kMlpOut];
-#pragma unroll
-        for (int a = 0; a < 8; a++) {
-            dout[a] = dL[a * (a + 1) / 2 + a] * L[a * (a + 1) / 2 + a];
-#pragma unroll
-            for (int b = 0; b < a; b++) dout[8 + a * (a - 1) / 2 + b] = dL[a * (a + 1) / 2 + b];
-        }
-        float da2[kMlpH2];
-#pragma unroll
-        for (int r = 0; r < kMlpH2; r++) {
-            float v = 0.f;
-#pragma unroll
-            for (int q = 0; q < kMlpOut; q++) v = fmaf(P[kOffW3 + q * kMlpH2 + r], dout[q], v);
-            da2[r] = (pos2 >> r) & 1u ? v : 0.01f * v;
-            col[(size_t)(kColDa2 + r) * batch] = da2[r];
-        }
-#pragma unroll
-        for (int k = 0; k < kMlpOut; k++) col[(size_t)(kColDo + k) * batch] = dout[k];
-#pragma unroll
-        for (int r = 0; r < kMlpH1; r++) {
-            float v = 0.f;
-#pragma unroll
-            for (int q = 0; q < kMlpH2; q++) v = fmaf(P[kOffW2 + q * kMlpH1 + r], da2[q], v);
-            col[(size_t)(kColDa1 + r) * batch] = (pos1 >> r) & 1u ? v : 0.01f * v;
-        }
-    }
-    block_sum<1>(lacc);
-    if (threadIdx.x == 0) loss_partials[blockIdx.x] = lacc[0];
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// One thread per parameter: sum over the batch, in order, of the outer
-// product that gives its gradient.
-__global__ __launch_bounds__(kBlock) void grad_kernel(const float *__restrict__ inter, int batch,
-                                                      float *__restrict__ grad)
+__global__ __launch_bounds__(64, 1) void train_kernel(const float4 *__restrict__ smp, size_t cap, size_t n_samples,
+                                                      int batch, int draws, uint64_t seed, uint64_t step, double beta,
+                                                      const float *__restrict__ P, const float *__restrict__ mean_std,
+                                                      const float *__restrict__ zin, float *__restrict__ inter,
+                                                      double *__restrict__ loss_partials)
 {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= kNParam) return;
-    int ca, cb;  // columns multiplied (cb < 0: bias, sum of ca)
-    if (p < kOffB1) {
-        ca = kColDa1 + (p - kOffW1) / kMlpIn;
-        cb = kColX + (p - kOffW1) % kMlpIn;
-    } else if (p < kOffW2) {
-        ca = kColDa1 + (p - kOffB1);
-        cb = -1;
-    } else if (p < kOffB2) {
-        ca = kColDa2 + (p - kOffW2) / kMlpH1;
-        cb = kColH1 + (p - kOffW2) % kMlpH1;
-    } else if (p < kOffW3) {
-        ca = kColDa2 + (p - kOffB2);
-        cb = -1;
-    } else if (p < kOffB3) {
-        ca = kColDo + (p - kOffW3) / kMlpH2;
-        cb = kColH2 + (p - kOffW3) % kMlpH2;
+    __shared__ TrainLds lds;
+    const int lane = threadIdx.x, j = lane & 15, slot = lane >> 4;
+    const int i_raw = blockIdx.x * kTrainSites + j;
+    const bool valid = i_raw < batch;
+    const int i = valid ? i_raw : batch - 1;  // idle columns mirror a real sample, with zero derivatives
+    size_t s;
+    if (zin) {
+        s = (size_t)i;
     } else {
-        ca = kColDo + (p - kOffB3);
-        cb = -1;
+        uint32_t c[4] = {(uint32_t)i, (uint32_t)(step >> 32), (uint32_t)step, 0x7E57u};
+        philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+        s = (size_t)((((uint64_t)c[0] << 32) | c[1]) % n_samples);
     }
-    const float *A = inter + (size_t)ca * batch;
-    double s = 0.0;
-    if (cb < 0) {
-        for (int i = 0; i < batch; i++) s += A[i];
-    } else {
-        const float *B = inter + (size_t)cb * batch;
-        for (int i = 0; i < batch; i++) s += (double)A[i] * B[i];
+    float v36[36];
+    read_sample<9>(smp, cap, s, v36);
+    const M3<float> A = matrix_of(v36), U = matrix_of(v36 + 18);
+    {
+        float fe[6], x[8];
+        staple_features(A, beta, fe);
+#pragma unroll
+        for (int k = 0; k < kMlpIn; k++) x[k] = (fe[k] - mean_std[k]) / mean_std[6 + k];
+        x[6] = x[7] = 0.f;
+        // forward, layer by layer; lane l of a tile's result holds units
+        // 4 (l / 16) + 0..3 of sample l % 16, and reads its operand columns back
+        // as input 4 k + l / 16 of that sample
+        if (slot == 0) {
+#pragma unroll
+            for (int k = 0; k < kMlpIn; k++) lds.col[kColX + k][j] = x[k];
+            lds.col[kColOne][j] = 1.f;
+        }
+        const float x0 = slot == 0 ? x[0] : (slot == 1 ? x[1] : (slot == 2 ? x[2] : x[3]));
+        const float x1 = slot == 0 ? x[4] : (slot == 1 ? x[5] : 0.f);
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            f32x4 d;
+#pragma unroll
+            for (int r = 0; r < 4; r++) d[r] = P[kOffB1 + 16 * m + 4 * slot + r];
+            const float *w = P + kOffW1 + (16 * m + j) * kMlpIn;
+            d = mfma_f32(w[slot], x0, d);
+            d = mfma_f32(slot < 2 ? w[4 + (slot & 1)] : 0.f, x1, d);
+#pragma unroll
+            for (int r = 0; r < 4; r++) lds.col[kColH1 + 16 * m + 4 * slot + r][j] = lrelu(d[r]);
+        }
     }
-    grad[p] = (float)s;
+    __syncthreads();
+    float h1[8], h2[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) h1[k] = lds.col[kColH1 + 4 * k + slot][j];
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        f32x4 d;
+#pragma unroll
+        for (int r = 0; r < 4; r++) d[r] = P[kOffB2 + 16 * m + 4 * slot + r];
+#pragma unroll
+        for (int k = 0; k < 8; k++) d = mfma_f32(P[kOffW2 + (16 * m + j) * kMlpH1 + 4 * k + slot], h1[k], d);
+#pragma unroll
+        for (int r = 0; r < 4; r++) lds.col[kColH2 + 16 * m + 4 * slot + r][j] = lrelu(d[r]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 8; k++) h2[k] = lds.col[kColH2 + 4 * k + slot][j];
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        const bool row = 16 * m + j < kMlpOut;  // the last tile has four units
+        f32x4 d;
+#pragma unroll
+        for (int r = 0; r < 4; r++) d[r] = 16 * m + 4 * slot + r < kMlpOut ? P[kOffB3 + 16 * m + 4 * slot + r] : 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            d = mfma_f32(row ? P[kOffW3 + (16 * m + j) * kMlpH2 + 4 * k + slot] : 0.f, h2[k], d);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (16 * m + 4 * slot + r < kMlpOut) lds.col[kColDo + 16 * m + 4 * slot + r][j] = d[r];
+    }
+    __syncthreads();
+    float L[36];
+    {
+        float o[kMlpOut];
+#pragma unroll
+        for (int k = 0; k < kMlpOut; k++) o[k] = lds.col[kColDo + k][j];
+        cholesky_from_output(o, L);
+    }
+    // this slot's nine outputs: d loss / d o, summed over the draws in order
+    constexpr int kPer = kMlpOut / 4;
+    float dout[kPer], diag[kPer];
+    int ia[kPer], ib[kPer];
+#pragma unroll
+    for (int e = 0; e < kPer; e++) {
+        const int q = slot * kPer + e, ab = kCholIndex[q];
+        ia[e] = ab >> 4;
+        ib[e] = 8 + (ab & 15);
+        dout[e] = 0.f;
+        diag[e] = q < 8 ? __expf(lds.col[kColDo + q][j]) : 1.f;
+    }
+    const float bf = (float)(beta / 3.0);
+    const float norm = 1.0f / ((float)batch * (float)draws);
+    const M3<float> W = mul(U, A);
+    float gW[8];
+    project_algebra(W, gW);
+    Stream rs(seed, (uint32_t)i, 0u, STREAM_TRAIN, step);
+    double lacc = 0.0;
+#pragma unroll 1
+    for (int k0 = 0; k0 < draws; k0 += 4) {
+        const int k = k0 + slot;
+        float z[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, w[8], dw[8];
+        if (zin) {
+#pragma unroll
+            for (int a = 0; a < 8; a++) z[a] = zin[((size_t)i * draws + (k < draws ? k : draws - 1)) * 8 + a];
+        } else {
+            // the stream gives every draw four outputs; this slot takes its own
+#pragma unroll 1
+            for (int t = 0; t < 4; t++) {
+                float y[8];
+#pragma unroll
+                for (int a = 0; a < 8; a += 2) sym_draw_pair(rs, y[a], y[a + 1]);
+#pragma unroll
+                for (int a = 0; a < 8; a++) z[a] = t == slot ? y[a] : z[a];
+            }
+        }
+        float w2 = 0.f;
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            float v = 0.f;
+#pragma unroll
+            for (int b = 0; b <= a; b++) v = fmaf(L[a * (a + 1) / 2 + b], z[b], v);
+            w[a] = v;
+            w2 = fmaf(v, v, w2);
+        }
+        const M3<float> Y = expand(algebra_from_omega<float>(w));
+        const M3<float> YW = mul(Y, W);
+        M3<float> Q = mul(W, Y);  // Q = YW + WY
+        add_to(Q, YW);
+        const float lin = retrace(YW);
+        const float quad = retrace_mul(Y, YW);
+        const float dS = -bf * (lin + 0.5f * quad);
+        const float alpha = dS > 0.f ? __expf(-dS) : 1.f;
+        if (valid && k < draws) lacc -= (double)(alpha * w2) * norm;
+        float gQ[8];
+        project_algebra(Q, gQ);
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            const float ddS = -bf * (gW[a] + 0.5f * gQ[a]);
+            const float dalpha = dS > 0.f ? -alpha * ddS : 0.f;
+            dw[a] = -(2.f * alpha * w[a] + w2 * dalpha) * norm;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            lds.dz[slot][a][j] = dw[a];
+            lds.dz[slot][8 + a][j] = z[a];
+        }
+        __syncthreads();
+        const int nd = min(4, draws - k0);
+        for (int t = 0; t < nd; t++) {
+#pragma unroll
+            for (int e = 0; e < kPer; e++) dout[e] = fmaf(lds.dz[t][ia[e]][j], lds.dz[t][ib[e]][j], dout[e]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kPer; e++) lds.col[kColDo + slot * kPer + e][j] = valid ? dout[e] * diag[e] : 0.f;
+    __syncthreads();
+    // backward: transposed weights, the slope of each unit from its activation's sign
+    {
+        float d9[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) d9[k] = lds.col[kColDo + 4 * k + slot][j];
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < 9; k++) d = mfma_f32(P[kOffW3 + (4 * k + slot) * kMlpH2 + 16 * m + j], d9[k], d);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int u = 16 * m + 4 * slot + r;
+                lds.col[kColDa2 + u][j] = lds.col[kColH2 + u][j] > 0.f ? d[r] : 0.01f * d[r];
+            }
+        }
+    }
+    __syncthreads();
+    {
+        float d8[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) d8[k] = lds.col[kColDa2 + 4 * k + slot][j];
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < 8; k++) d = mfma_f32(P[kOffW2 + (4 * k + slot) * kMlpH1 + 16 * m + j], d8[k], d);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int u = 16 * m + 4 * slot + r;
+                lds.col[kColDa1 + u][j] = lds.col[kColH1 + u][j] > 0.f ? d[r] : 0.01f * d[r];
+            }
+        }
+    }
+    __syncthreads();
+    // the columns of these 16 samples, each as update_kernel's lanes read them:
+    // entry 4 k + t holds sample 4 t + k
+    float *out = inter + (size_t)blockIdx.x * kCols * kTrainSites;
+#pragma unroll 4
+    for (int c0 = 0; c0 < kCols; c0 += 4) {
+        const int c = c0 + slot;
+        if (c < kCols) out[c * kTrainSites + j] = lds.col[c][4 * (j & 3) + (j >> 2)];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) lacc += __shfl_down(lacc, off, 64);
+    if (lane == 0) loss_partials[blockIdx.x] = lacc;
 }
 
 __device__ __forceinline__ unsigned short float_to_bf16(float v)
@@ -292,13 +392,100 @@ __device__ __forceinline__ unsigned short float_to_bf16(float v)
     return (unsigned short)(r >> 16);
 }
 
-__global__ __launch_bounds__(kBlock) void adam_kernel(float *__restrict__ params, float *__restrict__ m,
-                                                      float *__restrict__ v, const float *__restrict__ grad, float lr,
-                                                      float c1, float c2, unsigned short *__restrict__ bf16)
+// The gradient of every parameter, sum over the batch of (derivative of a
+// unit) x (input), FP64 products and sums in the samples' order, and with
+// `adam` the Adam update.  One wavefront per block holds four 4 x 4 tiles of a
+// layer's [units x (inputs, one)] matrix, the last column being the bias, as one
+// v_mfma_f64_4x4x4 accumulator: each instruction adds four samples to 64
+// parameters, one after the other with one rounding each (checked), so the
+// sum is that of a plain loop over the batch.  The last block adds up the loss.
+//
+// What bounds it: the chain of batch / 4 dependent matrix instructions.  One
+// thread per parameter looping over the batch (10 blocks, two uncoalesced
+// loads an iteration) took 876 us at batch 4096, and Adam 5 us more; 19 us
+// now.
+constexpr int kTiles1 = 8 * 2, kTiles2 = 8 * 9, kTiles3 = 9 * 9, kTiles = kTiles1 + kTiles2 + kTiles3;
+constexpr int kUpdateBlocks = (kTiles + 3) / 4;
+
+__global__ __launch_bounds__(64) void update_kernel(const float *__restrict__ inter,
+                                                    const double *__restrict__ loss_partials, int groups,
+                                                    double *__restrict__ loss, float *__restrict__ grad, int adam,
+                                                    float *__restrict__ params, float *__restrict__ m,
+                                                    float *__restrict__ v, float lr, float c1, float c2,
+                                                    unsigned short *__restrict__ bf16)
 {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= kNParam) return;
-    const float g = grad[p];
+    const int lane = threadIdx.x;
+    if (blockIdx.x == kUpdateBlocks) {
+        double s = 0.0;
+        for (int b = lane; b < groups; b += 64) s += loss_partials[b];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+        if (lane == 0) *loss = s;
+        return;
+    }
+    // operands: lane l holds A[l % 4][l / 16] and B[l / 16][l % 4] of tile
+    // (l / 4) % 4; result: row l / 16, column l % 4 of that tile
+    const int tile = blockIdx.x * 4 + ((lane >> 2) & 3), unit = lane & 3, quad = lane >> 4;
+    const bool live = tile < kTiles;
+    const int t = live ? tile : kTiles - 1;
+    int row, col, cols, ca, cb, offw, offb;
+    if (t < kTiles1) {
+        row = t >> 1, col = t & 1, cols = kMlpIn, ca = kColDa1, cb = kColX, offw = kOffW1, offb = kOffB1;
+    } else if (t < kTiles1 + kTiles2) {
+        row = (t - kTiles1) / 9, col = (t - kTiles1) % 9, cols = kMlpH1, ca = kColDa2, cb = kColH1, offw = kOffW2,
+        offb = kOffB2;
+    } else {
+        row = (t - kTiles1 - kTiles2) / 9, col = (t - kTiles1 - kTiles2) % 9, cols = kMlpH2, ca = kColDo, cb = kColH2,
+        offw = kOffW3, offb = kOffB3;
+    }
+    row *= 4, col *= 4;
+    const int in = col + unit < cols ? cb + col + unit : kColOne;  // results beyond the bias column are not written
+    // one buffer resource for a group's columns, moved on group by group
+    constexpr int kStep = kCols * kTrainSites * (int)sizeof(float);
+    const unsigned oa = ((ca + row + unit) * 4 + quad) * 16u, ob = (in * 4 + quad) * 16u;
+    double s = 0.0;
+    auto add_group = [&](const float4 &x, const float4 &y) {
+        s = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x.x, (double)y.x, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x.y, (double)y.y, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x.z, (double)y.z, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x.w, (double)y.w, s, 0, 0, 0);
+    };
+    // two sets of registers: one set's groups are in flight while the other's are added
+    constexpr int kSet = 8;
+    float4 a[2][kSet], b[2][kSet];
+    auto load_set = [&](int which, int g0) {
+#pragma unroll
+        for (int k = 0; k < kSet; k++) {
+            const size_t g = min(g0 + k, groups - 1);
+            const __amdgpu_buffer_rsrc_t r =
+                __builtin_amdgcn_make_buffer_rsrc((void *)(inter + g * kCols * kTrainSites), (short)0, kStep, kBufferFlags);
+            a[which][k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, oa, 0, 0));
+            b[which][k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, ob, 0, 0));
+        }
+    };
+    load_set(0, 0);
+    int g0 = 0;
+    for (; g0 + 2 * kSet <= groups; g0 += 2 * kSet) {
+        load_set(1, g0 + kSet);
+#pragma unroll
+        for (int k = 0; k < kSet; k++) add_group(a[0][k], b[0][k]);
+        load_set(0, g0 + 2 * kSet);
+#pragma unroll
+        for (int k = 0; k < kSet; k++) add_group(a[1][k], b[1][k]);
+    }
+    load_set(1, g0 + kSet);
+#pragma unroll
+    for (int k = 0; k < kSet; k++)
+        if (g0 + k < groups) add_group(a[0][k], b[0][k]);
+#pragma unroll
+    for (int k = 0; k < kSet; k++)
+        if (g0 + kSet + k < groups) add_group(a[1][k], b[1][k]);
+    const int r = row + quad, c = col + unit;
+    if (!live || c > cols) return;
+    const int p = c < cols ? offw + r * cols + c : offb + r;
+    const float g = (float)s;
+    grad[p] = g;
+    if (!adam) return;
     const float mm = 0.9f * m[p] + 0.1f * g;
     const float vv = 0.999f * v[p] + 0.001f * g * g;
     m[p] = mm;
@@ -436,31 +623,39 @@ void launch_collect(const void *f, const Geom &g, int mu, int parity, int stride
 {
     const int n = (g.vh + stride - 1) / stride;
     collect_kernel<T, R><<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>((const typename vec2<T>::type *)f, g, mu, parity,
-                                                                   stride, out, cap, base);
+                                                                   stride, (float4 *)out, cap, base);
 }
 
-int feature_moments_blocks(size_t n) { return (int)((n + kBlock - 1) / kBlock); }
+int feature_moments_blocks(size_t n)
+{
+    return (int)std::min<size_t>(kMomentBlocks, (n + kBlock - 1) / kBlock);
+}
 
 void launch_feature_moments(const float *smp, size_t cap, size_t n, double beta, double *partials, float *mean_std,
                             hipStream_t s)
 {
     const int nb = feature_moments_blocks(n);
-    feature_moments_kernel<<<nb, kBlock, 0, s>>>(smp, cap, n, beta, partials);
-    feature_moments_finish<<<1, 64, 0, s>>>(partials, nb, n, mean_std);
+    feature_moments_kernel<<<nb, kBlock, 0, s>>>((const float4 *)smp, cap, n, beta, partials);
+    feature_moments_finish<<<1, kBlock, 0, s>>>(partials, nb, n, mean_std);
 }
+
+size_t train_inter_floats(int batch)
+{
+    return (size_t)((batch + kTrainSites - 1) / kTrainSites) * kTrainSites * kCols;
+}
+int train_groups(int batch) { return (batch + kTrainSites - 1) / kTrainSites; }
 
 void launch_train_step(const float *smp, size_t cap, size_t n_samples, int batch, int draws, uint64_t seed,
                        uint64_t step, double beta, float *params, const float *mean_std, const float *zin,
-                       float *inter, double *loss_partials, float *grad, float *m, float *v, float lr, int adam_t,
-                       unsigned short *bf16, hipStream_t s)
+                       float *inter, double *loss_partials, double *loss, float *grad, float *m, float *v, float lr,
+                       int adam_t, unsigned short *bf16, hipStream_t s)
 {
-    train_kernel<<<(batch + kBlock - 1) / kBlock, kBlock, 0, s>>>(smp, cap, n_samples, batch, draws, seed, step, beta,
-                                                                 params, mean_std, zin, inter, loss_partials);
-    grad_kernel<<<(kNParam + kBlock - 1) / kBlock, kBlock, 0, s>>>(inter, batch, grad);
-    if (adam_t > 0) {
-        const float c1 = 1.f - powf(0.9f, (float)adam_t), c2 = 1.f - powf(0.999f, (float)adam_t);
-        adam_kernel<<<(kNParam + kBlock - 1) / kBlock, kBlock, 0, s>>>(params, m, v, grad, lr, c1, c2, bf16);
-    }
+    const int groups = train_groups(batch);
+    train_kernel<<<groups, 64, 0, s>>>((const float4 *)smp, cap, n_samples, batch, draws, seed, step, beta, params,
+                                       mean_std, zin, inter, loss_partials);
+    const float c1 = 1.f - powf(0.9f, (float)adam_t), c2 = 1.f - powf(0.999f, (float)adam_t);
+    update_kernel<<<kUpdateBlocks + 1, 64, 0, s>>>(inter, loss_partials, groups, loss, grad, adam_t > 0, params, m, v,
+                                                   lr, c1, c2, bf16);
 }
 
 void launch_to_bf16(const float *params, unsigned short *bf16, hipStream_t s)

@@ -98,8 +98,8 @@ void launch_metropolis(void *f, const Geom &g, int mu, int parity, const MetroPa
                        unsigned long long *count, hipStream_t s);
 
 // ---- learned proposal (k_learned.hip) ----------------------------------------
-// Samples are stored column-major: column c (0..35: A then U, 18 reals each)
-// of sample s at out[c * cap + s].
+// Samples are 36 reals (A then U, 18 each) in nine float4 planes: reals
+// 4q..4q+3 of sample s at (float4 *)out + q * cap + s.
 template <class T, int R>
 void launch_collect(const void *f, const Geom &g, int mu, int parity, int stride, float *out, size_t cap, size_t base,
                     hipStream_t s);
@@ -109,10 +109,14 @@ void launch_feature_moments(const float *smp, size_t cap, size_t n, double beta,
 // One training step over `batch` samples (drawn from the first n_samples, or
 // the first `batch` in order with draws read from zin when zin != nullptr);
 // adam_t > 0 applies an Adam update (bias corrections for step adam_t).
+// inter: train_inter_floats(batch) floats; loss_partials: train_groups(batch)
+// doubles; the step's loss goes to *loss.
+size_t train_inter_floats(int batch);
+int train_groups(int batch);
 void launch_train_step(const float *smp, size_t cap, size_t n_samples, int batch, int draws, uint64_t seed,
                        uint64_t step, double beta, float *params, const float *mean_std, const float *zin,
-                       float *inter, double *loss_partials, float *grad, float *m, float *v, float lr, int adam_t,
-                       unsigned short *bf16, hipStream_t s);
+                       float *inter, double *loss_partials, double *loss, float *grad, float *m, float *v, float lr,
+                       int adam_t, unsigned short *bf16, hipStream_t s);
 void launch_to_bf16(const float *params, unsigned short *bf16, hipStream_t s);
 template <class T, int R>
 void launch_metropolis_learned(void *f, const Geom &g, int mu, int parity, const MetroParams &p,
@@ -120,7 +124,6 @@ void launch_metropolis_learned(void *f, const Geom &g, int mu, int parity, const
                                hipStream_t s);
 void launch_proposal_eval(const float *feat, int n, const unsigned short *wbf16, const float *mean_std, float *out,
                           int *ok, hipStream_t s);
-constexpr int kTrainInterCols = 170;  // per-sample columns kept by the training step
 constexpr int kProposalParams = 2468;
 
 } // namespace glacx
