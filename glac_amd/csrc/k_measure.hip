@@ -14,6 +14,8 @@
 // one slice; per-site values are summed in FP64, the block partials are
 // combined per time slice and then over slices in a fixed order, which makes
 // the result independent of scheduling.
+#include <algorithm>
+
 #include "kernels.hpp"
 
 namespace glacx {
@@ -308,45 +310,85 @@ __global__ __launch_bounds__(64) void measure_finish_kernel(const double *__rest
     }
 }
 
-// Plaquette only: sum over sites and the 6 planes of
-// Re tr[U_mu(x) U_nu(x+mu) (U_nu(x) U_mu(x+nu))^dagger]
-// (GLAC/observables/plaquette.cpp:26-40).
+// Re tr P of one plane at x, P = U_mu(x) U_nu(x+mu) (U_nu(x) U_mu(x+nu))^dagger.
+// With two stored rows only the first two rows of the two products A and B are
+// formed: the third rows being conj(A0 x A1) and conj(B0 x B1), their inner
+// product is conj((A0.B0*)(A1.B1*) - (A0.B1*)(A1.B0*)), from the same inner
+// products that give the other two rows' part.
 template <class T, int R>
-__global__ __launch_bounds__(kBlock) void plaquette_kernel(const typename vec2<T>::type *__restrict__ f, Geom g,
-                                                           double *__restrict__ partials)
+__device__ __forceinline__ T plane_plaquette(const typename vec2<T>::type *__restrict__ f, const Geom &g, const Site &x,
+                                             int mu, int nu)
 {
-    const int idx = blockIdx.x * kBlock + threadIdx.x;
-    double acc[1] = {0.0};
-    if (idx < g.v) {
-        const Site x = site_of(g, idx);
-        T s = T(0);
-#pragma unroll 1
-        for (int mu = 0; mu < 3; mu++) {
-            const M3<T> umu = load_link<T, R>(f, g, mu, idx);
-            const int ipm = site_step(g, x, mu, +1).idx;
-#pragma unroll 1
-            for (int nu = mu + 1; nu < 4; nu++) {
-                const M3<T> a = mul(umu, load_link<T, R>(f, g, nu, ipm));
-                const M3<T> b = mul(load_link<T, R>(f, g, nu, idx), load_link<T, R>(f, g, mu, site_step(g, x, nu, +1).idx));
-                // Re tr(a b^dag) = sum_ij Re(a_ij conj(b_ij))
+    const DirView<T> vmu = dir_view<T>(f, g, mu), vnu = dir_view<T>(f, g, nu);
+    const int ipm = site_step(g, x, mu, +1).idx, ipn = site_step(g, x, nu, +1).idx;
+    if constexpr (R == 2) {
+        M3<T> a, b;
+        mm<false, false, false, 2>(a, load_rows01<T, R>(vmu, x.idx), load_link<T, R>(vnu, ipm));
+        mm<false, false, false, 2>(b, load_rows01<T, R>(vnu, x.idx), load_link<T, R>(vmu, ipn));
+        cpx<T> d[2][2];
 #pragma unroll
-                for (int i = 0; i < 3; i++)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-                    for (int j = 0; j < 3; j++) s += a.e[i][j].r * b.e[i][j].r + a.e[i][j].i * b.e[i][j].i;
+            for (int j = 0; j < 2; j++) {
+                T re = T(0), im = T(0);
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    re = fma(a.e[i][k].r, b.e[j][k].r, fma(a.e[i][k].i, b.e[j][k].i, re));
+                    im = fma(a.e[i][k].i, b.e[j][k].r, fma(-a.e[i][k].r, b.e[j][k].i, im));
+                }
+                d[i][j] = {re, im};
             }
-        }
-        acc[0] = s;
+        const cpx<T> p = cmul(d[0][0], d[1][1]), q = cmul(d[0][1], d[1][0]);
+        return d[0][0].r + d[1][1].r + (p.r - q.r);
+    } else {
+        const M3<T> a = mul(load_link<T, R>(vmu, x.idx), load_link<T, R>(vnu, ipm));
+        const M3<T> b = mul(load_link<T, R>(vnu, x.idx), load_link<T, R>(vmu, ipn));
+        // Re tr(a b^dag) = sum_ij Re(a_ij conj(b_ij))
+        T s = T(0);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) s = fma(a.e[i][j].r, b.e[i][j].r, fma(a.e[i][j].i, b.e[i][j].i, s));
+        return s;
     }
-    block_sum<1>(acc);
+}
+
+// Plaquette only: sum over sites and the 6 planes (GLAC/observables/
+// plaquette.cpp:26-40).  Launched as the clover kernel is: 64 sites (32 of each
+// parity, in the flow stage's order) x 3 wavefronts, wavefront w taking the
+// planes (0, w + 1) and (rho, sigma).
+//
+// What bounds it: VALU issue with FP32 links, memory latency with FP64 ones.
+// One thread per site looping over the planes in storage order kept too few
+// loads in flight and re-read links across XCDs: compressed FP32 104 us at
+// 32^4 and 96 us at 24^3 x 48, FP64 21.7 us at 16^4; now 51, 35 and 13 us
+// (32^4: 3.9 TB/s of links read once).  Blocks of two or four chunks, which would
+// leave fewer partials to the second kernel, took 59 and 70 us at 32^4: the
+// blocks running together then spread over more of the lattice than an L2 holds.
+template <class T, int R>
+__global__ __launch_bounds__(kMeasSites *kMeasWaves) void plaquette_kernel(const typename vec2<T>::type *__restrict__ f,
+                                                                          Geom g, double *__restrict__ partials)
+{
+    const int lane = threadIdx.x & 63;
+    const int nu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + 1, rho = nu % 3 + 1, sigma = rho % 3 + 1;
+    const int h = flow_chunk(g, xcd_block(blockIdx.x, gridDim.x)) * (kMeasSites / 2) + (lane & 31);
+    double acc[1] = {0.0};
+    if (h < g.vh) {
+        const Site x = site_of(g, parity_index(g, lane >> 5, h));
+        acc[0] = plane_plaquette<T, R>(f, g, x, 0, nu) + plane_plaquette<T, R>(f, g, x, rho, sigma);
+    }
+    block_sum<1, kMeasWaves>(acc);
     if (threadIdx.x == 0) partials[blockIdx.x] = acc[0];
 }
 
-__global__ __launch_bounds__(kBlock) void plaquette_finish_kernel(const double *__restrict__ partials, int n, Geom g,
-                                                                  double *__restrict__ out)
+constexpr int kFinishBlock = 1024;
+__global__ __launch_bounds__(kFinishBlock) void plaquette_finish_kernel(const double *__restrict__ partials, int n, Geom g,
+                                                                        double *__restrict__ out)
 {
     double acc[1] = {0.0};
-    for (int b = threadIdx.x; b < n; b += kBlock) acc[0] += partials[b];
-    block_sum<1>(acc);
+#pragma unroll 8
+    for (int b = threadIdx.x; b < n; b += kFinishBlock) acc[0] += partials[b];
+    block_sum<1, kFinishBlock / 64>(acc);
     if (threadIdx.x == 0) out[0] = acc[0] / (18.0 * (double)g.v);
 }
 
@@ -355,7 +397,7 @@ static inline int chunks_per_slab(const Geom &g) { return g.nzb * g.cpr; }
 
 // block partials followed by the per-slice sums
 int measure_partials_count(const Geom &g) { return kMeasAcc * g.n[3] * chunks_per_slab(g) + kMeasAcc * g.n[3]; }
-int plaquette_partials_count(const Geom &g) { return (g.v + kBlock - 1) / kBlock; }
+int plaquette_partials_count(const Geom &g) { return (g.vh + kMeasSites / 2 - 1) / (kMeasSites / 2); }
 
 template <class T, int R>
 void launch_measure(const void *f, const Geom &g, double *partials, int mode, double *density, hipStream_t s)
@@ -381,12 +423,13 @@ void launch_measure_finish(double *partials, const Geom &g, double *out, bool su
 
 template <class T, int R> void launch_plaquette(const void *f, const Geom &g, double *partials, hipStream_t s)
 {
-    plaquette_kernel<T, R><<<plaquette_partials_count(g), kBlock, 0, s>>>((const typename vec2<T>::type *)f, g, partials);
+    plaquette_kernel<T, R><<<plaquette_partials_count(g), kMeasSites * kMeasWaves, 0, s>>>(
+        (const typename vec2<T>::type *)f, g, partials);
 }
 
 void launch_plaquette_finish(const double *partials, int nparts, const Geom &g, double *out, hipStream_t s)
 {
-    plaquette_finish_kernel<<<1, kBlock, 0, s>>>(partials, nparts, g, out);
+    plaquette_finish_kernel<<<1, kFinishBlock, 0, s>>>(partials, nparts, g, out);
 }
 
 template void launch_measure<float, 3>(const void *, const Geom &, double *, int, double *, hipStream_t);
