@@ -154,24 +154,24 @@ int timed_end(glacx_ctx *c, int kernel, hipEvent_t start)
 // per-site densities written to `density` (2V doubles).
 // `partials` holds measure_partials_count(geom) doubles.
 template <class T, int R>
-int run_measure_into(glacx_ctx *c, const void *f, double *partials, double *out, int mode, double *density = nullptr)
+int run_measure_partials(glacx_ctx *c, const void *f, double *partials, int mode, double *density = nullptr)
 {
     hipEvent_t e0 = nullptr;
     int rc;
     if ((rc = timed_begin(c, &e0))) return rc;
     launch_measure<T, R>(f, c->geom, partials, mode, density, c->stream);
     CHECK_LAUNCH(c);
-    if ((rc = timed_end(c, GLACX_K_MEASURE, e0))) return rc;
-    launch_measure_finish(partials, c->geom, out, mode == 1, c->stream);
-    CHECK_LAUNCH(c);
-    return GLACX_OK;
+    return timed_end(c, GLACX_K_MEASURE, e0);
 }
 
 template <class T, int R> int run_measure(glacx_ctx *c, const void *f, double *out, int mode, double *density = nullptr)
 {
     int rc = ensure(c, &c->partials, &c->partials_len, (size_t)measure_partials_count(c->geom));
     if (rc) return rc;
-    return run_measure_into<T, R>(c, f, c->partials, out, mode, density);
+    if ((rc = run_measure_partials<T, R>(c, f, c->partials, mode, density))) return rc;
+    launch_measure_finish(c->partials, c->geom, out, mode == 1, 1, 0, c->stream);
+    CHECK_LAUNCH(c);
+    return GLACX_OK;
 }
 
 template <class T, int R> int run_plaquette(glacx_ctx *c, const void *f, double *out)
@@ -208,34 +208,36 @@ template <class T, int R> int run_flow_step(glacx_ctx *c, void *f, double eps, d
 }
 
 // n_steps flow steps of `field`, measuring before the first and after every
-// step into results (rows of `row` doubles) when results is set, with
-// `partials` (measure_partials_count(geom) doubles) as the reduction buffer.
-// Each step's stage 0 measures the field it reads (the previous step's
-// result), and the clover kernel measures once more after the last step; the
-// SuperSampler set and lattices whose runs are not whole 32-site chunks use
+// step into results (rows of `row` doubles) when results is set.  `partials`
+// holds `slots` measurements' partials (measure_partials_count(geom) doubles
+// each), which are summed to their rows together whenever the slots are full
+// and at the end.  Each step's stage 0 measures the field it reads (the previous
+// step's result), and the clover kernel measures once more after the last step;
+// the SuperSampler set and lattices whose runs are not whole 32-site chunks use
 // the clover kernel between steps.
 template <class T, int R>
 int run_flow(glacx_ctx *c, int field, int n_steps, double eps, double *results, size_t row, bool super,
-             double *partials)
+             double *partials, int slots)
 {
     const bool fuse = results && !super && flow_measure_fusable(c->geom);
     const int mode = super ? 1 : 0;
+    const size_t per = (size_t)measure_partials_count(c->geom);
     int rc;
-    if (results && !fuse && (rc = run_measure_into<T, R>(c, c->field[field], partials, results, mode))) return rc;
-    for (int i = 0; i < n_steps; i++) {
-        if ((rc = run_flow_step<T, R>(c, c->field[field], eps, fuse ? partials : nullptr))) return rc;
-        if (fuse) {
-            launch_measure_finish(partials, c->geom, results + row * (size_t)i, false, c->stream);
+    for (int i = 0; i <= n_steps; i++) {  // measurement i, then step i
+        const int slot = slots > 0 ? i % slots : 0;
+        double *part = partials + per * slot;
+        const bool fused = fuse && i < n_steps;
+        if (results && !fused && (rc = run_measure_partials<T, R>(c, c->field[field], part, mode))) return rc;
+        if (i < n_steps) {
+            if ((rc = run_flow_step<T, R>(c, c->field[field], eps, fused ? part : nullptr))) return rc;
+            // three stages leave the result in the work buffer: swap roles
+            std::swap(c->field[field], c->work);
+        }
+        if (results && (slot == slots - 1 || i == n_steps)) {
+            launch_measure_finish(partials, c->geom, results + row * (size_t)(i - slot), super, slot + 1, row, c->stream);
             CHECK_LAUNCH(c);
         }
-        // three stages leave the result in the work buffer: swap roles
-        std::swap(c->field[field], c->work);
-        if (results && !fuse &&
-            (rc = run_measure_into<T, R>(c, c->field[field], partials, results + row * (size_t)(i + 1), mode)))
-            return rc;
     }
-    if (fuse && (rc = run_measure_into<T, R>(c, c->field[field], partials, results + row * (size_t)n_steps, mode)))
-        return rc;
     return GLACX_OK;
 }
 
@@ -706,6 +708,15 @@ int glacx_plaquette(glacx_ctx *c, int field, double *plaq)
 
 namespace {
 
+// Measurements whose partials a flow holds before it sums them: all of them, or
+// as many as `limit` doubles take (kFlowPartials: 32 MiB of a context, which is
+// 64 measurements at 32^4 and six at 48^3 x 96).
+constexpr size_t kFlowPartials = (size_t)4 << 20;
+int flow_slots(size_t per, int n_steps, size_t limit)
+{
+    return (int)std::min<size_t>((size_t)n_steps + 1, std::max<size_t>(1, limit / per));
+}
+
 int flow_impl(glacx_ctx *c, int field, int n_steps, double eps, bool super, double *plaq, double *e_raw, double *q,
               double *w, double *q_t, double *w_t)
 {
@@ -715,8 +726,10 @@ int flow_impl(glacx_ctx *c, int field, int n_steps, double eps, bool super, doub
     const size_t row = super ? (size_t)4 + 2 * nt : (size_t)3 + nt;
     int rc;
     if (meas && (rc = ensure(c, &c->results, &c->results_len, row * (size_t)(n_steps + 1)))) return rc;
-    if (meas && (rc = ensure(c, &c->partials, &c->partials_len, (size_t)measure_partials_count(c->geom)))) return rc;
-    if ((rc = DISPATCH(c, run_flow, c, field, n_steps, eps, meas ? c->results : nullptr, row, super, c->partials)))
+    const size_t per = (size_t)measure_partials_count(c->geom);
+    const int slots = flow_slots(per, n_steps, kFlowPartials);
+    if (meas && (rc = ensure(c, &c->partials, &c->partials_len, per * slots))) return rc;
+    if ((rc = DISPATCH(c, run_flow, c, field, n_steps, eps, meas ? c->results : nullptr, row, super, c->partials, slots)))
         return rc;
     if (meas) {
         std::vector<double> h(row * (size_t)(n_steps + 1));
@@ -763,16 +776,18 @@ int glacx_flow_noalloc(glacx_ctx *c, int field, int n_steps, double eps, double 
     const int nt = c->dims[3];
     const size_t row = (size_t)3 + nt;
     const size_t np = (size_t)measure_partials_count(c->geom);
-    const size_t need = meas ? np + row * ((size_t)n_steps + 1) : 0;
+    const size_t rows_len = meas ? row * ((size_t)n_steps + 1) : 0, need = meas ? np + rows_len : 0;
     if (need * sizeof(double) > kScratchBytes)
         return fail(c, GLACX_E_ARG, "flow_noalloc: " + std::to_string(n_steps) + " measured steps on this lattice need " +
                                         std::to_string(need * sizeof(double)) + " bytes of scratch, above its " +
                                         std::to_string(kScratchBytes) + "; split the flow into shorter calls");
-    double *partials = c->scratch, *results = c->scratch + np;
+    // the results first, the measurements' partials in what is left
+    double *results = c->scratch, *partials = c->scratch + rows_len;
+    const int slots = flow_slots(np, n_steps, kScratchBytes / sizeof(double) - rows_len);
     // event timing would create events: off for this call
     const bool timing = c->timing;
     c->timing = false;
-    int rc = DISPATCH(c, run_flow, c, field, n_steps, eps, meas ? results : nullptr, row, false, partials);
+    int rc = DISPATCH(c, run_flow, c, field, n_steps, eps, meas ? results : nullptr, row, false, partials, slots);
     c->timing = timing;
     if (rc) return rc;
     // rows {plaq, E_raw, Q, Q(t)...} to the caller's arrays by strided copies

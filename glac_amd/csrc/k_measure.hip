@@ -255,35 +255,22 @@ __attribute__((amdgpu_waves_per_eu(meas_waves<T>(), meas_waves<T>()))) void meas
     }
 }
 
-// One block per time slice t: sums the partials of the chunks of slice t in
-// a fixed order into slice[kMeasAcc t ...].
-__global__ __launch_bounds__(kBlock) void measure_slice_kernel(const double *__restrict__ partials, Geom g, int cps,
-                                                               double *__restrict__ slice)
-{
-    const int t = blockIdx.x;
-    double acc[kMeasAcc] = {0.0, 0.0, 0.0, 0.0};
-    for (int c = threadIdx.x; c < cps; c += kBlock) {
-        const double *q = partials + kMeasAcc * (c * g.n[3] + t);
-#pragma unroll
-        for (int i = 0; i < kMeasAcc; i++) acc[i] += q[i];
-    }
-    block_sum<kMeasAcc>(acc);
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int i = 0; i < kMeasAcc; i++) slice[kMeasAcc * t + i] = acc[i];
-}
-
+// ---- from a measurement's partials to its row of results ---------------------
 // out = {plaq, E_raw, Q, Q(t = 0..Nt-1)}, or with `super`
 // {plaq, E_raw, Q, W, Q(t)..., W(t)...}; W's normalisation is GLAC's
-// 2 * 8 * 8 / (3 * 16^3) (GLAC/observables/supersampler.cpp:17-19).
-// One wavefront: lane l takes the slices t = l, l + 64, ... in order, then
-// the lanes' sums are combined by a fixed shuffle tree (the order never
-// depends on scheduling).
-__global__ __launch_bounds__(64) void measure_finish_kernel(const double *__restrict__ slice, Geom g, int super,
-                                                            double *__restrict__ out)
+// 2 * 8 * 8 / (3 * 16^3) (GLAC/observables/supersampler.cpp:17-19).  The
+// kernels take several measurements at once (blockIdx.y or .x): `stride`
+// doubles of partials and `pitch` of results from one to the next.  A flow
+// leaves its steps' partials side by side and sums them together: two small
+// launches after every step took 9.5 us of its 850 at 32^4 and 8 of 45 at
+// 8^3 x 16.  The order of every sum is fixed by the lattice alone.
+
+// The per-slice sums of one measurement by one wavefront, into its row.
+__device__ __forceinline__ void finish_row(const double *__restrict__ slice, const Geom &g, int super, int lane,
+                                           double *__restrict__ out)
 {
     const double qnorm = 1.0 / (256.0 * M_PI * M_PI), wnorm = 2.0 * 8.0 * 8.0 / (3.0 * 16.0 * 16.0 * 16.0);
-    const int nt = g.n[3], head = super ? 4 : 3, lane = threadIdx.x;
+    const int nt = g.n[3], head = super ? 4 : 3;
     double v[4] = {0.0, 0.0, 0.0, 0.0};  // plaquette, energy, q, w
     for (int t = lane; t < nt; t += 64) {
         const double *st = slice + kMeasAcc * t;
@@ -308,6 +295,62 @@ __global__ __launch_bounds__(64) void measure_finish_kernel(const double *__rest
         out[2] = v[2];
         if (super) out[3] = v[3];
     }
+}
+
+// Few chunks: one block per measurement, a wavefront per time slice.
+constexpr int kRowWaves = 16, kRowSlices = 512;  // a context's largest extent is 512
+constexpr int kRowChunks = 2048;
+__global__ __launch_bounds__(64 * kRowWaves) void measure_row_kernel(const double *__restrict__ partials, Geom g, int cps,
+                                                                     int super, size_t stride, size_t pitch,
+                                                                     double *__restrict__ out)
+{
+    __shared__ double slice[kMeasAcc * kRowSlices];
+    const double *p = partials + blockIdx.x * stride;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nt = g.n[3];
+    for (int t = wave; t < nt; t += kRowWaves) {
+        double acc[kMeasAcc] = {0.0, 0.0, 0.0, 0.0};
+        for (int c = lane; c < cps; c += 64) {
+            const double *q = p + kMeasAcc * (c * nt + t);
+#pragma unroll
+            for (int i = 0; i < kMeasAcc; i++) acc[i] += q[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kMeasAcc; i++)
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) acc[i] += __shfl_down(acc[i], off, 64);
+        if (lane == 0)
+#pragma unroll
+            for (int i = 0; i < kMeasAcc; i++) slice[kMeasAcc * t + i] = acc[i];
+    }
+    __syncthreads();
+    if (wave == 0) finish_row(slice, g, super, lane, out + blockIdx.x * pitch);
+}
+
+// Many chunks: one block per time slice and measurement sums the slice's
+// chunks behind the measurement's partials, ...
+__global__ __launch_bounds__(kBlock) void measure_slice_kernel(double *__restrict__ partials, Geom g, int cps,
+                                                               size_t stride)
+{
+    const int t = blockIdx.x;
+    double *p = partials + blockIdx.y * stride;
+    double acc[kMeasAcc] = {0.0, 0.0, 0.0, 0.0};
+    for (int c = threadIdx.x; c < cps; c += kBlock) {
+        const double *q = p + kMeasAcc * (c * g.n[3] + t);
+#pragma unroll
+        for (int i = 0; i < kMeasAcc; i++) acc[i] += q[i];
+    }
+    block_sum<kMeasAcc>(acc);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int i = 0; i < kMeasAcc; i++) p[kMeasAcc * (g.n[3] * cps + t) + i] = acc[i];
+}
+
+// ... then one wavefront per measurement.
+__global__ __launch_bounds__(64) void measure_finish_kernel(const double *__restrict__ partials, Geom g, int cps, int super,
+                                                            size_t stride, size_t pitch, double *__restrict__ out)
+{
+    finish_row(partials + blockIdx.x * stride + (size_t)kMeasAcc * g.n[3] * cps, g, super, threadIdx.x,
+               out + blockIdx.x * pitch);
 }
 
 // Re tr P of one plane at x, P = U_mu(x) U_nu(x+mu) (U_nu(x) U_mu(x+nu))^dagger.
@@ -413,12 +456,20 @@ void launch_measure(const void *f, const Geom &g, double *partials, int mode, do
         measure_kernel<T, R, MEAS_PLAIN><<<blocks, threads, 0, s>>>(fp, g, cps, partials, density);
 }
 
-void launch_measure_finish(double *partials, const Geom &g, double *out, bool super, hipStream_t s)
+void launch_measure_finish(double *partials, const Geom &g, double *out, bool super, int rows, size_t pitch,
+                           hipStream_t s)
 {
     const int cps = chunks_per_slab(g);
-    double *slice = partials + kMeasAcc * g.n[3] * cps;
-    measure_slice_kernel<<<g.n[3], kBlock, 0, s>>>(partials, g, cps, slice);
-    measure_finish_kernel<<<1, 64, 0, s>>>(slice, g, super ? 1 : 0, out);
+    const size_t stride = (size_t)measure_partials_count(g);
+    // 128 chunks (8^3 x 16) take 4.0 us in one kernel and 5.7 in two, 504 take
+    // 6.0 and 9.9, 10368 (24^3 x 48) 19.7 and 11.4: the line lies between, where
+    // one block's loads cost what the second launch does
+    if (cps * g.n[3] <= kRowChunks) {
+        measure_row_kernel<<<rows, 64 * kRowWaves, 0, s>>>(partials, g, cps, super ? 1 : 0, stride, pitch, out);
+    } else {
+        measure_slice_kernel<<<dim3(g.n[3], rows), kBlock, 0, s>>>(partials, g, cps, stride);
+        measure_finish_kernel<<<rows, 64, 0, s>>>(partials, g, cps, super ? 1 : 0, stride, pitch, out);
+    }
 }
 
 template <class T, int R> void launch_plaquette(const void *f, const Geom &g, double *partials, hipStream_t s)
