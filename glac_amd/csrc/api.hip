@@ -32,6 +32,8 @@ struct glacx_ctx {
     size_t results_len = 0;
     unsigned long long *counts = nullptr;  // accepted hits per sweep
     size_t counts_len = 0;
+    int *flag = nullptr;             // one int: the SU(3) check's answer
+    size_t flag_len = 0;
     double *stage = nullptr;         // AoS FP64 staging for host transfers
     double *scratch = nullptr;       // this device's copy of `scratch` (allocation-free calls)
     size_t device_bytes = 0;
@@ -345,16 +347,37 @@ double su3_defect(const double *m)
     return worst;
 }
 
-int require_su3(glacx_ctx *c, const double *links, size_t n_links, size_t stride, const char *who)
+constexpr double kSu3Bound = 1e-6;
+
+int require_su3(glacx_ctx *c, const double *links, size_t n_links, const char *who)
 {
-    if (c->precision != GLACX_FP32_COMPRESSED) return GLACX_OK;
     for (size_t i = 0; i < n_links; i++) {
-        const double d = su3_defect(links + i * stride);
-        if (!(d < 1e-6))
+        const double d = su3_defect(links + i * 18);
+        if (!(d < kSu3Bound))
             return fail(c, GLACX_E_ARG, std::string(who) + ": the compressed FP32 mode stores two rows per link and "
                                         "needs SU(3) links; link " + std::to_string(i) + " deviates by " +
                                         std::to_string(d));
     }
+    return GLACX_OK;
+}
+
+// Whether the 4 V links in the staging buffer need require_su3's look: the
+// device checks them all, with a bound that is lower by more than FP64 rounding
+// (a few 1e-15 for links near SU(3)), so that only links which are or may be
+// refused are looked at again.
+int su3_suspected(glacx_ctx *c, bool *suspected)
+{
+    *suspected = false;
+    if (c->precision != GLACX_FP32_COMPRESSED) return GLACX_OK;
+    int rc = ensure(c, &c->flag, &c->flag_len, 1);
+    if (rc) return rc;
+    HIP_TRY(c, hipMemsetAsync(c->flag, 0, sizeof(int), c->stream));
+    launch_su3_check(c->stage, 4 * c->geom.v, kSu3Bound * (1.0 - 1e-6), c->flag, c->stream);
+    CHECK_LAUNCH(c);
+    int h = 0;
+    HIP_TRY(c, hipMemcpyAsync(&h, c->flag, sizeof h, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    *suspected = h != 0;
     return GLACX_OK;
 }
 
@@ -441,7 +464,7 @@ int glacx_destroy(glacx_ctx *c)
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void *p : {c->field[0], c->field[1], c->work, c->acc, (void *)c->partials, (void *)c->results,
-                    (void *)c->counts, (void *)c->stage, (void *)c->samples, (void *)c->params,
+                    (void *)c->counts, (void *)c->flag, (void *)c->stage, (void *)c->samples, (void *)c->params,
                     (void *)c->params_bf16, (void *)c->mean_std, (void *)c->inter})
         if (p) (void)hipFree(p);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
@@ -472,13 +495,15 @@ int glacx_upload_field(glacx_ctx *c, int field, const double *const links[4])
     if (!valid_field(field) || !links) return fail(c, GLACX_E_ARG, "upload: bad field or pointer");
     for (int mu = 0; mu < 4; mu++)
         if (!links[mu]) return fail(c, GLACX_E_ARG, "upload: null link array");
-    int rc;
-    for (int mu = 0; mu < 4; mu++)
-        if ((rc = require_su3(c, links[mu], (size_t)c->geom.v, 18, "upload"))) return rc;
-    if ((rc = ensure_stage(c))) return rc;
+    int rc = ensure_stage(c);
+    if (rc) return rc;
     const size_t n = (size_t)c->geom.v * 18;
     for (int mu = 0; mu < 4; mu++)
         HIP_TRY(c, hipMemcpyAsync(c->stage + mu * n, links[mu], n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    bool suspected;
+    if ((rc = su3_suspected(c, &suspected))) return rc;
+    for (int mu = 0; suspected && mu < 4; mu++)
+        if ((rc = require_su3(c, links[mu], (size_t)c->geom.v, "upload"))) return rc;
     DISPATCH(c, launch_pack, c->stage, c->field[field], c->geom, 0, c->stream);
     CHECK_LAUNCH(c);
     HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -532,10 +557,12 @@ int load_site_major(glacx_ctx *c, int field, const char *path, bool byteswap, co
             u = __builtin_bswap64(u);
             std::memcpy(&buf[i], &u, sizeof u);
         }
-    int rc = require_su3(c, buf.data(), (size_t)c->geom.v * 4, 18, who);
+    int rc = ensure_stage(c);
     if (rc) return rc;
-    if ((rc = ensure_stage(c))) return rc;
     HIP_TRY(c, hipMemcpyAsync(c->stage, buf.data(), n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    bool suspected;
+    if ((rc = su3_suspected(c, &suspected))) return rc;
+    if (suspected && (rc = require_su3(c, buf.data(), (size_t)c->geom.v * 4, who))) return rc;
     DISPATCH(c, launch_pack, c->stage, c->field[field], c->geom, 1, c->stream);
     CHECK_LAUNCH(c);
     HIP_TRY(c, hipStreamSynchronize(c->stream));

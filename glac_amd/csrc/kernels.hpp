@@ -56,6 +56,9 @@ template <int N, int WAVES = kBlock / 64> __device__ __forceinline__ void block_
 // ---- launchers (explicitly instantiated for float and double) ------------
 template <class T, int R> void launch_pack(const double *stage, void *f, const Geom &g, int site_major, hipStream_t s);
 template <class T, int R> void launch_unpack(const void *f, double *stage, const Geom &g, int site_major, hipStream_t s);
+// *flag = 1 when one of n links (18 doubles each) is not within `bound` of SU(3)
+// (see su3_check_kernel); otherwise left as it is.
+void launch_su3_check(const double *links, int n, double bound, int *flag, hipStream_t s);
 // Hot-start kinds (the values of the C ABI's GLACX_HOT_*).
 enum HotKind { HOT_HAAR = 0, HOT_GLAC_RANDOM = 1, HOT_RST = 2 };
 template <class T, int R> void launch_hot_start(void *f, const Geom &g, uint64_t seed, int kind, double eps, hipStream_t s);
