@@ -13,6 +13,7 @@
 
 #include "../../include/glacx.h"
 #include "kernels.hpp"
+#include "transfer.hpp"
 
 using namespace glacx;
 
@@ -35,6 +36,7 @@ struct glacx_ctx {
     int *flag = nullptr;             // one int: the SU(3) check's answer
     size_t flag_len = 0;
     double *stage = nullptr;         // AoS FP64 staging for host transfers
+    Transfer transfer;               // pinned slices between host arrays and the device
     double *scratch = nullptr;       // this device's copy of `scratch` (allocation-free calls)
     size_t device_bytes = 0;
     std::string err;
@@ -112,6 +114,17 @@ int ensure_stage(glacx_ctx *c)
     int rc = dev_alloc(c, &p, (size_t)4 * c->geom.v * 18 * sizeof(double));
     c->stage = (double *)p;
     return rc;
+}
+
+// `n` doubles of each host array to the device buffer `dev`, one after the
+// other, or back (null arrays are passed over).
+int copy_host(glacx_ctx *c, double *dev, const double *const *host, int arrays, size_t n, bool up)
+{
+    std::vector<HostSpan> spans;
+    for (int k = 0; k < arrays; k++)
+        if (host[k]) spans.push_back({(char *)host[k], (char *)(dev + (size_t)k * n), n * sizeof(double)});
+    HIP_TRY(c, c->transfer.run(spans, up, c->device, c->stream));
+    return GLACX_OK;
 }
 
 // ---- event timing --------------------------------------------------------
@@ -498,8 +511,7 @@ int glacx_upload_field(glacx_ctx *c, int field, const double *const links[4])
     int rc = ensure_stage(c);
     if (rc) return rc;
     const size_t n = (size_t)c->geom.v * 18;
-    for (int mu = 0; mu < 4; mu++)
-        HIP_TRY(c, hipMemcpyAsync(c->stage + mu * n, links[mu], n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    if ((rc = copy_host(c, c->stage, links, 4, n, true))) return rc;
     bool suspected;
     if ((rc = su3_suspected(c, &suspected))) return rc;
     for (int mu = 0; suspected && mu < 4; mu++)
@@ -520,11 +532,7 @@ int glacx_download_field(glacx_ctx *c, int field, double *const links[4])
     if (rc) return rc;
     DISPATCH(c, launch_unpack, c->field[field], c->stage, c->geom, 0, c->stream);
     CHECK_LAUNCH(c);
-    const size_t n = (size_t)c->geom.v * 18;
-    for (int mu = 0; mu < 4; mu++)
-        HIP_TRY(c, hipMemcpyAsync(links[mu], c->stage + mu * n, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    return GLACX_OK;
+    return copy_host(c, c->stage, links, 4, (size_t)c->geom.v * 18, false);
 }
 
 int glacx_copy_field(glacx_ctx *c, int dst, int src)
@@ -559,7 +567,8 @@ int load_site_major(glacx_ctx *c, int field, const char *path, bool byteswap, co
         }
     int rc = ensure_stage(c);
     if (rc) return rc;
-    HIP_TRY(c, hipMemcpyAsync(c->stage, buf.data(), n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    const double *host = buf.data();
+    if ((rc = copy_host(c, c->stage, &host, 1, n, true))) return rc;
     bool suspected;
     if ((rc = su3_suspected(c, &suspected))) return rc;
     if (suspected && (rc = require_su3(c, buf.data(), (size_t)c->geom.v * 4, who))) return rc;
@@ -593,8 +602,8 @@ int glacx_save_bin(glacx_ctx *c, int field, const char *path)
     std::vector<double> buf(n);
     DISPATCH(c, launch_unpack, c->field[field], c->stage, c->geom, 1, c->stream);
     CHECK_LAUNCH(c);
-    HIP_TRY(c, hipMemcpyAsync(buf.data(), c->stage, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    const double *host = buf.data();
+    if ((rc = copy_host(c, c->stage, &host, 1, n, false))) return rc;
     FILE *fp = std::fopen(path, "wb");
     if (!fp) return fail(c, GLACX_E_IO, std::string("save_bin: cannot open ") + path);
     const size_t put = std::fwrite(buf.data(), sizeof(double), n, fp);
@@ -712,10 +721,8 @@ int glacx_measure_density(glacx_ctx *c, int field, double *q_density, double *e_
     const size_t v = (size_t)c->geom.v;
     double head[3];
     HIP_TRY(c, hipMemcpyAsync(head, c->results, sizeof head, hipMemcpyDeviceToHost, c->stream));
-    if (q_density) HIP_TRY(c, hipMemcpyAsync(q_density, c->stage, v * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    if (e_density)
-        HIP_TRY(c, hipMemcpyAsync(e_density, c->stage + v, v * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    const double *density[2] = {q_density, e_density};
+    if ((rc = copy_host(c, c->stage, density, 2, v, false))) return rc;
     if (plaq) *plaq = head[0];
     if (e_raw) *e_raw = head[1];
     if (q) *q = head[2];
@@ -840,10 +847,8 @@ int glacx_action_derivative(glacx_ctx *c, int field, int mu, double *z_out)
     if (rc) return rc;
     DISPATCH(c, launch_action_derivative, c->field[field], c->stage, c->geom, mu, c->stream);
     CHECK_LAUNCH(c);
-    HIP_TRY(c, hipMemcpyAsync(z_out, c->stage, (size_t)c->geom.v * 18 * sizeof(double), hipMemcpyDeviceToHost,
-                              c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    return GLACX_OK;
+    const double *host = z_out;
+    return copy_host(c, c->stage, &host, 1, (size_t)c->geom.v * 18, false);
 }
 
 int glacx_samples_reset(glacx_ctx *c, size_t capacity)
