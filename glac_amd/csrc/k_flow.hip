@@ -41,17 +41,33 @@ template <class T> using FlowLds = LdsMats<T, 8>;
 
 // RK3 accumulator: the 8 real parameters (a0, a1, p0..p5) of an su(3)
 // element per link, in 16-byte vectors: two float4 planes per direction in
-// FP32 (a0 a1 p0 p1 | p2 p3 p4 p5), four double2 planes in FP64.
+// FP32 (a0 a1 p0 p1 | p2 p3 p4 p5), four double2 planes in FP64.  Each link's
+// wavefront alone touches its entry, once per launch, so loads and stores are
+// non-temporal, as the stage's link stores are: they leave L2 to the links that
+// neighbouring blocks gather (FP64 24^3 x 48: 495 -> 479 us with the links'
+// stores, -> 465 with the accumulator; FP32 32^4 261 -> 256 us).
+template <class V> __device__ __forceinline__ V stream_load(const V *p)
+{
+    static_assert(sizeof(V) == 16, "16-byte vectors");
+    using U4 = unsigned __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(V, __builtin_nontemporal_load(reinterpret_cast<const U4 *>(p)));
+}
+template <class V> __device__ __forceinline__ void stream_store(V *p, const V &v)
+{
+    static_assert(sizeof(V) == 16, "16-byte vectors");
+    using U4 = unsigned __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(__builtin_bit_cast(U4, v), reinterpret_cast<U4 *>(p));
+}
 __device__ __forceinline__ void acc_store(float *acc, const Geom &g, int mu, int idx, const su3alg<float> &z)
 {
     float4 *q = reinterpret_cast<float4 *>(acc) + (size_t)mu * 2 * g.v + idx;
-    q[0] = make_float4(z.a0, z.a1, z.p[0], z.p[1]);
-    q[(size_t)g.v] = make_float4(z.p[2], z.p[3], z.p[4], z.p[5]);
+    stream_store(q, make_float4(z.a0, z.a1, z.p[0], z.p[1]));
+    stream_store(q + g.v, make_float4(z.p[2], z.p[3], z.p[4], z.p[5]));
 }
 __device__ __forceinline__ su3alg<float> acc_load(const float *acc, const Geom &g, int mu, int idx)
 {
     const float4 *q = reinterpret_cast<const float4 *>(acc) + (size_t)mu * 2 * g.v + idx;
-    const float4 u = q[0], v = q[(size_t)g.v];
+    const float4 u = stream_load(q), v = stream_load(q + g.v);
     su3alg<float> z;
     z.a0 = u.x, z.a1 = u.y, z.p[0] = u.z, z.p[1] = u.w, z.p[2] = v.x, z.p[3] = v.y, z.p[4] = v.z, z.p[5] = v.w;
     return z;
@@ -59,19 +75,19 @@ __device__ __forceinline__ su3alg<float> acc_load(const float *acc, const Geom &
 __device__ __forceinline__ void acc_store(double *acc, const Geom &g, int mu, int idx, const su3alg<double> &z)
 {
     double2 *q = reinterpret_cast<double2 *>(acc) + (size_t)mu * 4 * g.v + idx;
-    q[0] = make_double2(z.a0, z.a1);
+    stream_store(q, make_double2(z.a0, z.a1));
 #pragma unroll
-    for (int k = 0; k < 3; k++) q[(size_t)(k + 1) * g.v] = make_double2(z.p[2 * k], z.p[2 * k + 1]);
+    for (int k = 0; k < 3; k++) stream_store(q + (size_t)(k + 1) * g.v, make_double2(z.p[2 * k], z.p[2 * k + 1]));
 }
 __device__ __forceinline__ su3alg<double> acc_load(const double *acc, const Geom &g, int mu, int idx)
 {
     const double2 *q = reinterpret_cast<const double2 *>(acc) + (size_t)mu * 4 * g.v + idx;
     su3alg<double> z;
-    const double2 u = q[0];
+    const double2 u = stream_load(q);
     z.a0 = u.x, z.a1 = u.y;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        const double2 v = q[(size_t)(k + 1) * g.v];
+        const double2 v = stream_load(q + (size_t)(k + 1) * g.v);
         z.p[2 * k] = v.x, z.p[2 * k + 1] = v.y;
     }
     return z;
@@ -207,7 +223,11 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
 #pragma unroll 1
         for (int k = 0; k < 3; k++) {
             const int e = 3 * mu + k;
-            const int nu = MEAS ? (int)((kPhaseNu >> (4 * e)) & 0xF) : (mu + k + 1) & 3;
+            // FP64 plain stages: the two wavefronts of a plane reach it together, so
+            // that the upper links both of them gather come from L1 the second time
+            // (24^3 x 48 440 -> 435 us).  FP32 sums the terms in another order, which
+            // its results show in their last digits.
+            const int nu = MEAS ? (int)((kPhaseNu >> (4 * e)) & 0xF) : (sizeof(T) == 8 ? mu ^ (k + 1) : (mu + k + 1) & 3);
             const DirView<T> vnu = dir_view<T>(win, g, nu);
             const int ipn = nbr[0][nu][lane], imn = nbr[1][nu][lane];
             const int ipmmn = site_step(g, xpm, nu, -1).idx;
@@ -310,6 +330,14 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
                 mm<false, false, false, 2>(q, load_rows01<T, R>(vmu, imn), load_link<T, R>(vnu, ipmmn));
                 rebuild_third_row(q);
                 mm<true, false, true>(a, q, back_link(nu));
+            } else if constexpr (sizeof(T) == 8) {
+                // two waves per SIMD leave registers for all four gathers of the
+                // term in flight at once (230 of 256; 24^3 x 48 479 -> 454 us)
+                const M3<T> u1 = load_link<T, R>(vnu, ipm), u2 = load_link<T, R>(vmu, ipn);
+                const M3<T> l1 = load_link<T, R>(vnu, ipmmn), l2 = load_link<T, R>(vmu, imn);
+                __builtin_amdgcn_sched_barrier(0);
+                mm<false, true, true>(a, mul_ad(u1, u2), lds_get(sh, nu, lane));
+                mm<false, false, true>(a, mul_dd(l1, l2), back_link(nu));
             } else {
                 {
                     const M3<T> u1 = load_link<T, R>(vnu, ipm);
@@ -371,7 +399,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
                 orthonormalize_rows<true>(d);
             w = convert<T>(d);
         }
-        store_link<T, R>(wout, g, mu, idx, w);
+        store_link<T, R, true>(dir_view<T>(wout, g, mu), idx, w);
     }
     if constexpr (MEAS) {
         // every lane is a real site here (the launch requires whole chunks);

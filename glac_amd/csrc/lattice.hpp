@@ -363,15 +363,19 @@ __device__ __forceinline__ double2 buf_load(const DirView<double> &d, unsigned o
 {
     return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(d.r, off, k * d.plane_bytes, 0));
 }
-__device__ __forceinline__ void buf_store(const DirView<float> &d, unsigned off, int k, float2 z)
+// Stores marked `STREAM` go past L2's replacement (non-temporal): for what no
+// block of the same launch reads.
+template <bool STREAM> constexpr int store_policy() { return STREAM ? 2 : 0; }
+
+template <bool STREAM> __device__ __forceinline__ void buf_store(const DirView<float> &d, unsigned off, int k, float2 z)
 {
     using U2 = unsigned int __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, z), d.r, off, k * d.plane_bytes, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, z), d.r, off, k * d.plane_bytes, store_policy<STREAM>());
 }
-__device__ __forceinline__ void buf_store(const DirView<double> &d, unsigned off, int k, double2 z)
+template <bool STREAM> __device__ __forceinline__ void buf_store(const DirView<double> &d, unsigned off, int k, double2 z)
 {
     using U4 = unsigned int __attribute__((ext_vector_type(4)));
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, z), d.r, off, k * d.plane_bytes, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, z), d.r, off, k * d.plane_bytes, store_policy<STREAM>());
 }
 
 // Third row of an SU(3) matrix from its first two.
@@ -397,10 +401,12 @@ __device__ __forceinline__ float4 buf_load_pair(const DirView<float> &d, unsigne
 {
     return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(d.r, off16, q * 2 * d.plane_bytes, 0));
 }
+template <bool STREAM>
 __device__ __forceinline__ void buf_store_pair(const DirView<float> &d, unsigned off16, int q, float4 z)
 {
     using U4 = unsigned int __attribute__((ext_vector_type(4)));
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, z), d.r, off16, q * 2 * d.plane_bytes, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, z), d.r, off16, q * 2 * d.plane_bytes,
+                                           store_policy<STREAM>());
 }
 
 // First two rows only (row 2 left unset), for products that need no more of
@@ -453,16 +459,17 @@ template <class T, int R> __device__ __forceinline__ M3<T> load_link(const DirVi
     return m;
 }
 
-template <class T, int R> __device__ __forceinline__ void store_link(const DirView<T> &d, int idx, const M3<T> &m)
+template <class T, int R, bool STREAM = false>
+__device__ __forceinline__ void store_link(const DirView<T> &d, int idx, const M3<T> &m)
 {
     if constexpr (sizeof(T) == 4) {
         const unsigned off = (unsigned)idx * 16u;
 #pragma unroll
         for (int q = 0; q < (R == 2 ? 3 : 4); q++) {
             const cpx<T> a = m.e[(2 * q) / 3][(2 * q) % 3], b = m.e[(2 * q + 1) / 3][(2 * q + 1) % 3];
-            buf_store_pair(d, off, q, make_float4(a.r, a.i, b.r, b.i));
+            buf_store_pair<STREAM>(d, off, q, make_float4(a.r, a.i, b.r, b.i));
         }
-        if constexpr (R == 3) buf_store(d, (unsigned)idx * 8u, 8, make_float2(m.e[2][2].r, m.e[2][2].i));
+        if constexpr (R == 3) buf_store<STREAM>(d, (unsigned)idx * 8u, 8, make_float2(m.e[2][2].r, m.e[2][2].i));
     } else {
         using V2 = typename vec2<T>::type;
         const unsigned off = (unsigned)idx * (unsigned)sizeof(V2);
@@ -471,7 +478,7 @@ template <class T, int R> __device__ __forceinline__ void store_link(const DirVi
             V2 z;
             z.x = m.e[k / 3][k % 3].r;
             z.y = m.e[k / 3][k % 3].i;
-            buf_store(d, off, k, z);
+            buf_store<STREAM>(d, off, k, z);
         }
     }
 }
