@@ -31,7 +31,7 @@ struct glacx_ctx {
     size_t partials_len = 0;
     double *results = nullptr;       // device results (measurement rows)
     size_t results_len = 0;
-    unsigned long long *counts = nullptr;  // accepted hits per sweep
+    unsigned long long *counts = nullptr;  // accepted hits: kCountSlots slots per sweep, then a sum per sweep
     size_t counts_len = 0;
     int *flag = nullptr;             // one int: the SU(3) check's answer
     size_t flag_len = 0;
@@ -644,9 +644,10 @@ int glacx_metropolis(glacx_ctx *c, int n_sweeps, double beta, double eps, int n_
     if (n_sweeps < 0 || n_hit < 1 || !(eps > 0.0 && eps < 1.0))
         return fail(c, GLACX_E_ARG, "metropolis: need n_sweeps >= 0, n_hit >= 1, 0 < eps < 1");
     if (n_sweeps == 0) return GLACX_OK;
-    int rc = ensure(c, &c->counts, &c->counts_len, (size_t)n_sweeps);
+    const size_t slots = (size_t)n_sweeps * kCountSlots;
+    int rc = ensure(c, &c->counts, &c->counts_len, slots + n_sweeps);
     if (rc) return rc;
-    HIP_TRY(c, hipMemsetAsync(c->counts, 0, sizeof(unsigned long long) * n_sweeps, c->stream));
+    HIP_TRY(c, hipMemsetAsync(c->counts, 0, sizeof(unsigned long long) * slots, c->stream));
     if (plaq && (rc = ensure(c, &c->results, &c->results_len, (size_t)n_sweeps))) return rc;
     for (int i = 0; i < n_sweeps; i++) {
         MetroParams p;
@@ -656,11 +657,13 @@ int glacx_metropolis(glacx_ctx *c, int n_sweeps, double beta, double eps, int n_
         p.sweep = sweep_offset + (uint64_t)i;
         p.reunit = reunit_every > 0 && (p.sweep % (uint64_t)reunit_every) == 0;
         p.seed = seed;
-        if ((rc = DISPATCH(c, run_metropolis_sweep, c, p, c->counts + i))) return rc;
+        if ((rc = DISPATCH(c, run_metropolis_sweep, c, p, c->counts + (size_t)i * kCountSlots))) return rc;
         if (plaq && (rc = DISPATCH(c, run_plaquette, c, c->field[GLACX_FIELD_MAIN], c->results + i))) return rc;
     }
+    launch_count_sum(c->counts, c->counts + slots, n_sweeps, c->stream);
+    CHECK_LAUNCH(c);
     std::vector<unsigned long long> counts(n_sweeps);
-    HIP_TRY(c, hipMemcpyAsync(counts.data(), c->counts, sizeof(unsigned long long) * n_sweeps, hipMemcpyDeviceToHost,
+    HIP_TRY(c, hipMemcpyAsync(counts.data(), c->counts + slots, sizeof(unsigned long long) * n_sweeps, hipMemcpyDeviceToHost,
                               c->stream));
     if (plaq) HIP_TRY(c, hipMemcpyAsync(plaq, c->results, sizeof(double) * n_sweeps, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -1048,9 +1051,10 @@ int glacx_metropolis_learned(glacx_ctx *c, int n_sweeps, double beta, double eps
     if (n_sweeps < 0 || n_hit < 1 || !(eps > 0.0 && eps < 1.0))
         return fail(c, GLACX_E_ARG, "metropolis_learned: need n_sweeps >= 0, n_hit >= 1, 0 < eps < 1");
     if (n_sweeps == 0) return GLACX_OK;
-    int rc = ensure(c, &c->counts, &c->counts_len, (size_t)n_sweeps);
+    const size_t slots = (size_t)n_sweeps * kCountSlots;
+    int rc = ensure(c, &c->counts, &c->counts_len, slots + n_sweeps);
     if (rc) return rc;
-    HIP_TRY(c, hipMemsetAsync(c->counts, 0, sizeof(unsigned long long) * n_sweeps, c->stream));
+    HIP_TRY(c, hipMemsetAsync(c->counts, 0, sizeof(unsigned long long) * slots, c->stream));
     if (plaq && (rc = ensure(c, &c->results, &c->results_len, (size_t)n_sweeps))) return rc;
     for (int i = 0; i < n_sweeps; i++) {
         MetroParams p;
@@ -1060,11 +1064,13 @@ int glacx_metropolis_learned(glacx_ctx *c, int n_sweeps, double beta, double eps
         p.sweep = sweep_offset + (uint64_t)i;
         p.reunit = reunit_every > 0 && (p.sweep % (uint64_t)reunit_every) == 0;
         p.seed = seed;
-        if ((rc = DISPATCH(c, run_metropolis_learned_sweep, c, p, c->counts + i))) return rc;
+        if ((rc = DISPATCH(c, run_metropolis_learned_sweep, c, p, c->counts + (size_t)i * kCountSlots))) return rc;
         if (plaq && (rc = DISPATCH(c, run_plaquette, c, c->field[GLACX_FIELD_MAIN], c->results + i))) return rc;
     }
+    launch_count_sum(c->counts, c->counts + slots, n_sweeps, c->stream);
+    CHECK_LAUNCH(c);
     std::vector<unsigned long long> counts(n_sweeps);
-    HIP_TRY(c, hipMemcpyAsync(counts.data(), c->counts, sizeof(unsigned long long) * n_sweeps, hipMemcpyDeviceToHost,
+    HIP_TRY(c, hipMemcpyAsync(counts.data(), c->counts + slots, sizeof(unsigned long long) * n_sweeps, hipMemcpyDeviceToHost,
                               c->stream));
     if (plaq) HIP_TRY(c, hipMemcpyAsync(plaq, c->results, sizeof(double) * n_sweeps, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));

@@ -581,7 +581,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? GLACX_LEARNED_WAVES : 1) v
         }
     }
     block_sum<1>(nacc);
-    if (threadIdx.x == 0) atomicAdd(count, (unsigned long long)nacc[0]);
+    if (threadIdx.x == 0) atomicAdd(count + count_slot(blockIdx.x), (unsigned long long)nacc[0]);
 }
 
 // The sampling kernels' matrix-core forward pass on n given feature rows (6

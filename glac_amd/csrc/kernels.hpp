@@ -97,8 +97,16 @@ void launch_flow_stage(const void *win, void *wout, void *acc, const Geom &g, in
                        hipStream_t s);
 bool flow_measure_fusable(const Geom &g);
 
+// Accepted hits of a sweep are counted in kCountSlots slots, block b's in slot
+// b % kCountSlots: on one address the blocks of a small lattice, which end
+// together, queue for 5 of their 18 us (512 blocks).  launch_count_sum adds up
+// `sweeps` sweeps' slots.
+constexpr int kCountSlots = 256;
+__device__ __forceinline__ int count_slot(unsigned block) { return (int)(block & (kCountSlots - 1)); }
+void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, hipStream_t s);
+
 // One checkerboard sub-sweep (mu, parity), in place; accepted hits are added
-// to *count.
+// to the sweep's slots at `count`.
 template <class T, int R>
 void launch_metropolis(void *f, const Geom &g, int mu, int parity, const MetroParams &p,
                        unsigned long long *count, hipStream_t s);

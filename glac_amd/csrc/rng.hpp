@@ -77,7 +77,8 @@ struct Stream {
     __device__ __forceinline__ double symmetric() { return ((double)next() + 0.5) * 0x1p-31 - 1.0; }
 
     // uniform in (0, 1) with 32 bits, in double
-    __device__ __forceinline__ double open() { return ((double)next() + 0.5) * 0x1p-32; }
+    __device__ __forceinline__ double open() { return open_of(next()); }
+    static __device__ __forceinline__ double open_of(uint32_t output) { return ((double)output + 0.5) * 0x1p-32; }
 };
 
 } // namespace glacx
