@@ -162,6 +162,88 @@ template <class T> __device__ __forceinline__ FlowMeasLds<T> &flow_meas_lds()
     return s;
 }
 
+// The end of a stage for one link: RK3 combination of the force z with the
+// accumulator, exp, product with the link u, and in FP32 the projection.
+template <class T, int R, int STAGE>
+__device__ __forceinline__ void finish_link(typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc, const Geom &g,
+                                            int mu, int idx, const M3<T> &u, const su3alg<T> &z, const su3alg<T> &cacc,
+                                            T cz, T ca)
+{
+    su3alg<T> y;
+    if constexpr (STAGE == 0) {
+        acc_store(acc, g, mu, idx, z);
+        y.a0 = cz * z.a0;
+        y.a1 = cz * z.a1;
+#pragma unroll
+        for (int k = 0; k < 6; k++) y.p[k] = cz * z.p[k];
+    } else {
+        y.a0 = cz * z.a0 - ca * cacc.a0;
+        y.a1 = cz * z.a1 - ca * cacc.a1;
+#pragma unroll
+        for (int k = 0; k < 6; k++) y.p[k] = cz * z.p[k] - ca * cacc.p[k];
+        if (STAGE == 1) acc_store(acc, g, mu, idx, y);
+    }
+    M3<T> w = zero3<T>();
+    mm<false, false, false, R>(w, exp_su3(y), u);  // two rows suffice when two are stored
+    if constexpr (sizeof(T) == 4 && STAGE == 2) {
+        // FP32 links: project back onto the group in FP64 once per flow
+        // step, as the last stage stores them.  Without it the rounding of
+        // exp(Y) W drifts the links off it (|U U^dag - 1| ~ 1e-4 after 1000
+        // steps at 24^3 x 48), and that drift, not the FP32 measurement,
+        // dominates the error of E(t) at large t; within a step the two
+        // unprojected stores add two roundings (~1e-7), which the
+        // projection then removes.  Three stored rows are orthonormalised
+        // row by row, which keeps det U (GLAC's det = -1 starts stay
+        // det = -1); two stored rows are SU(3) and the third is rebuilt on
+        // load.
+        M3<double> d = convert<double>(w);
+        if constexpr (R == 2)
+            reunitarize<2, true>(d);
+        else
+            orthonormalize_rows<true>(d);
+        w = convert<T>(d);
+    }
+    store_link<T, R, true>(dir_view<T>(wout, g, mu), idx, w);
+}
+
+// Z = -1/2 T(U A), the form force_from_omega evaluates
+template <class T> __device__ __forceinline__ su3alg<T> force_from_ta2(const T (&t)[8])
+{
+    su3alg<T> z;
+    z.a0 = T(-0.5) * t[0];
+    z.a1 = T(-0.5) * t[1];
+#pragma unroll
+    for (int k = 0; k < 6; k++) z.p[k] = T(-0.5) * t[2 + k];
+    return z;
+}
+
+// The end of a measuring stage, by its four wavefronts: wavefront mu < 3 gives F
+// of its pair of planes per site, all the plaquette sums; the block's sums go
+// to its chunk's slot.
+template <class T>
+__device__ __forceinline__ void measure_block(const Geom &g, int hb, int mu, T plaq, const T (&fa)[8], const T (&fb)[8],
+                                              double *__restrict__ meas)
+{
+    double s[kMeasAcc] = {(double)plaq, 0.0, 0.0, 0.0};
+    if (mu < 3) {
+        s[1] = retrace_ta2(fa, fa) + retrace_ta2(fb, fb);
+        s[2] = -retrace_ta2(fa, fb);
+    }
+    block_sum<kMeasAcc>(s);
+    if (threadIdx.x == 0) {
+        // the block's 32 sites per parity are chunk jc of the run (blk, lt)
+        const int h0 = hb * (kFlowSites / 2);
+        const int blk = fdiv(h0, g.d_bh);
+        const int rem = h0 - blk * g.bh;
+        const int lt = fdiv(rem, g.d_run);
+        const int jc = (rem - lt * g.run) >> 5;
+        const int bt = fdiv(blk, g.d_nzb), zb = blk - bt * g.nzb;
+        double *o = meas + kMeasAcc * ((zb * g.cpr + jc) * g.n[3] + (bt << g.lbt) + lt);
+#pragma unroll
+        for (int i = 0; i < kMeasAcc; i++) o[i] = s[i];
+    }
+}
+
 // FP64 tuning knobs (build time): waves per SIMD the stage is compiled for,
 // and whether its plain stages share the backward links through LDS.
 #ifndef GLACX_FP64_FLOW_WAVES
@@ -356,79 +438,207 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
         const M3<T> u = lds_get(sh, mu, lane);
         su3alg<T> z;
         if constexpr (kCompactForce) {
-            // Z = -1/2 T(U A) (the form force_from_omega evaluates)
-            z.a0 = T(-0.5) * tz[0];
-            z.a1 = T(-0.5) * tz[1];
-#pragma unroll
-            for (int k = 0; k < 6; k++) z.p[k] = T(-0.5) * tz[2 + k];
+            z = force_from_ta2(tz);
         } else {
             z = force_from_omega(mul(u, a));
         }
-        su3alg<T> y;
-        if (STAGE == 0) {
-            acc_store(acc, g, mu, idx, z);
-            y.a0 = cz * z.a0;
-            y.a1 = cz * z.a1;
-#pragma unroll
-            for (int k = 0; k < 6; k++) y.p[k] = cz * z.p[k];
-        } else {
-            const su3alg<T> &c = cacc;
-            y.a0 = cz * z.a0 - ca * c.a0;
-            y.a1 = cz * z.a1 - ca * c.a1;
-#pragma unroll
-            for (int k = 0; k < 6; k++) y.p[k] = cz * z.p[k] - ca * c.p[k];
-            if (STAGE == 1) acc_store(acc, g, mu, idx, y);
-        }
-        M3<T> w = zero3<T>();
-        mm<false, false, false, R>(w, exp_su3(y), u);  // two rows suffice when two are stored
-        if constexpr (sizeof(T) == 4 && STAGE == 2) {
-            // FP32 links: project back onto the group in FP64 once per flow
-            // step, as the last stage stores them.  Without it the rounding of
-            // exp(Y) W drifts the links off it (|U U^dag - 1| ~ 1e-4 after 1000
-            // steps at 24^3 x 48), and that drift, not the FP32 measurement,
-            // dominates the error of E(t) at large t; within a step the two
-            // unprojected stores add two roundings (~1e-7), which the
-            // projection then removes.  Three stored rows are orthonormalised
-            // row by row, which keeps det U (GLAC's det = -1 starts stay
-            // det = -1); two stored rows are SU(3) and the third is rebuilt on
-            // load.
-            M3<double> d = convert<double>(w);
-            if constexpr (R == 2)
-                reunitarize<2, true>(d);
-            else
-                orthonormalize_rows<true>(d);
-            w = convert<T>(d);
-        }
-        store_link<T, R, true>(dir_view<T>(wout, g, mu), idx, w);
+        finish_link<T, R, STAGE>(wout, acc, g, mu, idx, u, z, cacc, cz, ca);
     }
     if constexpr (MEAS) {
         // every lane is a real site here (the launch requires whole chunks);
         // the last phase's barrier has completed every slot
-        double s[kMeasAcc] = {(double)plaq, 0.0, 0.0, 0.0};
+        T fa[8], fb[8];
         if (mu < 3) {
-            T fa[8], fb[8];
 #pragma unroll
             for (int k = 0; k < 8; k++) {
                 fa[k] = flow_meas_lds<T>().f[mu][k][lane];
                 fb[k] = flow_meas_lds<T>().f[mu + 3][k][lane];
             }
-            s[1] = retrace_ta2(fa, fa) + retrace_ta2(fb, fb);
-            s[2] = -retrace_ta2(fa, fb);
         }
-        block_sum<kMeasAcc>(s);
-        if (threadIdx.x == 0) {
-            // the block's 32 sites per parity are chunk jc of the run (blk, lt)
-            const int h0 = hb * (kFlowSites / 2);
-            const int blk = fdiv(h0, g.d_bh);
-            const int rem = h0 - blk * g.bh;
-            const int lt = fdiv(rem, g.d_run);
-            const int jc = (rem - lt * g.run) >> 5;
-            const int bt = fdiv(blk, g.d_nzb), zb = blk - bt * g.nzb;
-            double *o = meas + kMeasAcc * ((zb * g.cpr + jc) * g.n[3] + (bt << g.lbt) + lt);
+        measure_block<T>(g, hb, mu, plaq, fa, fb, meas);
+    }
+}
+
+// ---- measuring stage of a small lattice ----------------------------------------
+// Where the blocks do not fill the chip, the kernel above is four wavefronts alone
+// on their SIMDs, and its time the chain of three phases, each two gathers,
+// five to eight products and a barrier.  Here a block has twelve wavefronts:
+// wavefront (mu, k) works out mu's phase k by itself, gathering the links that the
+// kernel above shares; those of k = 1, 2 leave their part of the force in LDS, and
+// (mu, 0) adds the parts in the phases' order and finishes the link.  F's two
+// contributions per plane stand side by side instead of the later one being
+// added to the earlier.  The same sums as above.
+//
+// What bounds it: a launch and the chain gathers, products, force, exponential
+// (at 4^4 it takes hardly less than at 8^3 x 16).  Microseconds with 2 of event
+// timing, the kernel above and this one, compressed FP32, FP32 and FP64:
+//     64 blocks    14.7 11.1    16.8 12.4    18.1 17.1
+//    256 blocks    16.0 12.1    18.1 13.6    19.5 18.8
+//    768 blocks    22.2 28.9    26.4 33.7    48.2 52.1
+// For the plain stages, whose four wavefronts hold no phases, the same split gains
+// 0.6 us of 8.3 (compressed FP32) and nothing otherwise, so they have none.
+constexpr int kWideBlocks = 256;  // one block of twelve wavefronts per CU
+
+template <class T, int R> struct WideLds {
+    using V2 = typename vec2<T>::type;
+    V2 mat[R == 2 ? 4 : 1][4][R == 2 ? 9 : 1][R == 2 ? 64 : 1];  // two stored rows: a phase's two staple terms
+    T part[2][4][R == 2 ? 1 : 9][64];                           // plaquette; three: also T(U_mu (up + low))
+    T f[2][6][8][64];                                           // F of a plane: the earlier phase's part, the later's
+};
+
+template <class T, class V2> __device__ __forceinline__ void wide_put(V2 (&s)[9][64], int lane, const M3<T> &m)
+{
 #pragma unroll
-            for (int i = 0; i < kMeasAcc; i++) o[i] = s[i];
+    for (int e = 0; e < 9; e++) {
+        V2 z;
+        z.x = m.e[e / 3][e % 3].r;
+        z.y = m.e[e / 3][e % 3].i;
+        s[e][lane] = z;
+    }
+}
+template <class T, class V2> __device__ __forceinline__ M3<T> wide_get(const V2 (&s)[9][64], int lane)
+{
+    M3<T> m;
+#pragma unroll
+    for (int e = 0; e < 9; e++) m.e[e / 3][e % 3] = {s[e][lane].x, s[e][lane].y};
+    return m;
+}
+
+template <class T, int R>
+__global__ __launch_bounds__(3 * kBlock, 3) void flow_measure_wide_kernel(const typename vec2<T>::type *__restrict__ win,
+                                                                        typename vec2<T>::type *__restrict__ wout,
+                                                                        T *__restrict__ acc, Geom g, T cz,
+                                                                        double *__restrict__ meas)
+{
+    __shared__ __align__(16) WideLds<T, R> lds;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), mu = wave & 3, k = wave >> 2;
+    const int lane = threadIdx.x & 63;
+    const int hb = flow_chunk(g, xcd_block(blockIdx.x, gridDim.x));
+    // every lane is a real site (the launch requires whole chunks)
+    const int idx = parity_index(g, lane >> 5, hb * (kFlowSites / 2) + (lane & 31));
+    const Site x = site_of(g, idx);
+    const int e = 3 * mu + k, nu = (int)((kPhaseNu >> (4 * e)) & 0xF);
+    const bool first = plane_first(mu, nu);
+    const int d1 = first ? mu : nu, d2 = first ? nu : mu;
+    const DirView<T> vmu = dir_view<T>(win, g, mu), vnu = dir_view<T>(win, g, nu);
+    const Site xpm = site_step(g, x, mu, +1);
+    const int ipm = xpm.idx, ipn = site_step(g, x, nu, +1).idx, imn = site_step(g, x, nu, -1).idx;
+    const int ipmmn = site_step(g, xpm, nu, -1).idx;
+    T plaq = T(0), f[8], tz[8];
+    M3<T> a = zero3<T>();
+    {
+        // the phase's staple terms and their part of F, as above
+        M3<T> up, low;
+        if constexpr (R == 2) {
+            M3<T> p;
+            mm<false, true, false, 2>(p, load_rows01<T, R>(vnu, ipm), load_link<T, R>(vmu, ipn));
+            mm<false, true, false, 2>(up, p, load_link<T, R>(vnu, idx));
+            rebuild_third_row(up);
+            const M3<T> q = su3_product<false>(load_rows01<T, R>(vmu, imn), load_link<T, R>(vnu, ipmmn));
+            mm<true, false, false>(low, q, load_link<T, R>(vnu, imn));
+            if (k > 0) {
+                wide_put(lds.mat[2 * (k - 1)][mu], lane, up);
+                wide_put(lds.mat[2 * (k - 1) + 1][mu], lane, low);
+            } else {
+                add_to(a, up);
+                add_to(a, low);
+            }
+            const M3<T> u = load_link<T, R>(vmu, idx);
+            if (first) {
+                plaq = retrace_mul(u, up);
+                sub_from(up, low);
+                ta2_product<false>(u, up, f);
+            } else {
+                ta2_product<false>(u, low, f);
+            }
+        } else {
+            T tu[8], fl[8];
+            {
+                M3<T> p = mul_ad(load_link<T, R>(vnu, ipm), load_link<T, R>(vmu, ipn));
+                form(p);
+                mm<false, true, false>(up, p, load_link<T, R>(vnu, idx));
+                form(up);
+                const M3<T> u = load_link<T, R>(vmu, idx);
+                if (first) plaq = retrace_mul(u, up);
+                ta2_product<false>(u, up, tu);
+                form(tu);
+            }
+            {
+                M3<T> p = mul_dd(load_link<T, R>(vnu, ipmmn), load_link<T, R>(vmu, imn));
+                form(p);
+                mm<false, false, false>(low, p, load_link<T, R>(vnu, imn));
+                form(low);
+                ta2_product<false>(load_link<T, R>(vmu, idx), low, fl);
+                form(fl);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                tz[j] = tu[j] + fl[j];
+                f[j] = first ? tu[j] - fl[j] : fl[j];
+            }
+            if (k > 0) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) lds.part[k - 1][mu][1 + j][lane] = tz[j];
+            }
+        }
+        if (k > 0) lds.part[k - 1][mu][0][lane] = plaq;
+    }
+    if ((kPhaseL3 >> e) & 1) {
+        const Site xm1 = site_step(g, x, d1, -1);
+        const int i1 = xm1.idx, i2 = site_step(g, x, d2, -1).idx, iy = site_step(g, xm1, d2, -1).idx;
+        const DirView<T> v1 = first ? vmu : vnu, v2 = first ? vnu : vmu;
+        T f3[8];
+        if constexpr (R == 2) {
+            const M3<T> m1 = su3_product<false>(load_rows01<T, R>(v1, iy), load_link<T, R>(v2, i2));
+            const M3<T> m2 = su3_product<false>(load_rows01<T, R>(v2, iy), load_link<T, R>(v1, i1));
+            ta2_product<true>(m2, m1, f3);
+        } else {
+            M3<T> c1, c2;
+            mm<true, true, false>(c1, load_link<T, R>(v1, i1), load_link<T, R>(v2, iy));
+            form(c1);
+            mm<false, false, false>(c2, c1, load_link<T, R>(v1, iy));
+            form(c2);
+            mm<false, false, false>(c1, c2, load_link<T, R>(v2, i2));
+            ta2_of(c1, f3);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) f[j] += f3[j];
+    }
+    T(&fs)[8][64] = lds.f[(kPhaseAdd >> e) & 1][plane_slot(d1, d2)];
+#pragma unroll
+    for (int j = 0; j < 8; j++) fs[j][lane] = f[j];
+    __syncthreads();
+    if (k > 0) {
+        __syncthreads();  // measure_block's
+        return;
+    }
+    const M3<T> u = load_link<T, R>(vmu, idx);
+    su3alg<T> z;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        plaq += lds.part[h][mu][0][lane];
+        if constexpr (R == 2) {
+            add_to(a, wide_get<T>(lds.mat[2 * h][mu], lane));
+            add_to(a, wide_get<T>(lds.mat[2 * h + 1][mu], lane));
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; j++) tz[j] += lds.part[h][mu][1 + j][lane];
         }
     }
+    if constexpr (R == 2)
+        z = force_from_omega(mul(u, a));
+    else
+        z = force_from_ta2(tz);
+    finish_link<T, R, 0>(wout, acc, g, mu, idx, u, z, z, cz, T(0));
+    T fa[8], fb[8];
+    if (mu < 3) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            fa[j] = lds.f[0][mu][j][lane] + lds.f[1][mu][j][lane];
+            fb[j] = lds.f[0][mu + 3][j][lane] + lds.f[1][mu + 3][j][lane];
+        }
+    }
+    measure_block<T>(g, hb, mu, plaq, fa, fb, meas);
 }
 
 // Dynamic LDS reserved per block; nonzero values cap the blocks resident per
@@ -454,8 +664,11 @@ void launch_flow_stage(const void *win, void *wout, void *acc, const Geom &g, in
     switch (stage) {
     case 0:
         if (meas) {
-            flow_stage_kernel<T, R, 0, true>
-                <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), meas);
+            if (blocks <= kWideBlocks)
+                flow_measure_wide_kernel<T, R><<<blocks, 3 * kBlock, 0, s>>>(in, out, a, g, T(0.25 * eps), meas);
+            else
+                flow_stage_kernel<T, R, 0, true>
+                    <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), meas);
             break;
         }
         flow_stage_kernel<T, R, 0, false>

@@ -125,17 +125,6 @@ template <class T> __device__ __forceinline__ M3<T> get18(const T (&s)[18][64], 
     return m;
 }
 
-// Forms m here: the compiler would otherwise put the product off and hold its
-// operands, whose loads it does not move, in twice the registers.
-template <class T> __device__ __forceinline__ void form(M3<T> &m)
-{
-#pragma unroll
-    for (int e = 0; e < 9; e++) {
-        asm volatile("" : "+v"(m.e[e / 3][e % 3].r));
-        asm volatile("" : "+v"(m.e[e / 3][e % 3].i));
-    }
-}
-
 // The two terms of plane (mu, nu) of the staple at x, in the factors whose sums
 // staple() adds: with two stored rows the terms themselves; with three the
 // left factor of each term's last product.

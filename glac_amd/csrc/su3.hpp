@@ -158,6 +158,22 @@ template <class T> __device__ __forceinline__ void sub_from(M3<T> &c, const M3<T
         }
 }
 
+// Forms m here: the compiler would otherwise put the product off and hold its
+// operands, whose loads it does not move, in twice the registers.
+template <class T> __device__ __forceinline__ void form(M3<T> &m)
+{
+#pragma unroll
+    for (int e = 0; e < 9; e++) {
+        asm volatile("" : "+v"(m.e[e / 3][e % 3].r));
+        asm volatile("" : "+v"(m.e[e / 3][e % 3].i));
+    }
+}
+template <class T> __device__ __forceinline__ void form(T (&v)[8])
+{
+#pragma unroll
+    for (int k = 0; k < 8; k++) asm volatile("" : "+v"(v[k]));
+}
+
 // Re tr(A B)
 template <class T> __device__ __forceinline__ T retrace_mul(const M3<T> &a, const M3<T> &b)
 {
