@@ -36,13 +36,37 @@ template <class T, int R> __device__ __forceinline__ M3<T> reunitarized(const M3
     return convert<T>(d);
 }
 
-template <class T, int R>
-__global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 2 : 1) void metropolis_kernel(typename vec2<T>::type *__restrict__ f, Geom g, int mu,
-                                                            int parity, MetroParams prm,
-                                                            unsigned long long *__restrict__ count)
+// The wavefront's accepted hits into its slot.
+__device__ __forceinline__ void add_count(unsigned long long *count, unsigned wavefront, int n)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(count + count_slot(wavefront), (unsigned long long)n);
+}
+
+// What bounds it: FP32 the vector ALU, which is busy all the time (32^4: 5377
+// instructions in each of eight wavefronts per SIMD, 72 us at 2.4 GHz; measured
+// 70 to 72); FP64 the same unit with two wavefronts.  Wavefronts in flight: with WAVES = 3 per SIMD a block's loads
+// fall into the hits of the two others, with four all blocks of a round load
+// together and then compute together, and a last block stays alone more often;
+// once there are many rounds the blocks are out of step by themselves, and the
+// fourth pays.  Microseconds per sub-sweep by blocks per CU, three | four (four
+// with compressed links take 116 registers, which they get with no bound on
+// WAVES; bounded they are scheduled into 104 and 2 % slower):
+//     blocks per CU      4     5     6     8    10    12    16    20    40    81
+//     compressed FP32   43    49    56    70    84   103   143   178   347   693
+//                       46    52    59    73    87   105   142   176   340   678
+//     FP32              51    59    67    86   110   133   180   225   439   862
+//                       58    64    72    92   115   137   179   222   434   848
+// (FP32 with four at up to 12: 118 registers and the block's sum at the end, as
+// they were; now 127 and no sum.)
+template <class T, int R, int WAVES>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(1, WAVES))) void metropolis_kernel(
+    typename vec2<T>::type *__restrict__ f, Geom g, int mu, int parity, MetroParams prm,
+    unsigned long long *__restrict__ count)
 {
     const int h = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    double nacc[1] = {0.0};
+    int n = 0;
     if (h < g.vh) {
         const int idx = parity_index(g, parity, h);
         const Site x = site_of(g, idx);
@@ -67,10 +91,9 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 2 : 1) void metropolis_ker
         }
         if (prm.reunit) u = reunitarized<T, R>(u);
         store_link<T, R>(f, g, mu, idx, u);
-        nacc[0] = (double)accepted;
+        n = accepted;
     }
-    block_sum<1>(nacc);
-    if (threadIdx.x == 0) atomicAdd(count + count_slot(blockIdx.x), (unsigned long long)nacc[0]);
+    add_count(count, blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), n);
 }
 
 // ---- small lattices: one sub-sweep's links do not fill the chip -----------------
@@ -300,10 +323,7 @@ __global__ __launch_bounds__(64 * (STAPLERS + PROPOSERS), STAPLERS > 1 ? 4 : 2) 
         if (prm.reunit) u = reunitarized<T, R>(u);
         store_link<T, R>(f, g, mu, idx, u);
     }
-    int n = valid ? accepted : 0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
-    if (lane == 0) atomicAdd(count + count_slot(blockIdx.x), (unsigned long long)n);
+    add_count(count, blockIdx.x, valid ? accepted : 0);
 }
 
 __global__ __launch_bounds__(64) void count_sum_kernel(const unsigned long long *__restrict__ slots,
@@ -328,20 +348,22 @@ void launch_metropolis(void *f, const Geom &g, int mu, int parity, const MetroPa
                        hipStream_t s)
 {
     auto *links = (typename vec2<T>::type *)f;
-    const int groups = (g.vh + 63) / 64;
+    const int groups = (g.vh + 63) / 64, blocks = (g.vh + kBlock - 1) / kBlock;
     // the table at metropolis_small_kernel
     if constexpr (sizeof(T) == 4) {
         if (groups <= 256)
             metropolis_small_kernel<T, R, 3, 5><<<groups, 64 * 8, 0, s>>>(links, g, mu, parity, p, count);
         else if (groups <= 768)
             metropolis_small_kernel<T, R, 1, 1><<<groups, 64 * 2, 0, s>>>(links, g, mu, parity, p, count);
+        else if (blocks <= 3072)  // the table at metropolis_kernel
+            metropolis_kernel<T, R, 3><<<blocks, kBlock, 0, s>>>(links, g, mu, parity, p, count);
         else
-            metropolis_kernel<T, R><<<(g.vh + kBlock - 1) / kBlock, kBlock, 0, s>>>(links, g, mu, parity, p, count);
+            metropolis_kernel<T, R, R == 2 ? 8 : 4><<<blocks, kBlock, 0, s>>>(links, g, mu, parity, p, count);
     } else {
         if (groups <= 512)
             metropolis_small_kernel<T, R, 1, 2><<<groups, 64 * 3, 0, s>>>(links, g, mu, parity, p, count);
         else
-            metropolis_kernel<T, R><<<(g.vh + kBlock - 1) / kBlock, kBlock, 0, s>>>(links, g, mu, parity, p, count);
+            metropolis_kernel<T, R, 2><<<blocks, kBlock, 0, s>>>(links, g, mu, parity, p, count);
     }
 }
 
