@@ -503,9 +503,15 @@ __global__ __launch_bounds__(kBlock) void to_bf16_kernel(const float *__restrict
 }
 
 // ---- sampling with the learned proposal ----------------------------------------
+// What bounds it: the vector ALU (7500 instructions a wavefront, three quarters
+// of the time) and, beside it, LDS.  Against outputs and weights in plain rows
+// (a sixth of the time went to bank conflicts) and a parameter at a time into
+// LDS before the staple's loads: 24^3x48 79.5 -> 76.5 us a sub-sweep, 32^4 102 ->
+// 99, 32^3x8 43 -> 38.5.
 // Waves per SIMD the FP32 sampling kernel is compiled for (build-time tuning):
 // four fit 128 VGPRs and, with the network's output buffer at 32 floats per
-// link, 38.7 KB of LDS per block.
+// link, 38.7 KB of LDS per block.  Three are 3 % ahead at five or six blocks per
+// CU and 3 % behind from twelve on.
 #ifndef GLACX_LEARNED_WAVES
 #define GLACX_LEARNED_WAVES 4
 #endif
@@ -519,7 +525,6 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? GLACX_LEARNED_WAVES : 1) v
     __shared__ __align__(16) MlpImage im;
     __shared__ __align__(16) float obuf[kBlock / 64][64 * kMlpObuf];
     mlp_image_fill(im, wbf16, threadIdx.x, kBlock);
-    __syncthreads();
     const int h_raw = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
     const bool valid = h_raw < g.vh;
     const int h = valid ? h_raw : g.vh - 1;  // idle lanes mirror a real link for the network GEMMs, store nothing
@@ -531,6 +536,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? GLACX_LEARNED_WAVES : 1) v
         M3<T> u = load_link<T, R>(f, g, mu, idx);
         float fe[6], o[36], L[36];
         staple_features(a, prm.beta, fe);
+        __syncthreads();  // the image is whole; its loads travelled beside the staple's
         const bool learned =
             mlp_forward_mfma(im, mean_std, mean_std + 6, fe, obuf[threadIdx.x >> 6], o);  // whole wavefront
         cholesky_from_output(o, L);

@@ -97,7 +97,10 @@ __device__ __forceinline__ bf16x4 lrelu_bf16(const f32x4 &d)
 }
 // The network's parameters as the GEMMs read them (bf16 bits, zero padded so
 // every fragment is one aligned 8-byte LDS read): W1 with rows of 8, W3 and
-// b3 with 48 rows.
+// b3 with 48 rows.  Rows of W2 and W3 are sixteen banks long, so the sixteen
+// rows of a fragment read meet in the banks four at a time; with the two halves
+// of a row exchanged in every second group of four rows (mlp_col) they use all
+// 64 banks.
 struct MlpImage {
     unsigned short w1[kMlpH1][8];
     unsigned short b1[kMlpH1];
@@ -106,33 +109,31 @@ struct MlpImage {
     unsigned short w3[48][kMlpH2];
     unsigned short b3[48];
 };
+static_assert(kMlpH1 == 32 && kMlpH2 == 32, "rows of W2 and W3 are two halves of sixteen");
+// where column c of a row of W2 or W3 stands
+__device__ __forceinline__ int mlp_col(int row, int c) { return c ^ ((row & 4) << 2); }
 
-// Fill the image from the packed bf16 parameters (all threads of a block).
+// Fill the image from the packed bf16 parameters (all threads of a block), two
+// parameters at a time: every matrix row and bias starts at an even parameter.
+// The caller passes a barrier before the image is read.
 __device__ __forceinline__ void mlp_image_fill(MlpImage &im, const unsigned short *__restrict__ wbf16, int tid,
                                                int nthreads)
 {
-    unsigned short *dst = &im.w1[0][0];
-    constexpr int n = (int)(sizeof(MlpImage) / sizeof(unsigned short));
-    for (int k = tid; k < n; k += nthreads) {
-        int src = -1;
-        if (k < kMlpH1 * 8) {
-            const int r = k >> 3, c = k & 7;
-            src = c < kMlpIn ? kOffW1 + r * kMlpIn + c : -1;
-        } else if (k < kMlpH1 * 9) {
-            src = kOffB1 + (k - kMlpH1 * 8);
-        } else if (k < kMlpH1 * 9 + kMlpH2 * kMlpH1) {
-            src = kOffW2 + (k - kMlpH1 * 9);
-        } else if (k < kMlpH1 * 9 + kMlpH2 * (kMlpH1 + 1)) {
-            src = kOffB2 + (k - kMlpH1 * 9 - kMlpH2 * kMlpH1);
-        } else if (k < kMlpH1 * 9 + kMlpH2 * (kMlpH1 + 1) + 48 * kMlpH2) {
-            const int j = k - (kMlpH1 * 9 + kMlpH2 * (kMlpH1 + 1));
-            src = (j >> 5) < kMlpOut ? kOffW3 + j : -1;
-        } else {
-            const int j = k - (kMlpH1 * 9 + kMlpH2 * (kMlpH1 + 1) + 48 * kMlpH2);
-            src = j < kMlpOut ? kOffB3 + j : -1;
-        }
-        dst[k] = src >= 0 ? wbf16[src] : (unsigned short)0;
-    }
+    static_assert((kMlpIn | kOffB1 | kOffW2 | kOffB2 | kOffW3 | kOffB3 | kMlpOut) % 2 == 0, "pairs of parameters");
+    const unsigned *src = reinterpret_cast<const unsigned *>(wbf16);
+    const auto put = [](unsigned short *p, unsigned v) { *reinterpret_cast<unsigned *>(p) = v; };
+    for (int k = tid; k < kMlpH1 * 4; k += nthreads)
+        put(&im.w1[0][0] + 2 * k, (k & 3) < kMlpIn / 2 ? src[(k >> 2) * (kMlpIn / 2) + (k & 3)] : 0u);
+    for (int k = tid; k < kMlpH2 * 16; k += nthreads)
+        put(&im.w2[k >> 4][mlp_col(k >> 4, 2 * (k & 15))], src[kOffW2 / 2 + k]);
+    for (int k = tid; k < 48 * 16; k += nthreads)
+        put(&im.w3[k >> 4][mlp_col(k >> 4, 2 * (k & 15))], (k >> 4) < kMlpOut ? src[kOffW3 / 2 + k] : 0u);
+    if (tid < 16)
+        put(&im.b1[2 * tid], src[kOffB1 / 2 + tid]);
+    else if (tid < 32)
+        put(&im.b2[2 * (tid - 16)], src[kOffB2 / 2 + tid - 16]);
+    else if (tid < 56)
+        put(&im.b3[2 * (tid - 32)], tid - 32 < kMlpOut / 2 ? src[kOffB3 / 2 + tid - 32] : 0u);
 }
 
 __device__ __forceinline__ bf16x4 lds_frag(const unsigned short *p)
@@ -147,6 +148,11 @@ __device__ __forceinline__ f32x4 lds_bias(const unsigned short *p)
     for (int e = 0; e < 4; e++) c[e] = __uint_as_float((unsigned)((v >> (16 * e)) & 0xFFFFu) << 16);
     return c;
 }
+
+// Where outputs o .. o + 3 (o a multiple of four) of a wavefront's link stand in
+// its LDS buffer: the eight groups of four are permuted from link to link, since
+// at one place in every link's 32 floats they would all be in the same banks.
+__device__ __forceinline__ int mlp_out(int link, int o) { return link * kMlpObuf + (o ^ ((link & 7) << 2)); }
 
 // Network outputs o[36] of this lane's link; every lane of the wavefront must
 // call it (the GEMMs span the wavefront).  im: the parameter image (LDS),
@@ -182,19 +188,19 @@ __device__ __forceinline__ bool mlp_forward_mfma(const MlpImage &im, const float
         }
 #pragma unroll
         for (int m = 0; m < 2; m++) {
-            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w2[16 * m + row][4 * grp]), a1[0],
+            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w2[16 * m + row][mlp_col(row, 4 * grp)]), a1[0],
                                                                 lds_bias(&im.b2[16 * m + 4 * grp]), 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w2[16 * m + row][16 + 4 * grp]), a1[1], d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w2[16 * m + row][mlp_col(row, 16 + 4 * grp)]), a1[1], d, 0, 0, 0);
             a2[m] = lrelu_bf16(d);
         }
 #pragma unroll
         for (int m = 0; m < 3; m++) {
-            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w3[16 * m + row][4 * grp]), a2[0],
+            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w3[16 * m + row][mlp_col(row, 4 * grp)]), a2[0],
                                                                 lds_bias(&im.b3[16 * m + 4 * grp]), 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w3[16 * m + row][16 + 4 * grp]), a2[1], d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w3[16 * m + row][mlp_col(row, 16 + 4 * grp)]), a2[1], d, 0, 0, 0);
             const int r0 = 16 * m + 4 * grp;
             if (m < 2) {
-                *reinterpret_cast<f32x4 *>(obuf + (16 * nt + row) * kMlpObuf + r0) = d;
+                *reinterpret_cast<f32x4 *>(obuf + mlp_out(16 * nt + row, r0)) = d;
             } else {
                 // outputs 32..35 of link 16 nt + row sit in lane row (grp 0):
                 // the link's own lane takes them by shuffles
@@ -211,7 +217,7 @@ __device__ __forceinline__ bool mlp_forward_mfma(const MlpImage &im, const float
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int i = 0; i < kMlpObuf; i += 4) {
-        const f32x4 v = *reinterpret_cast<const f32x4 *>(obuf + lane * kMlpObuf + i);
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(obuf + mlp_out(lane, i));
         o[i] = v[0];
         o[i + 1] = v[1];
         o[i + 2] = v[2];
