@@ -42,37 +42,30 @@ __device__ __forceinline__ void su2_near_unity(const T r0, const T r1, const T r
     b = {x2, x1};
 }
 
-// X = R S T with r in block (0,1), s in block (0,2), t in block (1,2).
+// X = R S T with r in block (0,1), s in block (0,2), t in block (1,2), each
+// [[a, b], [-conj(b), conj(a)]] there.  Which product of a pair is rounded before
+// the other is added is written out, so that a proposal has the same bits in
+// every kernel: a chain follows its seed whichever of them a lattice's size picks.
 template <class T>
 __device__ __forceinline__ M3<T> rst_product(cpx<T> ra, cpx<T> rb, cpx<T> sa, cpx<T> sb, cpx<T> ta, cpx<T> tb)
 {
-    // 2x2 entries: m00 = a, m01 = b, m10 = -conj(b), m11 = conj(a)
-    const cpx<T> r00 = ra, r01 = rb, r10 = {-rb.r, rb.i}, r11 = {ra.r, -ra.i};
-    const cpx<T> s00 = sa, s01 = sb, s10 = {-sb.r, sb.i}, s11 = {sa.r, -sa.i};
-    const cpx<T> t00 = ta, t01 = tb, t10 = {-tb.r, tb.i}, t11 = {ta.r, -ta.i};
-    const cpx<T> r00s01 = cmul(r00, s01), r10s01 = cmul(r10, s01);
+    // R_00 S_01 and R_10 S_01
+    const T pr = fma(ra.r, sb.r, -(ra.i * sb.i)), pi = fma(ra.r, sb.i, ra.i * sb.r);
+    const T qr = fma(-rb.r, sb.r, -(rb.i * sb.i)), qi = fma(rb.i, sb.r, -(rb.r * sb.i));
     M3<T> x;
-    x.e[0][0] = cmul(r00, s00);
-    {
-        const cpx<T> u = cmul(r01, t00), v = cmul(r00s01, t10);
-        x.e[0][1] = {u.r + v.r, u.i + v.i};
-    }
-    {
-        const cpx<T> u = cmul(r01, t01), v = cmul(r00s01, t11);
-        x.e[0][2] = {u.r + v.r, u.i + v.i};
-    }
-    x.e[1][0] = cmul(r10, s00);
-    {
-        const cpx<T> u = cmul(r11, t00), v = cmul(r10s01, t10);
-        x.e[1][1] = {u.r + v.r, u.i + v.i};
-    }
-    {
-        const cpx<T> u = cmul(r11, t01), v = cmul(r10s01, t11);
-        x.e[1][2] = {u.r + v.r, u.i + v.i};
-    }
-    x.e[2][0] = s10;
-    x.e[2][1] = cmul(s11, t10);
-    x.e[2][2] = cmul(s11, t11);
+    x.e[0][0] = {fma(ra.r, sa.r, -(ra.i * sa.i)), fma(ra.i, sa.r, ra.r * sa.i)};
+    x.e[0][1] = {fma(rb.r, ta.r, -(rb.i * ta.i)) + fma(-tb.r, pr, -(tb.i * pi)),
+                 fma(rb.i, ta.r, rb.r * ta.i) + fma(tb.i, pr, -(tb.r * pi))};
+    x.e[0][2] = {fma(rb.r, tb.r, -(rb.i * tb.i)) + fma(pr, ta.r, ta.i * pi),
+                 fma(rb.r, tb.i, rb.i * tb.r) + fma(pi, ta.r, -(ta.i * pr))};
+    x.e[1][0] = {fma(-rb.r, sa.r, -(rb.i * sa.i)), fma(rb.i, sa.r, -(rb.r * sa.i))};
+    x.e[1][1] = {fma(ra.r, ta.r, ra.i * ta.i) + fma(-tb.r, qr, -(tb.i * qi)),
+                 fma(ra.r, ta.i, -(ra.i * ta.r)) + fma(tb.i, qr, -(tb.r * qi))};
+    x.e[1][2] = {fma(ra.r, tb.r, ra.i * tb.i) + fma(qr, ta.r, ta.i * qi),
+                 fma(ra.r, tb.i, -(ra.i * tb.r)) + fma(qi, ta.r, -(ta.i * qr))};
+    x.e[2][0] = {-sb.r, sb.i};
+    x.e[2][1] = {fma(sa.i, tb.i, -(sa.r * tb.r)), fma(sa.r, tb.i, sa.i * tb.r)};
+    x.e[2][2] = {fma(sa.r, ta.r, -(sa.i * ta.i)), fma(-sa.i, ta.r, -(sa.r * ta.i))};
     return x;
 }
 
