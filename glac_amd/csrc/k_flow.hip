@@ -271,10 +271,11 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
     const int h = valid ? h_raw : g.vh - 1;  // idle lanes of a partial block mirror a real site, store nothing
     const int idx = parity_index(g, lane >> 5, h);
     const Site x = site_of(g, idx);
-    // stages 1 and 2 read the link's accumulator now, so that its latency
-    // passes under the staple loop instead of stalling the step after it
+    // FP32: stages 1 and 2 read the link's accumulator now, so that its latency
+    // passes under the staple loop instead of stalling the step after it; FP64 has
+    // no registers left for it (with it in place early, 504 for 391 us)
     su3alg<T> cacc;
-    if constexpr (STAGE != 0) cacc = acc_load(acc, g, mu, idx);
+    if constexpr (STAGE != 0 && sizeof(T) == 4) cacc = acc_load(acc, g, mu, idx);
     const DirView<T> vmu = dir_view<T>(win, g, mu);
     // the site's neighbours x + mu and x - mu, shared with the other
     // wavefronts, whose staples step the same way in direction mu
@@ -293,6 +294,38 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
             return lds_get(sh, 4 + d, lane);
         else
             return load_link<T, R>(dir_view<T>(win, g, d), nbr[1][d][lane]);
+    };
+    // FP64 plain stages: the x- and y-neighbours that are sites of this block, whose
+    // own links are in LDS (with the block's sites in two whole runs of entries:
+    // nearly every x-neighbour, and half the y-neighbours).  near_slot: such a
+    // site's slot, -1 for the others; gather: the link, unless it is there;
+    // take_near: the link, if it is.  These stages are bound by the lines a CU's L1
+    // can have on their way at a time (load the links and multiply nothing, and
+    // they take as long); this saves a fifth of the requests: 24^3 x 48 415 -> 391
+    // and 387 -> 360 us.  The measuring stage has no registers for it (596 -> 645).
+    constexpr bool kNear = sizeof(T) == 8 && !MEAS;
+    const bool near = kNear && (g.bh & 31) == 0;
+    const int base0 = kNear ? parity_index(g, 0, hb * (kFlowSites / 2)) : 0, base1 = base0 + g.bh;
+    auto near_slot = [&](bool xy, int at, bool same_parity) -> int {
+        if (!near || !xy) return -1;
+        const int p = (lane >> 5) ^ (same_parity ? 0 : 1), r = at - (p ? base1 : base0);
+        return (unsigned)r < 32u ? p * 32 + r : -1;
+    };
+    auto gather = [&](const DirView<T> &d, int at, int slot) -> M3<T> {
+        if constexpr (kNear)
+            return load_link_at(d, slot >= 0 ? kNoLink : tile_off(at));
+        else
+            return load_link<T, R>(d, at);
+    };
+    auto take_near = [&](M3<T> &m, bool xy, int d, int slot) {
+        if (near && xy) {
+            const M3<T> n = lds_get(sh, d, slot >= 0 ? slot : lane);
+#pragma unroll
+            for (int e = 0; e < 9; e++) {
+                m.e[e / 3][e % 3].r = slot >= 0 ? n.e[e / 3][e % 3].r : m.e[e / 3][e % 3].r;
+                m.e[e / 3][e % 3].i = slot >= 0 ? n.e[e / 3][e % 3].i : m.e[e / 3][e % 3].i;
+            }
+        }
     };
     // staple A_mu(x) = sum_{nu != mu} [ U_nu(x+mu) U_mu(x+nu)^dag U_nu(x)^dag
     //                                 + U_nu(x+mu-nu)^dag U_mu(x-nu)^dag U_nu(x-nu) ]
@@ -414,11 +447,17 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
                 mm<true, false, true>(a, q, back_link(nu));
             } else if constexpr (sizeof(T) == 8) {
                 // two waves per SIMD leave registers for all four gathers of the
-                // term in flight at once (230 of 256; 24^3 x 48 479 -> 454 us)
-                const M3<T> u1 = load_link<T, R>(vnu, ipm), u2 = load_link<T, R>(vmu, ipn);
-                const M3<T> l1 = load_link<T, R>(vnu, ipmmn), l2 = load_link<T, R>(vmu, imn);
+                // term in flight at once (24^3 x 48 479 -> 454 us)
+                const int sm = near_slot(mu < 2, ipm, false), sp = near_slot(nu < 2, ipn, false),
+                          sn = near_slot(nu < 2, imn, false), sc = near_slot(mu < 2 && nu < 2, ipmmn, true);
+                M3<T> u1 = gather(vnu, ipm, sm), u2 = gather(vmu, ipn, sp);
+                M3<T> l1 = gather(vnu, ipmmn, sc), l2 = gather(vmu, imn, sn);
                 __builtin_amdgcn_sched_barrier(0);
+                take_near(u1, mu < 2, nu, sm);
+                take_near(u2, nu < 2, mu, sp);
                 mm<false, true, true>(a, mul_ad(u1, u2), lds_get(sh, nu, lane));
+                take_near(l1, mu < 2 && nu < 2, nu, sc);
+                take_near(l2, nu < 2, mu, sn);
                 mm<false, false, true>(a, mul_dd(l1, l2), back_link(nu));
             } else {
                 {
@@ -434,6 +473,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
             }
         }
     }
+    if constexpr (STAGE != 0 && sizeof(T) == 8) cacc = acc_load(acc, g, mu, idx);
     if (valid) {
         const M3<T> u = lds_get(sh, mu, lane);
         su3alg<T> z;

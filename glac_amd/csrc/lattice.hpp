@@ -22,9 +22,8 @@
 // where plain rows would put it a whole 3D slice away.
 //
 // A field is four direction regions of 9 V complex entries (mu-major).  In
-// FP64 each region is 9 planes, entry (i, j) of U_mu at idx at
-// plane[(mu * 9 + 3 i + j) * V + idx]; FP32 pairs entries into float4 planes
-// (see load_rows01 below).
+// FP64 a region lies in tiles of 16 indices (see tile_off below); FP32 pairs
+// entries into float4 planes (see load_rows01 below).
 //
 // GLAC's shift() and Communicator link getters (GLAC/math/lattice.h:824-1144,
 // GLAC/parallelization/communicator.cpp:83-258) become the index arithmetic
@@ -324,12 +323,13 @@ template <> struct vec2<double> {
     using type = double2;
 };
 
-// Field access.  The 9 complex planes of one direction mu are addressed
-// through one buffer resource (base = plane (mu, 0), range 9 V entries, in
-// scalar registers when mu is wave-uniform); a link load is then 9
-// buffer_load_dwordx2/x4 with the per-lane byte offset idx * sizeof(V2) in a
-// VGPR and the plane offset k V sizeof(V2) in an SGPR -- no per-load address
-// arithmetic.  The context limits 9 V sizeof(V2) to below 2^32 bytes.
+// Field access.  The 9 V complex entries of one direction mu are addressed
+// through one buffer resource (base = its first entry, range 9 V entries, in
+// scalar registers when mu is wave-uniform).  An FP32 link load is then four or
+// five buffer loads with one per-lane byte offset and the plane offset in an
+// SGPR -- no per-load address arithmetic; an FP64 link's nine differ by
+// constants in the instruction.  The context limits 9 V sizeof(V2) to below
+// 2^32 bytes.
 //
 // Stored rows R (a template parameter of every kernel that touches links):
 // R = 3 stores the whole matrix; R = 2 (the compressed FP32 mode) stores and
@@ -339,9 +339,26 @@ template <> struct vec2<double> {
 // is then never moved.
 constexpr int kBufferFlags = 0x00020000;  // gfx9 raw buffer: 32-bit data format, no swizzle
 
+// FP64 links lie in tiles: the links of 16 consecutive indices side by side,
+// entry e = 3 i + j of all 16 as one run of 256 bytes (V is a multiple of 16, as
+// every extent is even).  A link's nine loads then fall into 2.3 KB instead of
+// nine planes V apart, which L2 and what lies behind it answer faster
+// (24^3 x 48: flow stages 437 -> 415 and 405 -> 387 us, the measuring one
+// 612 -> 596, clover 403 -> 390; tiles of 32 420 and 390; of 8 as of 16; of 4
+// clover 430).  FP32 links, whose kernels the vector ALU bounds, keep planes of V
+// entries, one shift away from the index (in tiles the stages of 32^4 were 1 %
+// slower).
+constexpr int kTile = 16;
+// byte offset of an index's first FP64 entry
+__host__ __device__ __forceinline__ unsigned tile_off(int idx)
+{
+    return ((unsigned)idx / kTile) * (unsigned)(kTile * 144) + ((unsigned)idx % kTile) * 16u;
+}
+constexpr int kTileRun = kTile * 16;  // bytes from one entry of a tile's links to the next
+
 template <class T> struct DirView {
     __amdgpu_buffer_rsrc_t r;
-    int plane_bytes;
+    int plane_bytes;  // FP32
 };
 
 template <class T>
@@ -361,7 +378,7 @@ __device__ __forceinline__ float2 buf_load(const DirView<float> &d, unsigned off
 }
 __device__ __forceinline__ double2 buf_load(const DirView<double> &d, unsigned off, int k)
 {
-    return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(d.r, off, k * d.plane_bytes, 0));
+    return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(d.r, off + k * kTileRun, 0, 0));
 }
 // Stores marked `STREAM` go past L2's replacement (non-temporal): for what no
 // block of the same launch reads.
@@ -375,7 +392,7 @@ template <bool STREAM> __device__ __forceinline__ void buf_store(const DirView<f
 template <bool STREAM> __device__ __forceinline__ void buf_store(const DirView<double> &d, unsigned off, int k, double2 z)
 {
     using U4 = unsigned int __attribute__((ext_vector_type(4)));
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, z), d.r, off, k * d.plane_bytes, store_policy<STREAM>());
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, z), d.r, off + k * kTileRun, 0, store_policy<STREAM>());
 }
 
 // Third row of an SU(3) matrix from its first two.
@@ -396,7 +413,7 @@ template <class T> __host__ __device__ __forceinline__ void rebuild_third_row(M3
 // are three 16-byte loads; with three stored rows a fourth pair holds
 // entries 6, 7 and entry 8 follows as a float2 plane (byte offset 64 V).  The
 // direction's region is 72 V bytes either way; compressed links (R = 2) use
-// its first 48 V.  FP64 links keep one double2 plane per entry.
+// its first 48 V.
 __device__ __forceinline__ float4 buf_load_pair(const DirView<float> &d, unsigned off16, int q)
 {
     return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(d.r, off16, q * 2 * d.plane_bytes, 0));
@@ -424,7 +441,7 @@ template <class T, int R> __device__ __forceinline__ M3<T> load_rows01(const Dir
         }
     } else {
         using V2 = typename vec2<T>::type;
-        const unsigned off = (unsigned)idx * (unsigned)sizeof(V2);
+        const unsigned off = tile_off(idx);
 #pragma unroll
         for (int k = 0; k < 6; k++) {
             const V2 z = buf_load(d, off, k);
@@ -449,12 +466,26 @@ template <class T, int R> __device__ __forceinline__ M3<T> load_link(const DirVi
         m.e[2][2] = {w.x, w.y};
     } else {
         using V2 = typename vec2<T>::type;
-        const unsigned off = (unsigned)idx * (unsigned)sizeof(V2);
+        const unsigned off = tile_off(idx);
 #pragma unroll
         for (int k = 6; k < 9; k++) {
             const V2 z = buf_load(d, off, k);
             m.e[2][k - 6] = {z.x, z.y};
         }
+    }
+    return m;
+}
+
+// FP64: the link whose first entry is `off` bytes into the direction, or with
+// kNoLink, which no entry's bytes reach, none: the loads ask for nothing.
+constexpr unsigned kNoLink = 0xFFFFF000u;
+__device__ __forceinline__ M3<double> load_link_at(const DirView<double> &d, unsigned off)
+{
+    M3<double> m;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const double2 z = buf_load(d, off, k);
+        m.e[k / 3][k % 3] = {z.x, z.y};
     }
     return m;
 }
@@ -472,7 +503,7 @@ __device__ __forceinline__ void store_link(const DirView<T> &d, int idx, const M
         if constexpr (R == 3) buf_store<STREAM>(d, (unsigned)idx * 8u, 8, make_float2(m.e[2][2].r, m.e[2][2].i));
     } else {
         using V2 = typename vec2<T>::type;
-        const unsigned off = (unsigned)idx * (unsigned)sizeof(V2);
+        const unsigned off = tile_off(idx);
 #pragma unroll
         for (int k = 0; k < 9; k++) {
             V2 z;
@@ -515,7 +546,7 @@ __device__ __forceinline__ void store_link_any(typename vec2<T>::type *__restric
             typename vec2<T>::type z;
             z.x = m.e[k / 3][k % 3].r;
             z.y = m.e[k / 3][k % 3].i;
-            p[(size_t)k * g.v + idx] = z;
+            *reinterpret_cast<typename vec2<T>::type *>(reinterpret_cast<char *>(p) + tile_off(idx) + k * kTileRun) = z;
         }
     }
 }
