@@ -114,22 +114,19 @@ __device__ __forceinline__ su3alg<double> acc_load(const double *acc, const Geom
 // one extra product per term, and the L3 leaves are dealt 2, 2, 1, 1.
 //
 // F of a plane is 8 reals {Im F00, Im F11, F01, F02, F12} in one LDS slot
-// per plane.  The three staple terms run as three phases separated by
-// barriers, in a per-wavefront order chosen so that the two wavefronts of a
-// plane reach it in different phases: the earlier one stores its
-// contribution, the later one adds its own to it.  No atomics, and the sum
-// of the two is formed in a fixed order.  The L3 leaves go two per phase.
-// After the last phase wavefront w < 3 evaluates the pair (w, w + 3) =
-// ((0, w+1), (rho, sigma)) per site as the clover kernel does:
+// per plane.  The three staple terms run as three phases, in a per-wavefront
+// order in which the two wavefronts of a plane reach it in different phases: the
+// earlier one stores its contribution, the later one holds its own back and adds
+// it when all three phases of all are done, so that no wavefront waits for
+// another between them (with a barrier after each phase and the sum formed there,
+// 32^4 compressed took 398 us for 378, 48^3 x 96 4120 for 3750; the barrier stands
+// before the exponential, whose registers are then free of what was held: behind
+// it 389).  No atomics, and the sum of the two is formed in a fixed order.  The L3
+// leaves go two per phase.  At the end wavefront w < 3 evaluates the pair
+// (w, w + 3) = ((0, w+1), (rho, sigma)) per site as the clover kernel does:
 //   E += Re tr(F_a F_a) + Re tr(F_b F_b),  q -= Re tr(F_a F_b),
 // and the plaquette sum takes Re tr L1 of each plane from its first-index
 // wavefront.  The block's sums go to the clover kernel's (chunk, t) slot.
-
-// With FP64 links the F slots (24.6 KB per block) and the eight shared links
-// (73.7 KB) would leave room for one block per CU; the FP64 measuring stage
-// therefore shares only U_mu(x) through LDS and gathers the backward links
-// U_nu(x - nu) from memory (four more gathers per link), which keeps it at
-// two blocks per CU.
 
 // Slot of GLAC's plane {d1, d2} stored as (d1, d2): 0..2 = (0, nu), 3 = (2,3),
 // 4 = (3,1), 5 = (1,2); (mu, nu) is stored as such when mu = 0 or nu = mu % 3 + 1.
@@ -137,7 +134,7 @@ __device__ __forceinline__ bool plane_first(int mu, int nu) { return mu == 0 || 
 __device__ __forceinline__ int plane_slot(int d1, int d2) { return d1 == 0 ? d2 - 1 : (d1 == 1 ? 5 : d1 + 1); }
 // Phase schedule, entry e = 3 mu + k for wavefront mu in phase k:
 //   kPhaseNu:  the term nu (4 bits each): mu 0: 1 2 3, mu 1: 2 0 3, mu 2: 0 3 1, mu 3: 0 1 2
-//   kPhaseAdd: the plane's other wavefront stored first (add to the slot)
+//   kPhaseAdd: the plane's other wavefront stored first (hold, and add at the end)
 //   kPhaseL3:  this wavefront also adds the plane's L3 leaf
 constexpr unsigned long long kPhaseNu = 0x210130302321ull;
 constexpr unsigned kPhaseAdd = 0x936u;  // entries 1 2 4 5 8 11
@@ -244,25 +241,19 @@ __device__ __forceinline__ void measure_block(const Geom &g, int hb, int mu, T p
     }
 }
 
-// FP64 tuning knobs (build time): waves per SIMD the stage is compiled for,
-// and whether its plain stages share the backward links through LDS.
+// FP64 tuning knob (build time): waves per SIMD the plain stages are compiled for.
 #ifndef GLACX_FP64_FLOW_WAVES
 #define GLACX_FP64_FLOW_WAVES 2
 #endif
-#ifndef GLACX_FP64_BACK_LDS
-#define GLACX_FP64_BACK_LDS 1
-#endif
 
 template <class T, int R, int STAGE, bool MEAS>
-__global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2 : GLACX_FP64_FLOW_WAVES)) void flow_stage_kernel(const typename vec2<T>::type *__restrict__ win,
+__global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP64_FLOW_WAVES) void flow_stage_kernel(const typename vec2<T>::type *__restrict__ win,
                                                             typename vec2<T>::type *__restrict__ wout,
                                                             T *__restrict__ acc, Geom g, T cz, T ca,
                                                             double *__restrict__ meas)
 {
-    static_assert(!MEAS || STAGE == 0, "the measurement is fused into stage 0 only");
-    // backward links U_nu(x - nu) shared through LDS, except in the FP64 measuring stage
-    constexpr bool BACK_LDS = !(sizeof(T) == 8 && (MEAS || !GLACX_FP64_BACK_LDS));
-    __shared__ LdsMats<T, BACK_LDS ? 8 : 4> sh;
+    static_assert(!MEAS || (STAGE == 0 && sizeof(T) == 4), "the measurement is fused into stage 0 only, FP64 has its own");
+    __shared__ FlowLds<T> sh;
     const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // one direction per wavefront
     const int lane = threadIdx.x & 63;
     const int hb = flow_chunk(g, xcd_block(blockIdx.x, gridDim.x));
@@ -285,16 +276,10 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
     nbr[0][mu][lane] = ipm;
     nbr[1][mu][lane] = imm;
     lds_put(sh, mu, lane, load_link<T, R>(vmu, idx));
-    if constexpr (BACK_LDS) lds_put(sh, 4 + mu, lane, load_link<T, R>(vmu, imm));
+    lds_put(sh, 4 + mu, lane, load_link<T, R>(vmu, imm));
     T plaq = T(0);
     __syncthreads();
-    // U_d(x - d), from LDS or gathered (x - d from the wavefront of d)
-    auto back_link = [&](int d) -> M3<T> {
-        if constexpr (BACK_LDS)
-            return lds_get(sh, 4 + d, lane);
-        else
-            return load_link<T, R>(dir_view<T>(win, g, d), nbr[1][d][lane]);
-    };
+    auto back_link = [&](int d) -> M3<T> { return lds_get(sh, 4 + d, lane); };  // U_d(x - d)
     // FP64 plain stages: the x- and y-neighbours that are sites of this block, whose
     // own links are in LDS (with the block's sites in two whole runs of entries:
     // nearly every x-neighbour, and half the y-neighbours).  near_slot: such a
@@ -334,6 +319,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
     // measuring stage with three stored rows: T(U_mu(x) A_mu(x)) in compact form
     constexpr bool kCompactForce = MEAS && R == 3;
     T tz[8] = {T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
+    T held[2][8];  // measuring stage: see the end of a phase
     {
 #pragma unroll 1
         for (int k = 0; k < 3; k++) {
@@ -420,14 +406,21 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
 #pragma unroll
                     for (int j = 0; j < 8; j++) f[j] += f3[j];
                 }
-                T(&fs)[8][kFlowSites] = flow_meas_lds<T>().f[slot];
+                // the plane's earlier contribution goes to its slot now, the later one
+                // is held back and added once all the earlier ones are there
                 if ((kPhaseAdd >> e) & 1) {
+                    if (k == 1) {
 #pragma unroll
-                    for (int j = 0; j < 8; j++) f[j] = fs[j][lane] + f[j];
+                        for (int j = 0; j < 8; j++) held[0][j] = f[j];
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 8; j++) held[1][j] = f[j];
+                    }
+                } else {
+                    T(&fs)[8][kFlowSites] = flow_meas_lds<T>().f[slot];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) fs[j][lane] = f[j];
                 }
-#pragma unroll
-                for (int j = 0; j < 8; j++) fs[j][lane] = f[j];
-                __syncthreads();
             } else if constexpr (R == 2) {
                 // Two stored rows: form each SU(3) product's first two rows
                 // from operands of which only those are needed, and rebuild
@@ -473,6 +466,19 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
             }
         }
     }
+    if constexpr (MEAS) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 1; k < 3; k++) {
+            const int e = 3 * mu + k, nu = (int)((kPhaseNu >> (4 * e)) & 0xF);
+            if ((kPhaseAdd >> e) & 1) {
+                T(&fs)[8][kFlowSites] =
+                    flow_meas_lds<T>().f[plane_first(mu, nu) ? plane_slot(mu, nu) : plane_slot(nu, mu)];
+#pragma unroll
+                for (int j = 0; j < 8; j++) fs[j][lane] = fs[j][lane] + held[k - 1][j];
+            }
+        }
+    }
     if constexpr (STAGE != 0 && sizeof(T) == 8) cacc = acc_load(acc, g, mu, idx);
     if (valid) {
         const M3<T> u = lds_get(sh, mu, lane);
@@ -485,8 +491,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
         finish_link<T, R, STAGE>(wout, acc, g, mu, idx, u, z, cacc, cz, ca);
     }
     if constexpr (MEAS) {
-        // every lane is a real site here (the launch requires whole chunks);
-        // the last phase's barrier has completed every slot
+        // every lane is a real site here (the launch requires whole chunks)
+        __syncthreads();
         T fa[8], fb[8];
         if (mu < 3) {
 #pragma unroll
@@ -499,22 +505,138 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : (MEAS ? 2
     }
 }
 
+// ---- measuring stage of FP64 links --------------------------------------------
+// FP64 has the registers to keep all three of a wavefront's contributions to F (48)
+// until the end, so nothing waits between the terms, and they are handed over in the
+// LDS of the shared links, which nobody needs any more by then.  The six planes'
+// slots of the kernel above would leave no room at two blocks per CU to share the
+// backward links; without them it is 68 link gathers per site for 88, and the
+// gathers are what bounds FP64 stages.
+//
+// 24^3 x 48: 529 us, where the kernel above (backward links gathered, a barrier after
+// each phase) took 600; the phases with both planes of a pair at a time, slots
+// for those and three shared backward links 585.  More gathers in flight or
+// x- and y-neighbours from LDS gain nothing here (516 to 557).
+struct Measure64Lds {
+    union {
+        LdsMats<double, 8> sh;               // U_mu(x), then U_mu(x - mu)
+        double part[2][6][8][kFlowSites];    // F of a plane: its first wavefront's part, its second's
+    };
+};
+
+__global__ __launch_bounds__(kBlock, 2) void flow_measure64_kernel(const double2 *__restrict__ win,
+                                                                   double2 *__restrict__ wout, double *__restrict__ acc,
+                                                                   Geom g, double cz, double *__restrict__ meas)
+{
+    using T = double;
+    constexpr int R = 3;
+    __shared__ __align__(16) Measure64Lds lds;
+    __shared__ int nbr[2][4][kFlowSites];
+    const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int hb = flow_chunk(g, xcd_block(blockIdx.x, gridDim.x));
+    // every lane is a real site (the launch requires whole chunks)
+    const int idx = parity_index(g, lane >> 5, hb * (kFlowSites / 2) + (lane & 31));
+    const Site x = site_of(g, idx);
+    const DirView<T> vmu = dir_view<T>(win, g, mu);
+    const Site xpm = site_step(g, x, mu, +1);
+    const int ipm = xpm.idx, imm = site_step(g, x, mu, -1).idx;
+    nbr[0][mu][lane] = ipm;
+    nbr[1][mu][lane] = imm;
+    lds_put(lds.sh, mu, lane, load_link<T, R>(vmu, idx));
+    lds_put(lds.sh, 4 + mu, lane, load_link<T, R>(vmu, imm));
+    __syncthreads();
+    T plaq = 0, tz[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // tz: T(U_mu(x) A_mu(x)), as above
+    T f[3][8];
+    // form() keeps the loads of the next product behind the one before (200 to 230
+    // registers; free to move them the compiler spills)
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int e = 3 * mu + k, nu = (int)((kPhaseNu >> (4 * e)) & 0xF);
+        const bool first = plane_first(mu, nu);
+        const DirView<T> vnu = dir_view<T>(win, g, nu);
+        const int ipn = nbr[0][nu][lane], imn = nbr[1][nu][lane];
+        const int ipmmn = site_step(g, xpm, nu, -1).idx;
+        {
+            M3<T> up, low;
+            M3<T> p = mul_ad(load_link<T, R>(vnu, ipm), load_link<T, R>(vmu, ipn));
+            form(p);
+            mm<false, true, false>(up, p, lds_get(lds.sh, nu, lane));
+            form(up);
+            T tu[8], fl[8];
+            {
+                const M3<T> u = lds_get(lds.sh, mu, lane);
+                if (first) plaq += retrace_mul(u, up);
+                ta2_product<false>(u, up, tu);
+                form(tu);
+            }
+            p = mul_dd(load_link<T, R>(vnu, ipmmn), load_link<T, R>(vmu, imn));
+            form(p);
+            mm<false, false, false>(low, p, lds_get(lds.sh, 4 + nu, lane));
+            form(low);
+            ta2_product<false>(lds_get(lds.sh, mu, lane), low, fl);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                tz[j] += tu[j] + fl[j];
+                f[k][j] = first ? tu[j] - fl[j] : fl[j];
+            }
+        }
+        if ((kPhaseL3 >> e) & 1) {
+            const int d1 = first ? mu : nu, d2 = first ? nu : mu;
+            const int iy = site_step(g, site_step(g, x, d1, -1), d2, -1).idx;
+            const DirView<T> v1 = first ? vmu : vnu, v2 = first ? vnu : vmu;
+            M3<T> c1, c2;
+            mm<true, true, false>(c1, lds_get(lds.sh, 4 + d1, lane), load_link<T, R>(v2, iy));
+            form(c1);
+            mm<false, false, false>(c2, c1, load_link<T, R>(v1, iy));
+            form(c2);
+            mm<false, false, false>(c1, c2, lds_get(lds.sh, 4 + d2, lane));
+            T f3[8];
+            ta2_of(c1, f3);
+#pragma unroll
+            for (int j = 0; j < 8; j++) f[k][j] += f3[j];
+        }
+        form(f[k]);
+        form(tz);
+    }
+    const su3alg<T> z = force_from_ta2(tz);
+    finish_link<T, R, 0>(wout, acc, g, mu, idx, lds_get(lds.sh, mu, lane), z, z, cz, 0.0);
+    __syncthreads();  // the shared links are done with
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int nu = (int)((kPhaseNu >> (4 * (3 * mu + k))) & 0xF);
+        const bool first = plane_first(mu, nu);
+        T(&o)[8][kFlowSites] = lds.part[first ? 0 : 1][first ? plane_slot(mu, nu) : plane_slot(nu, mu)];
+#pragma unroll
+        for (int j = 0; j < 8; j++) o[j][lane] = f[k][j];
+    }
+    __syncthreads();
+    T fa[8], fb[8];
+    if (mu < 3) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            fa[j] = lds.part[0][mu][j][lane] + lds.part[1][mu][j][lane];
+            fb[j] = lds.part[0][mu + 3][j][lane] + lds.part[1][mu + 3][j][lane];
+        }
+    }
+    measure_block<T>(g, hb, mu, plaq, fa, fb, meas);
+}
+
 // ---- measuring stage of a small lattice ----------------------------------------
-// Where the blocks do not fill the chip, the kernel above is four wavefronts alone
-// on their SIMDs, and its time the chain of three phases, each two gathers,
-// five to eight products and a barrier.  Here a block has twelve wavefronts:
+// Where the blocks do not fill the chip, the kernels above are four wavefronts
+// alone on their SIMDs, and their time the chain of three phases, each two gathers
+// and five to eight products.  Here a block has twelve wavefronts:
 // wavefront (mu, k) works out mu's phase k by itself, gathering the links that the
-// kernel above shares; those of k = 1, 2 leave their part of the force in LDS, and
+// kernels above share; those of k = 1, 2 leave their part of the force in LDS, and
 // (mu, 0) adds the parts in the phases' order and finishes the link.  F's two
 // contributions per plane stand side by side instead of the later one being
 // added to the earlier.  The same sums as above.
 //
 // What bounds it: a launch and the chain gathers, products, force, exponential
 // (at 4^4 it takes hardly less than at 8^3 x 16).  Microseconds with 2 of event
-// timing, the kernel above and this one, compressed FP32, FP32 and FP64:
-//     64 blocks    14.7 11.1    16.8 12.4    18.1 17.1
-//    256 blocks    16.0 12.1    18.1 13.6    19.5 18.8
-//    768 blocks    22.2 28.9    26.4 33.7    48.2 52.1
+// timing, the kernels above and this one, compressed FP32, FP32 and FP64:
+//     64 blocks    14.2 11.2    15.6 12.5    17.5 16.9
+//    256 blocks    14.7 12.1    16.5 13.6    18.5 18.6
+//    768 blocks    19.7 28.9    23.8 33.7    40.5 52.1
 // For the plain stages, whose four wavefronts hold no phases, the same split gains
 // 0.6 us of 8.3 (compressed FP32) and nothing otherwise, so they have none.
 constexpr int kWideBlocks = 256;  // one block of twelve wavefronts per CU
@@ -706,6 +828,8 @@ void launch_flow_stage(const void *win, void *wout, void *acc, const Geom &g, in
         if (meas) {
             if (blocks <= kWideBlocks)
                 flow_measure_wide_kernel<T, R><<<blocks, 3 * kBlock, 0, s>>>(in, out, a, g, T(0.25 * eps), meas);
+            else if constexpr (sizeof(T) == 8)
+                flow_measure64_kernel<<<blocks, kBlock, 0, s>>>(in, out, a, g, T(0.25 * eps), meas);
             else
                 flow_stage_kernel<T, R, 0, true>
                     <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), meas);
