@@ -103,7 +103,8 @@ bool flow_measure_fusable(const Geom &g);
 // `sweeps` sweeps' slots.
 constexpr int kCountSlots = 256;
 __device__ __forceinline__ int count_slot(unsigned block) { return (int)(block & (kCountSlots - 1)); }
-void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, hipStream_t s);
+void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, const double *plaq,
+                      double *plaq_out, hipStream_t s);
 
 // One checkerboard sub-sweep (mu, parity), in place; accepted hits are added
 // to the sweep's slots at `count`.
