@@ -112,9 +112,7 @@ template <class P> int ensure(glacx_ctx *c, P **buf, size_t *len, size_t n)
 // host memory that the context holds: a copy of a few hundred bytes at the end of a
 // call costs more than the stores (a measurement of 8^3 x 16 FP64, two launches:
 // 38.7 us a call with the copy, 29.5 without).  Longer ones, and those of a
-// context that got no pinned memory, go to `results` and are copied.  A chain's
-// plaquettes stay on the device until its end: a store to the host at each would
-// hold up the sweep behind it.
+// context that got no pinned memory, go to `results` and are copied.
 constexpr size_t kHostRows = 8192;
 
 int result_rows(glacx_ctx *c, size_t n, double **rows)
@@ -220,19 +218,23 @@ template <class T, int R> int run_measure(glacx_ctx *c, const void *f, double *o
     return GLACX_OK;
 }
 
-template <class T, int R> int run_plaquette(glacx_ctx *c, const void *f, double *out)
+template <class T, int R> int run_plaquette_partials(glacx_ctx *c, const void *f, double *partials)
 {
-    const int np = plaquette_partials_count(c->geom);
-    int rc = ensure(c, &c->partials, &c->partials_len, (size_t)np);
-    if (rc) return rc;
     hipEvent_t e0 = nullptr;
+    int rc;
     if ((rc = timed_begin(c, &e0))) return rc;
-    launch_plaquette<T, R>(f, c->geom, c->partials, c->stream);
+    launch_plaquette<T, R>(f, c->geom, partials, c->stream);
     CHECK_LAUNCH(c);
-    if ((rc = timed_end(c, GLACX_K_PLAQUETTE, e0))) return rc;
-    launch_plaquette_finish(c->partials, np, c->geom, out, c->stream);
-    CHECK_LAUNCH(c);
-    return GLACX_OK;
+    return timed_end(c, GLACX_K_PLAQUETTE, e0);
+}
+
+// Measurements whose partials a flow (or a chain, its plaquettes') holds before it
+// sums them: all of them, or as many as `limit` doubles take (kFlowPartials: 32 MiB of a context, which is
+// 64 measurements at 32^4 and six at 48^3 x 96).
+constexpr size_t kFlowPartials = (size_t)4 << 20;
+int flow_slots(size_t per, int n_steps, size_t limit)
+{
+    return (int)std::min<size_t>((size_t)n_steps + 1, std::max<size_t>(1, limit / per));
 }
 
 // One RK3 step on `f`: three stages ping-ponging through the work buffer
@@ -675,27 +677,61 @@ int glacx_hot_start(glacx_ctx *c, int field, uint64_t seed, int kind, double eps
 
 namespace {
 
-// The end of a chain of sweeps: accepted hits summed from their slots, and with the
-// plaquettes (in `results`) to the host.
-int finish_sweeps(glacx_ctx *c, int n_sweeps, int n_hit, double *accept, double *plaq)
+// What a chain of sweeps leaves: a plaquette and a count of accepted hits per
+// sweep, in host_rows or in device memory.  The sweeps' plaquette partials wait side
+// by side, as a flow's do, and are summed together: a launch after every sweep took
+// 4.7 of its 174 us at 16^4 FP64.
+struct SweepEnd {
+    int sweeps = 0, slots = 1;
+    double *plaq = nullptr;
+    unsigned long long *counts = nullptr;
+    bool on_host = false;
+};
+
+int begin_sweeps(glacx_ctx *c, int n_sweeps, bool plaq, SweepEnd *end)
 {
     const size_t n = (size_t)n_sweeps;
-    unsigned long long *sums = c->counts + n * kCountSlots;
-    std::vector<unsigned long long> counts(n);
     static_assert(sizeof(double) == sizeof(unsigned long long), "both in host_rows");
-    if (c->host_rows && 2 * n <= kHostRows) {
-        auto *host = reinterpret_cast<unsigned long long *>(c->host_rows + n);
-        launch_count_sum(c->counts, host, n_sweeps, plaq ? c->results : nullptr, c->host_rows, c->stream);
+    end->sweeps = n_sweeps;
+    end->on_host = c->host_rows && 2 * n <= kHostRows;
+    end->counts = end->on_host ? reinterpret_cast<unsigned long long *>(c->host_rows + n) : c->counts + n * kCountSlots;
+    if (!plaq) return GLACX_OK;
+    int rc;
+    if (!end->on_host && (rc = ensure(c, &c->results, &c->results_len, n))) return rc;
+    end->plaq = end->on_host ? c->host_rows : c->results;
+    const size_t per = (size_t)plaquette_partials_count(c->geom);
+    end->slots = flow_slots(per, n_sweeps - 1, kFlowPartials);
+    return ensure(c, &c->partials, &c->partials_len, per * end->slots);
+}
+
+int sweep_plaquette(glacx_ctx *c, int i, const SweepEnd &end)
+{
+    const int np = plaquette_partials_count(c->geom), slot = i % end.slots;
+    double *part = c->partials + (size_t)slot * np;
+    int rc = DISPATCH(c, run_plaquette_partials, c, c->field[GLACX_FIELD_MAIN], part);
+    if (rc) return rc;
+    if (slot == end.slots - 1 || i == end.sweeps - 1) {
+        launch_plaquette_finish(c->partials, np, c->geom, end.plaq + (i - slot), slot + 1, c->stream);
         CHECK_LAUNCH(c);
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
-        std::memcpy(counts.data(), host, n * sizeof(unsigned long long));
-        if (plaq) std::memcpy(plaq, c->host_rows, n * sizeof(double));
-    } else {
-        launch_count_sum(c->counts, sums, n_sweeps, nullptr, nullptr, c->stream);
-        CHECK_LAUNCH(c);
-        HIP_TRY(c, hipMemcpyAsync(counts.data(), sums, n * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
-        if (plaq) HIP_TRY(c, hipMemcpyAsync(plaq, c->results, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
+    }
+    return GLACX_OK;
+}
+
+int finish_sweeps(glacx_ctx *c, const SweepEnd &end, int n_hit, double *accept, double *plaq)
+{
+    const size_t n = (size_t)end.sweeps;
+    launch_count_sum(c->counts, end.counts, end.sweeps, c->stream);
+    CHECK_LAUNCH(c);
+    std::vector<unsigned long long> counts(n);
+    if (!end.on_host) {
+        HIP_TRY(c, hipMemcpyAsync(counts.data(), end.counts, n * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                                  c->stream));
+        if (plaq) HIP_TRY(c, hipMemcpyAsync(plaq, end.plaq, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    }
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    if (end.on_host) {
+        std::memcpy(counts.data(), end.counts, n * sizeof(unsigned long long));
+        if (plaq) std::memcpy(plaq, end.plaq, n * sizeof(double));
     }
     if (accept)
         for (size_t i = 0; i < n; i++) accept[i] = (double)counts[i] / (4.0 * n_hit * (double)c->geom.v);
@@ -715,7 +751,8 @@ int glacx_metropolis(glacx_ctx *c, int n_sweeps, double beta, double eps, int n_
     int rc = ensure(c, &c->counts, &c->counts_len, slots + n_sweeps);
     if (rc) return rc;
     HIP_TRY(c, hipMemsetAsync(c->counts, 0, sizeof(unsigned long long) * slots, c->stream));
-    if (plaq && (rc = ensure(c, &c->results, &c->results_len, (size_t)n_sweeps))) return rc;
+    SweepEnd end;
+    if ((rc = begin_sweeps(c, n_sweeps, plaq != nullptr, &end))) return rc;
     for (int i = 0; i < n_sweeps; i++) {
         MetroParams p;
         p.beta = beta;
@@ -725,9 +762,9 @@ int glacx_metropolis(glacx_ctx *c, int n_sweeps, double beta, double eps, int n_
         p.reunit = reunit_every > 0 && (p.sweep % (uint64_t)reunit_every) == 0;
         p.seed = seed;
         if ((rc = DISPATCH(c, run_metropolis_sweep, c, p, c->counts + (size_t)i * kCountSlots))) return rc;
-        if (plaq && (rc = DISPATCH(c, run_plaquette, c, c->field[GLACX_FIELD_MAIN], c->results + i))) return rc;
+        if (plaq && (rc = sweep_plaquette(c, i, end))) return rc;
     }
-    return finish_sweeps(c, n_sweeps, n_hit, accept, plaq);
+    return finish_sweeps(c, end, n_hit, accept, plaq);
 }
 
 namespace {
@@ -798,20 +835,15 @@ int glacx_plaquette(glacx_ctx *c, int field, double *plaq)
     double *rows;
     int rc = result_rows(c, 1, &rows);
     if (rc) return rc;
-    if ((rc = DISPATCH(c, run_plaquette, c, c->field[field], rows))) return rc;
+    const int np = plaquette_partials_count(c->geom);
+    if ((rc = ensure(c, &c->partials, &c->partials_len, (size_t)np))) return rc;
+    if ((rc = DISPATCH(c, run_plaquette_partials, c, c->field[field], c->partials))) return rc;
+    launch_plaquette_finish(c->partials, np, c->geom, rows, 1, c->stream);
+    CHECK_LAUNCH(c);
     return read_rows(c, rows, plaq, 1);
 }
 
 namespace {
-
-// Measurements whose partials a flow holds before it sums them: all of them, or
-// as many as `limit` doubles take (kFlowPartials: 32 MiB of a context, which is
-// 64 measurements at 32^4 and six at 48^3 x 96).
-constexpr size_t kFlowPartials = (size_t)4 << 20;
-int flow_slots(size_t per, int n_steps, size_t limit)
-{
-    return (int)std::min<size_t>((size_t)n_steps + 1, std::max<size_t>(1, limit / per));
-}
 
 int flow_impl(glacx_ctx *c, int field, int n_steps, double eps, bool super, double *plaq, double *e_raw, double *q,
               double *w, double *q_t, double *w_t)
@@ -1113,7 +1145,8 @@ int glacx_metropolis_learned(glacx_ctx *c, int n_sweeps, double beta, double eps
     int rc = ensure(c, &c->counts, &c->counts_len, slots + n_sweeps);
     if (rc) return rc;
     HIP_TRY(c, hipMemsetAsync(c->counts, 0, sizeof(unsigned long long) * slots, c->stream));
-    if (plaq && (rc = ensure(c, &c->results, &c->results_len, (size_t)n_sweeps))) return rc;
+    SweepEnd end;
+    if ((rc = begin_sweeps(c, n_sweeps, plaq != nullptr, &end))) return rc;
     for (int i = 0; i < n_sweeps; i++) {
         MetroParams p;
         p.beta = beta;
@@ -1123,9 +1156,9 @@ int glacx_metropolis_learned(glacx_ctx *c, int n_sweeps, double beta, double eps
         p.reunit = reunit_every > 0 && (p.sweep % (uint64_t)reunit_every) == 0;
         p.seed = seed;
         if ((rc = DISPATCH(c, run_metropolis_learned_sweep, c, p, c->counts + (size_t)i * kCountSlots))) return rc;
-        if (plaq && (rc = DISPATCH(c, run_plaquette, c, c->field[GLACX_FIELD_MAIN], c->results + i))) return rc;
+        if (plaq && (rc = sweep_plaquette(c, i, end))) return rc;
     }
-    return finish_sweeps(c, n_sweeps, n_hit, accept, plaq);
+    return finish_sweeps(c, end, n_hit, accept, plaq);
 }
 
 int glacx_timing_enable(glacx_ctx *c, int on)

@@ -430,9 +430,9 @@ __global__ __launch_bounds__(kFinishBlock) void plaquette_finish_kernel(const do
 {
     double acc[1] = {0.0};
 #pragma unroll 8
-    for (int b = threadIdx.x; b < n; b += kFinishBlock) acc[0] += partials[b];
+    for (int b = threadIdx.x; b < n; b += kFinishBlock) acc[0] += partials[(size_t)blockIdx.x * n + b];
     block_sum<1, kFinishBlock / 64>(acc);
-    if (threadIdx.x == 0) out[0] = acc[0] / (18.0 * (double)g.v);
+    if (threadIdx.x == 0) out[blockIdx.x] = acc[0] / (18.0 * (double)g.v);
 }
 
 // 64-site chunks per time slice: nzb runs of each slice, cpr chunks per run
@@ -478,9 +478,9 @@ template <class T, int R> void launch_plaquette(const void *f, const Geom &g, do
         (const typename vec2<T>::type *)f, g, partials);
 }
 
-void launch_plaquette_finish(const double *partials, int nparts, const Geom &g, double *out, hipStream_t s)
+void launch_plaquette_finish(const double *partials, int nparts, const Geom &g, double *out, int rows, hipStream_t s)
 {
-    plaquette_finish_kernel<<<1, kFinishBlock, 0, s>>>(partials, nparts, g, out);
+    plaquette_finish_kernel<<<rows, kFinishBlock, 0, s>>>(partials, nparts, g, out);
 }
 
 template void launch_measure<float, 3>(const void *, const Geom &, double *, int, double *, hipStream_t);

@@ -327,8 +327,7 @@ __global__ __launch_bounds__(64 * (STAPLERS + PROPOSERS), STAPLERS > 1 ? 4 : 2) 
 }
 
 __global__ __launch_bounds__(64) void count_sum_kernel(const unsigned long long *__restrict__ slots,
-                                                       unsigned long long *__restrict__ counts,
-                                                       const double *__restrict__ plaq, double *__restrict__ plaq_out)
+                                                       unsigned long long *__restrict__ counts)
 {
     const unsigned long long *p = slots + (size_t)blockIdx.x * kCountSlots;
     unsigned long long n = 0;
@@ -336,16 +335,12 @@ __global__ __launch_bounds__(64) void count_sum_kernel(const unsigned long long 
     for (int k = threadIdx.x; k < kCountSlots; k += 64) n += p[k];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
-    if (threadIdx.x == 0) {
-        counts[blockIdx.x] = n;
-        if (plaq) plaq_out[blockIdx.x] = plaq[blockIdx.x];
-    }
+    if (threadIdx.x == 0) counts[blockIdx.x] = n;
 }
 
-void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, const double *plaq,
-                      double *plaq_out, hipStream_t s)
+void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, hipStream_t s)
 {
-    count_sum_kernel<<<sweeps, 64, 0, s>>>(slots, counts, plaq, plaq_out);
+    count_sum_kernel<<<sweeps, 64, 0, s>>>(slots, counts);
 }
 
 template <class T, int R>

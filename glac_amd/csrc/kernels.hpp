@@ -86,7 +86,7 @@ void launch_measure_finish(double *partials, const Geom &g, double *out, bool su
 
 int plaquette_partials_count(const Geom &g);
 template <class T, int R> void launch_plaquette(const void *f, const Geom &g, double *partials, hipStream_t s);
-void launch_plaquette_finish(const double *partials, int nparts, const Geom &g, double *out, hipStream_t s);
+void launch_plaquette_finish(const double *partials, int nparts, const Geom &g, double *out, int rows, hipStream_t s);
 
 // One RK3 stage (0, 1, 2): win -> wout, accumulator read/written in acc.
 // With `meas` (stage 0 only, FP32 links, flow_measure_fusable(g)) the stage
@@ -103,8 +103,7 @@ bool flow_measure_fusable(const Geom &g);
 // `sweeps` sweeps' slots.
 constexpr int kCountSlots = 256;
 __device__ __forceinline__ int count_slot(unsigned block) { return (int)(block & (kCountSlots - 1)); }
-void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, const double *plaq,
-                      double *plaq_out, hipStream_t s);
+void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, hipStream_t s);
 
 // One checkerboard sub-sweep (mu, parity), in place; accepted hits are added
 // to the sweep's slots at `count`.

@@ -1,5 +1,6 @@
 """Results that fit the context's pinned rows (8192 doubles) are stored there by the
-kernels, longer ones are copied: a long call gives what two short ones give."""
+kernels, longer ones are copied; a chain's plaquettes are summed together, in batches of
+32 MiB of partials: a long call gives what two short ones give."""
 import numpy as np
 import pytest
 
@@ -22,6 +23,19 @@ def test_long_chain_equals_two_short_ones(sweeps):
         assert np.array_equal(links, L.download())
     assert np.array_equal(acc, np.concatenate([h[0] for h in half]))
     assert np.array_equal(plaq, np.concatenate([h[1] for h in half]))
+
+
+def test_plaquettes_summed_in_two_batches():
+    """1024 partials a sweep at 16^4: 4096 sweeps fill the batch."""
+    print("\n[gpu case] host rows, plaquettes in two batches", flush=True)
+    n = (16, 16, 16, 16)
+    with glacx.Lattice(n, glacx.FP32_COMPRESSED) as L:
+        L.hot_start(3)
+        _, plaq = L.metropolis(4099, 6.0, 0.24, 1, seed=5, plaquette=True)
+        L.hot_start(3)
+        _, a = L.metropolis(4090, 6.0, 0.24, 1, seed=5, plaquette=True)
+        _, b = L.metropolis(9, 6.0, 0.24, 1, seed=5, sweep_offset=4090, plaquette=True)
+    assert np.array_equal(plaq, np.concatenate([a, b]))
 
 
 @pytest.mark.parametrize("steps", [1169, 1170, 1500])  # rows of 7 doubles: 8190, 8197, 10507
