@@ -42,52 +42,85 @@ template <class T> using FlowLds = LdsMats<T, 8>;
 // RK3 accumulator: the 8 real parameters (a0, a1, p0..p5) of an su(3)
 // element per link, in 16-byte vectors: two float4 planes per direction in
 // FP32 (a0 a1 p0 p1 | p2 p3 p4 p5), four double2 planes in FP64.  Each link's
-// wavefront alone touches its entry, once per launch, so loads and stores are
-// non-temporal, as the stage's link stores are: they leave L2 to the links that
-// neighbouring blocks gather (FP64 24^3 x 48: 495 -> 479 us with the links'
-// stores, -> 465 with the accumulator; FP32 32^4 261 -> 256 us).
-template <class V> __device__ __forceinline__ V stream_load(const V *p)
+// wavefront alone touches its entry, once per launch, and nobody reads a link that
+// the launch stores.  Stored and loaded as non-temporal (kStreamAcc, kStreamLinks) they
+// leave the caches to the links that neighbouring blocks gather; while the Infinity
+// Cache's 256 MiB hold what the next stage reads, that throws away what it would
+// find there.  So the accumulator is streamed once the two fields and it take
+// 256 MiB, the links once the two fields alone exceed that.  Both are also while
+// the two fields fit in the eight L2s (32 MiB), where a launch otherwise ends with
+// writing out what they hold: twenty steps of 12 x 10 x 14 x 18 FP32 994 us for
+// 1054, forty of 8^3 x 16 FP64 1550 for 1584; 16^4 FP64 (72 MiB) is the other way,
+// 39.6 us a stage for 36.5.  Microseconds of a plain stage, with nothing, the
+// accumulator, and both streamed:
+//     MiB of two fields, with accumulator    nothing     acc    both
+//     compressed  16^2 x 32 x 48   144  192      81.0    84.8    87.7
+//                 32^3 x 16        192  256     115.8   114.1   117.5
+//                 24^3 x 48        243  324     163.8   145.5   160.1
+//                 32^3 x 24        288  384     189.0   183.9   179.6
+//                 48^3 x 96       3888 5184      2633    2593    2555
+//     FP32        24^4             182  223      89.6    96.3   109.1
+//                 32^3 x 16        288  352     168.1   160.9   162.9
+//                 32^4             576  704       344     323     315
+//     FP64        16^3 x 32        144  176      65.9    70.6    75.4
+//                 16^3 x 48        216  264     101.7   100.2   109.3
+//                 24^3 x 48        729  891     390.2   380.1   370.1
+enum StreamBits : unsigned { kStreamAcc = 1, kStreamLinks = 2 };
+// One direction's accumulator as a buffer of 8 V reals.  Buffer accesses carry the
+// policy as an operand; of plain ones in the two arms of a branch the compiler makes
+// one, without it.
+template <class T> __device__ __forceinline__ __amdgpu_buffer_rsrc_t acc_view(const T *acc, const Geom &g, int mu)
 {
-    static_assert(sizeof(V) == 16, "16-byte vectors");
-    using U4 = unsigned __attribute__((ext_vector_type(4)));
-    return __builtin_bit_cast(V, __builtin_nontemporal_load(reinterpret_cast<const U4 *>(p)));
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(acc + (size_t)mu * 8 * g.v), (short)0,
+                                             (int)(8u * (unsigned)g.v * (unsigned)sizeof(T)), kBufferFlags);
 }
-template <class V> __device__ __forceinline__ void stream_store(V *p, const V &v)
+using AccVec = unsigned __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ AccVec acc_get(__amdgpu_buffer_rsrc_t r, const Geom &g, int idx, int plane, bool stream)
 {
-    static_assert(sizeof(V) == 16, "16-byte vectors");
-    using U4 = unsigned __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store(__builtin_bit_cast(U4, v), reinterpret_cast<U4 *>(p));
+    const unsigned off = (unsigned)idx * 16u, at = (unsigned)plane * 16u * (unsigned)g.v;
+    return stream ? __builtin_amdgcn_raw_buffer_load_b128(r, off, at, store_policy<true>())
+                  : __builtin_amdgcn_raw_buffer_load_b128(r, off, at, store_policy<false>());
 }
-__device__ __forceinline__ void acc_store(float *acc, const Geom &g, int mu, int idx, const su3alg<float> &z)
+__device__ __forceinline__ void acc_put(__amdgpu_buffer_rsrc_t r, const Geom &g, int idx, int plane, bool stream, AccVec v)
 {
-    float4 *q = reinterpret_cast<float4 *>(acc) + (size_t)mu * 2 * g.v + idx;
-    stream_store(q, make_float4(z.a0, z.a1, z.p[0], z.p[1]));
-    stream_store(q + g.v, make_float4(z.p[2], z.p[3], z.p[4], z.p[5]));
+    const unsigned off = (unsigned)idx * 16u, at = (unsigned)plane * 16u * (unsigned)g.v;
+    if (stream)
+        __builtin_amdgcn_raw_buffer_store_b128(v, r, off, at, store_policy<true>());
+    else
+        __builtin_amdgcn_raw_buffer_store_b128(v, r, off, at, store_policy<false>());
 }
-__device__ __forceinline__ su3alg<float> acc_load(const float *acc, const Geom &g, int mu, int idx)
+__device__ __forceinline__ void acc_store(float *acc, const Geom &g, int mu, int idx, const su3alg<float> &z, bool stream)
 {
-    const float4 *q = reinterpret_cast<const float4 *>(acc) + (size_t)mu * 2 * g.v + idx;
-    const float4 u = stream_load(q), v = stream_load(q + g.v);
+    const auto r = acc_view(acc, g, mu);
+    acc_put(r, g, idx, 0, stream, __builtin_bit_cast(AccVec, make_float4(z.a0, z.a1, z.p[0], z.p[1])));
+    acc_put(r, g, idx, 1, stream, __builtin_bit_cast(AccVec, make_float4(z.p[2], z.p[3], z.p[4], z.p[5])));
+}
+__device__ __forceinline__ su3alg<float> acc_load(const float *acc, const Geom &g, int mu, int idx, bool stream)
+{
+    const auto r = acc_view(acc, g, mu);
+    const float4 u = __builtin_bit_cast(float4, acc_get(r, g, idx, 0, stream));
+    const float4 v = __builtin_bit_cast(float4, acc_get(r, g, idx, 1, stream));
     su3alg<float> z;
     z.a0 = u.x, z.a1 = u.y, z.p[0] = u.z, z.p[1] = u.w, z.p[2] = v.x, z.p[3] = v.y, z.p[4] = v.z, z.p[5] = v.w;
     return z;
 }
-__device__ __forceinline__ void acc_store(double *acc, const Geom &g, int mu, int idx, const su3alg<double> &z)
+__device__ __forceinline__ void acc_store(double *acc, const Geom &g, int mu, int idx, const su3alg<double> &z, bool stream)
 {
-    double2 *q = reinterpret_cast<double2 *>(acc) + (size_t)mu * 4 * g.v + idx;
-    stream_store(q, make_double2(z.a0, z.a1));
+    const auto r = acc_view(acc, g, mu);
+    acc_put(r, g, idx, 0, stream, __builtin_bit_cast(AccVec, make_double2(z.a0, z.a1)));
 #pragma unroll
-    for (int k = 0; k < 3; k++) stream_store(q + (size_t)(k + 1) * g.v, make_double2(z.p[2 * k], z.p[2 * k + 1]));
+    for (int k = 0; k < 3; k++)
+        acc_put(r, g, idx, k + 1, stream, __builtin_bit_cast(AccVec, make_double2(z.p[2 * k], z.p[2 * k + 1])));
 }
-__device__ __forceinline__ su3alg<double> acc_load(const double *acc, const Geom &g, int mu, int idx)
+__device__ __forceinline__ su3alg<double> acc_load(const double *acc, const Geom &g, int mu, int idx, bool stream)
 {
-    const double2 *q = reinterpret_cast<const double2 *>(acc) + (size_t)mu * 4 * g.v + idx;
+    const auto r = acc_view(acc, g, mu);
     su3alg<double> z;
-    const double2 u = stream_load(q);
+    const double2 u = __builtin_bit_cast(double2, acc_get(r, g, idx, 0, stream));
     z.a0 = u.x, z.a1 = u.y;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        const double2 v = stream_load(q + (size_t)(k + 1) * g.v);
+        const double2 v = __builtin_bit_cast(double2, acc_get(r, g, idx, k + 1, stream));
         z.p[2 * k] = v.x, z.p[2 * k + 1] = v.y;
     }
     return z;
@@ -164,11 +197,11 @@ template <class T> __device__ __forceinline__ FlowMeasLds<T> &flow_meas_lds()
 template <class T, int R, int STAGE>
 __device__ __forceinline__ void finish_link(typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc, const Geom &g,
                                             int mu, int idx, const M3<T> &u, const su3alg<T> &z, const su3alg<T> &cacc,
-                                            T cz, T ca)
+                                            T cz, T ca, unsigned stream)
 {
     su3alg<T> y;
     if constexpr (STAGE == 0) {
-        acc_store(acc, g, mu, idx, z);
+        acc_store(acc, g, mu, idx, z, stream & kStreamAcc);
         y.a0 = cz * z.a0;
         y.a1 = cz * z.a1;
 #pragma unroll
@@ -178,7 +211,7 @@ __device__ __forceinline__ void finish_link(typename vec2<T>::type *__restrict__
         y.a1 = cz * z.a1 - ca * cacc.a1;
 #pragma unroll
         for (int k = 0; k < 6; k++) y.p[k] = cz * z.p[k] - ca * cacc.p[k];
-        if (STAGE == 1) acc_store(acc, g, mu, idx, y);
+        if (STAGE == 1) acc_store(acc, g, mu, idx, y, stream & kStreamAcc);
     }
     M3<T> w = zero3<T>();
     mm<false, false, false, R>(w, exp_su3(y), u);  // two rows suffice when two are stored
@@ -200,7 +233,10 @@ __device__ __forceinline__ void finish_link(typename vec2<T>::type *__restrict__
             orthonormalize_rows<true>(d);
         w = convert<T>(d);
     }
-    store_link<T, R, true>(dir_view<T>(wout, g, mu), idx, w);
+    if (stream & kStreamLinks)
+        store_link<T, R, true>(dir_view<T>(wout, g, mu), idx, w);
+    else
+        store_link<T, R, false>(dir_view<T>(wout, g, mu), idx, w);
 }
 
 // Z = -1/2 T(U A), the form force_from_omega evaluates
@@ -249,7 +285,7 @@ __device__ __forceinline__ void measure_block(const Geom &g, int hb, int mu, T p
 template <class T, int R, int STAGE, bool MEAS>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP64_FLOW_WAVES) void flow_stage_kernel(const typename vec2<T>::type *__restrict__ win,
                                                             typename vec2<T>::type *__restrict__ wout,
-                                                            T *__restrict__ acc, Geom g, T cz, T ca,
+                                                            T *__restrict__ acc, Geom g, T cz, T ca, unsigned stream,
                                                             double *__restrict__ meas)
 {
     static_assert(!MEAS || (STAGE == 0 && sizeof(T) == 4), "the measurement is fused into stage 0 only, FP64 has its own");
@@ -266,7 +302,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
     // passes under the staple loop instead of stalling the step after it; FP64 has
     // no registers left for it (with it in place early, 504 for 391 us)
     su3alg<T> cacc;
-    if constexpr (STAGE != 0 && sizeof(T) == 4) cacc = acc_load(acc, g, mu, idx);
+    if constexpr (STAGE != 0 && sizeof(T) == 4) cacc = acc_load(acc, g, mu, idx, stream & kStreamAcc);
     const DirView<T> vmu = dir_view<T>(win, g, mu);
     // the site's neighbours x + mu and x - mu, shared with the other
     // wavefronts, whose staples step the same way in direction mu
@@ -479,7 +515,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
             }
         }
     }
-    if constexpr (STAGE != 0 && sizeof(T) == 8) cacc = acc_load(acc, g, mu, idx);
+    if constexpr (STAGE != 0 && sizeof(T) == 8) cacc = acc_load(acc, g, mu, idx, stream & kStreamAcc);
     if (valid) {
         const M3<T> u = lds_get(sh, mu, lane);
         su3alg<T> z;
@@ -488,7 +524,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
         } else {
             z = force_from_omega(mul(u, a));
         }
-        finish_link<T, R, STAGE>(wout, acc, g, mu, idx, u, z, cacc, cz, ca);
+        finish_link<T, R, STAGE>(wout, acc, g, mu, idx, u, z, cacc, cz, ca, stream);
     }
     if constexpr (MEAS) {
         // every lane is a real site here (the launch requires whole chunks)
@@ -526,7 +562,8 @@ struct Measure64Lds {
 
 __global__ __launch_bounds__(kBlock, 2) void flow_measure64_kernel(const double2 *__restrict__ win,
                                                                    double2 *__restrict__ wout, double *__restrict__ acc,
-                                                                   Geom g, double cz, double *__restrict__ meas)
+                                                                   Geom g, double cz, unsigned stream,
+                                                                   double *__restrict__ meas)
 {
     using T = double;
     constexpr int R = 3;
@@ -599,7 +636,7 @@ __global__ __launch_bounds__(kBlock, 2) void flow_measure64_kernel(const double2
         form(tz);
     }
     const su3alg<T> z = force_from_ta2(tz);
-    finish_link<T, R, 0>(wout, acc, g, mu, idx, lds_get(lds.sh, mu, lane), z, z, cz, 0.0);
+    finish_link<T, R, 0>(wout, acc, g, mu, idx, lds_get(lds.sh, mu, lane), z, z, cz, 0.0, stream);
     __syncthreads();  // the shared links are done with
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -791,7 +828,7 @@ __global__ __launch_bounds__(3 * kBlock, 3) void flow_measure_wide_kernel(const 
         z = force_from_omega(mul(u, a));
     else
         z = force_from_ta2(tz);
-    finish_link<T, R, 0>(wout, acc, g, mu, idx, u, z, z, cz, T(0));
+    finish_link<T, R, 0>(wout, acc, g, mu, idx, u, z, z, cz, T(0), kStreamAcc | kStreamLinks);  // fields below 32 MiB
     T fa[8], fb[8];
     if (mu < 3) {
 #pragma unroll
@@ -823,28 +860,33 @@ void launch_flow_stage(const void *win, void *wout, void *acc, const Geom &g, in
     const V2 *in = (const V2 *)win;
     V2 *out = (V2 *)wout;
     T *a = (T *)acc;
+    const size_t fields = (size_t)2 * 4 * g.v * 6 * R * sizeof(T), accumulator = (size_t)32 * g.v * sizeof(T);
+    constexpr size_t kInfinityCache = (size_t)256 << 20;
+    const unsigned stream = fields < ((size_t)32 << 20) ? kStreamAcc | kStreamLinks
+                                                        : (fields + accumulator >= kInfinityCache ? kStreamAcc : 0u) |
+                                                              (fields > kInfinityCache ? kStreamLinks : 0u);
     switch (stage) {
     case 0:
         if (meas) {
             if (blocks <= kWideBlocks)
                 flow_measure_wide_kernel<T, R><<<blocks, 3 * kBlock, 0, s>>>(in, out, a, g, T(0.25 * eps), meas);
             else if constexpr (sizeof(T) == 8)
-                flow_measure64_kernel<<<blocks, kBlock, 0, s>>>(in, out, a, g, T(0.25 * eps), meas);
+                flow_measure64_kernel<<<blocks, kBlock, 0, s>>>(in, out, a, g, T(0.25 * eps), stream, meas);
             else
                 flow_stage_kernel<T, R, 0, true>
-                    <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), meas);
+                    <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), stream, meas);
             break;
         }
         flow_stage_kernel<T, R, 0, false>
-            <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), nullptr);
+            <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), stream, nullptr);
         break;
     case 1:
         flow_stage_kernel<T, R, 1, false><<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(
-            in, out, a, g, T(8.0 / 9.0 * eps), T(17.0 / 36.0 * eps), nullptr);
+            in, out, a, g, T(8.0 / 9.0 * eps), T(17.0 / 36.0 * eps), stream, nullptr);
         break;
     default:
         flow_stage_kernel<T, R, 2, false>
-            <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.75 * eps), T(1), nullptr);
+            <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.75 * eps), T(1), stream, nullptr);
         break;
     }
 }
