@@ -335,7 +335,7 @@ def main():
     metro_gbs = metro_bytes / (metro_ms * 1e-3) / 1e9
     prof_stage = profiled(n, [f"flow_stage_kernel<float, {rows}, {k}, false>" for k in plain_stages])
     prof_stage0 = profiled(n, [f"flow_stage_kernel<float, {rows}, 0, true>"])
-    prof_metro = profiled(n, [f"metropolis_kernel<float, {rows}>"])
+    prof_metro = profiled(n, [f"metropolis_kernel<float, {rows}, 3>"])
 
     # ---------------------------------------------------------------- FP64 flow
     fp64 = None
