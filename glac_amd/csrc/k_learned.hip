@@ -508,19 +508,18 @@ __global__ __launch_bounds__(kBlock) void to_bf16_kernel(const float *__restrict
 // (a sixth of the time went to bank conflicts) and a parameter at a time into
 // LDS before the staple's loads: 24^3x48 79.5 -> 76.5 us a sub-sweep, 32^4 102 ->
 // 99, 32^3x8 43 -> 38.5.
-// Waves per SIMD the FP32 sampling kernel is compiled for (build-time tuning):
-// four fit 128 VGPRs and, with the network's output buffer at 32 floats per
-// link, 38.7 KB of LDS per block.  Three are 3 % ahead at five or six blocks per
-// CU and 3 % behind from twelve on.
-#ifndef GLACX_LEARNED_WAVES
-#define GLACX_LEARNED_WAVES 4
-#endif
-template <class T, int R>
-__global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? GLACX_LEARNED_WAVES : 1) void metropolis_learned_kernel(typename vec2<T>::type *__restrict__ f, Geom g,
-                                                                    int mu, int parity, MetroParams prm,
-                                                                    const unsigned short *__restrict__ wbf16,
-                                                                    const float *__restrict__ mean_std,
-                                                                    unsigned long long *__restrict__ count)
+// WAVES: FP32 wavefronts per SIMD.  Four fit 128 VGPRs and, with the network's
+// output buffer at 32 floats per link, 38.7 KB of LDS per block.  Three are ahead
+// where four would leave a last block or two alone on a CU, and behind once there
+// are many rounds (microseconds per sub-sweep, compressed, three | four):
+//     blocks per CU    4.0    4.5    5.0    6.0    8.0    12    16
+//                     62.0   69.9   70.6   79.5   99.4   145   196
+//                     62.2   71.7   73.2   81.5   99.3   142   190
+template <class T, int R, int WAVES>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? WAVES : 1, sizeof(T) == 4 ? WAVES : 2)))
+void metropolis_learned_kernel(typename vec2<T>::type *__restrict__ f, Geom g, int mu, int parity, MetroParams prm,
+                               const unsigned short *__restrict__ wbf16, const float *__restrict__ mean_std,
+                               unsigned long long *__restrict__ count)
 {
     __shared__ __align__(16) MlpImage im;
     __shared__ __align__(16) float obuf[kBlock / 64][64 * kMlpObuf];
@@ -528,7 +527,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? GLACX_LEARNED_WAVES : 1) v
     const int h_raw = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
     const bool valid = h_raw < g.vh;
     const int h = valid ? h_raw : g.vh - 1;  // idle lanes mirror a real link for the network GEMMs, store nothing
-    double nacc[1] = {0.0};
+    int n = 0;
     {
         const int idx = parity_index(g, parity, h);
         const Site x = site_of(g, idx);
@@ -583,11 +582,10 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? GLACX_LEARNED_WAVES : 1) v
                 u = convert<T>(d);
             }
             store_link<T, R>(f, g, mu, idx, u);
-            nacc[0] = (double)accepted;
+            n = accepted;
         }
     }
-    block_sum<1>(nacc);
-    if (threadIdx.x == 0) atomicAdd(count + count_slot(blockIdx.x), (unsigned long long)nacc[0]);
+    add_count(count, blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), n);
 }
 
 // The sampling kernels' matrix-core forward pass on n given feature rows (6
@@ -675,8 +673,14 @@ void launch_metropolis_learned(void *f, const Geom &g, int mu, int parity, const
                                hipStream_t s)
 {
     const unsigned blocks = (unsigned)((g.vh + kBlock - 1) / kBlock);
-    metropolis_learned_kernel<T, R><<<blocks, kBlock, 0, s>>>((typename vec2<T>::type *)f, g, mu, parity, p, wbf16,
-                                                           mean_std, count);
+    auto *links = (typename vec2<T>::type *)f;
+    if constexpr (sizeof(T) == 4) {
+        if (blocks <= 6 * 256) {  // the table at metropolis_learned_kernel; 256 CUs
+            metropolis_learned_kernel<T, R, 3><<<blocks, kBlock, 0, s>>>(links, g, mu, parity, p, wbf16, mean_std, count);
+            return;
+        }
+    }
+    metropolis_learned_kernel<T, R, 4><<<blocks, kBlock, 0, s>>>(links, g, mu, parity, p, wbf16, mean_std, count);
 }
 
 template void launch_collect<float, 3>(const void *, const Geom &, int, int, int, float *, size_t, size_t, hipStream_t);

@@ -36,14 +36,6 @@ template <class T, int R> __device__ __forceinline__ M3<T> reunitarized(const M3
     return convert<T>(d);
 }
 
-// The wavefront's accepted hits into its slot.
-__device__ __forceinline__ void add_count(unsigned long long *count, unsigned wavefront, int n)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(count + count_slot(wavefront), (unsigned long long)n);
-}
-
 // What bounds it: FP32 the vector ALU, which is busy all the time (32^4: 5377
 // instructions in each of eight wavefronts per SIMD, 72 us at 2.4 GHz; measured
 // 70 to 72); FP64 the same unit with two wavefronts.  Wavefronts in flight: with WAVES = 3 per SIMD a block's loads

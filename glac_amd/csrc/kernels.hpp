@@ -103,6 +103,13 @@ bool flow_measure_fusable(const Geom &g);
 // `sweeps` sweeps' slots.
 constexpr int kCountSlots = 256;
 __device__ __forceinline__ int count_slot(unsigned block) { return (int)(block & (kCountSlots - 1)); }
+// The wavefront's accepted hits into its slot.
+__device__ __forceinline__ void add_count(unsigned long long *count, unsigned wavefront, int n)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(count + count_slot(wavefront), (unsigned long long)n);
+}
 void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, hipStream_t s);
 
 // One checkerboard sub-sweep (mu, parity), in place; accepted hits are added
