@@ -33,6 +33,7 @@ Run ``python bench.py [--steps K] [--warmup W]``; one JSON line on stdout.
 import argparse
 import json
 import os
+import re
 import sys
 import time
 
@@ -76,16 +77,28 @@ def profiled(n, kernels):
     """Mean over `kernels` of the committed rocprofv3 figures per launch
     (profiles/counters_<lattice>.json: SQ counters per wavefront, HBM bytes
     from FETCH_SIZE / WRITE_SIZE), or None when the lattice or a kernel was
-    not profiled."""
+    not profiled.  A kernel is a regular expression of its name, which must fit
+    one of the file's."""
     path = os.path.join(ROOT, "profiles", "counters_%s.json" % "x".join(map(str, n)))
     if not os.path.exists(path):
         return None
     with open(path) as f:
         table = json.load(f)["kernels"]
-    rows = [table.get(k) for k in kernels]
-    if not all(rows):
+    rows = [[r for name, r in table.items() if re.fullmatch(k, name)] for k in kernels]
+    if any(len(r) != 1 for r in rows):
         return None
+    rows = [r[0] for r in rows]
     return {key: sum(r[key] for r in rows) / len(rows) for key in ("waves", "valu_per_wave", "traffic_bytes")}
+
+
+def sweep_kernel(rows):
+    """The FP32 sub-sweep's kernel, whichever of them a lattice's size picks."""
+    return rf"metropolis(_small)?_kernel<float, {rows}(, \d+)+>"
+
+
+def stage0_kernel(rows):
+    """The FP32 flow's measuring stage, likewise."""
+    return rf"flow_stage_kernel<float, {rows}, 0, true>|flow_measure_wide_kernel<float, {rows}>"
 
 
 def valu_issue_frac(prof, launch_ms):
@@ -334,8 +347,8 @@ def main():
     metro_ms = m_ms / max(m_launches, 1)
     metro_gbs = metro_bytes / (metro_ms * 1e-3) / 1e9
     prof_stage = profiled(n, [f"flow_stage_kernel<float, {rows}, {k}, false>" for k in plain_stages])
-    prof_stage0 = profiled(n, [f"flow_stage_kernel<float, {rows}, 0, true>"])
-    prof_metro = profiled(n, [f"metropolis_kernel<float, {rows}, 3>"])
+    prof_stage0 = profiled(n, [stage0_kernel(rows)])
+    prof_metro = profiled(n, [sweep_kernel(rows)])
 
     # ---------------------------------------------------------------- FP64 flow
     fp64 = None
