@@ -32,7 +32,8 @@ struct glacx_ctx {
     double *results = nullptr;       // device results (measurement rows)
     size_t results_len = 0;
     double *host_rows = nullptr;     // kHostRows doubles of pinned host memory, or none
-    unsigned long long *counts = nullptr;  // accepted hits: kCountSlots slots per sweep, then a sum per sweep
+    unsigned long long *counts = nullptr;  // accepted hits: kCountSlots slots for each of kCountSweeps sweeps,
+                                           // then a sum per sweep
     size_t counts_len = 0;
     int *flag = nullptr;             // one int: the SU(3) check's answer
     size_t flag_len = 0;
@@ -680,9 +681,11 @@ namespace {
 // What a chain of sweeps leaves: a plaquette and a count of accepted hits per
 // sweep, in host_rows or in device memory.  The sweeps' plaquette partials wait side
 // by side, as a flow's do, and are summed together: a launch after every sweep took
-// 4.7 of its 174 us at 16^4 FP64.
+// 4.7 of its 174 us at 16^4 FP64.  So do their hit counts, kCountSweeps sweeps' slots
+// (2 MiB) at most: only the sum per sweep grows with the call.
+constexpr int kCountSweeps = 1024;
 struct SweepEnd {
-    int sweeps = 0, slots = 1;
+    int sweeps = 0, slots = 1, count_sweeps = 1;
     double *plaq = nullptr;
     unsigned long long *counts = nullptr;
     bool on_host = false;
@@ -694,14 +697,33 @@ int begin_sweeps(glacx_ctx *c, int n_sweeps, bool plaq, SweepEnd *end)
     static_assert(sizeof(double) == sizeof(unsigned long long), "both in host_rows");
     end->sweeps = n_sweeps;
     end->on_host = c->host_rows && 2 * n <= kHostRows;
-    end->counts = end->on_host ? reinterpret_cast<unsigned long long *>(c->host_rows + n) : c->counts + n * kCountSlots;
+    end->count_sweeps = std::min(n_sweeps, kCountSweeps);
+    const size_t slots = (size_t)end->count_sweeps * kCountSlots;
+    int rc = ensure(c, &c->counts, &c->counts_len, slots + (end->on_host ? 0 : n));
+    if (rc) return rc;
+    HIP_TRY(c, hipMemsetAsync(c->counts, 0, sizeof(unsigned long long) * slots, c->stream));
+    end->counts = end->on_host ? reinterpret_cast<unsigned long long *>(c->host_rows + n) : c->counts + slots;
     if (!plaq) return GLACX_OK;
-    int rc;
     if (!end->on_host && (rc = ensure(c, &c->results, &c->results_len, n))) return rc;
     end->plaq = end->on_host ? c->host_rows : c->results;
     const size_t per = (size_t)plaquette_partials_count(c->geom);
     end->slots = flow_slots(per, n_sweeps - 1, kFlowPartials);
     return ensure(c, &c->partials, &c->partials_len, per * end->slots);
+}
+
+// Sweep i's slots, and what its end is: the slots of a whole batch are summed, and
+// cleared for the next one.
+unsigned long long *sweep_counts(glacx_ctx *c, int i, const SweepEnd &end)
+{
+    return c->counts + (size_t)(i % end.count_sweeps) * kCountSlots;
+}
+int end_sweep(glacx_ctx *c, int i, const SweepEnd &end)
+{
+    const int slot = i % end.count_sweeps;
+    if (slot != end.count_sweeps - 1 && i != end.sweeps - 1) return GLACX_OK;
+    launch_count_sum(c->counts, end.counts + (i - slot), slot + 1, c->stream);
+    CHECK_LAUNCH(c);
+    return GLACX_OK;
 }
 
 int sweep_plaquette(glacx_ctx *c, int i, const SweepEnd &end)
@@ -720,8 +742,6 @@ int sweep_plaquette(glacx_ctx *c, int i, const SweepEnd &end)
 int finish_sweeps(glacx_ctx *c, const SweepEnd &end, int n_hit, double *accept, double *plaq)
 {
     const size_t n = (size_t)end.sweeps;
-    launch_count_sum(c->counts, end.counts, end.sweeps, c->stream);
-    CHECK_LAUNCH(c);
     std::vector<unsigned long long> counts(n);
     if (!end.on_host) {
         HIP_TRY(c, hipMemcpyAsync(counts.data(), end.counts, n * sizeof(unsigned long long), hipMemcpyDeviceToHost,
@@ -747,12 +767,9 @@ int glacx_metropolis(glacx_ctx *c, int n_sweeps, double beta, double eps, int n_
     if (n_sweeps < 0 || n_hit < 1 || !(eps > 0.0 && eps < 1.0))
         return fail(c, GLACX_E_ARG, "metropolis: need n_sweeps >= 0, n_hit >= 1, 0 < eps < 1");
     if (n_sweeps == 0) return GLACX_OK;
-    const size_t slots = (size_t)n_sweeps * kCountSlots;
-    int rc = ensure(c, &c->counts, &c->counts_len, slots + n_sweeps);
-    if (rc) return rc;
-    HIP_TRY(c, hipMemsetAsync(c->counts, 0, sizeof(unsigned long long) * slots, c->stream));
     SweepEnd end;
-    if ((rc = begin_sweeps(c, n_sweeps, plaq != nullptr, &end))) return rc;
+    int rc = begin_sweeps(c, n_sweeps, plaq != nullptr, &end);
+    if (rc) return rc;
     for (int i = 0; i < n_sweeps; i++) {
         MetroParams p;
         p.beta = beta;
@@ -761,7 +778,8 @@ int glacx_metropolis(glacx_ctx *c, int n_sweeps, double beta, double eps, int n_
         p.sweep = sweep_offset + (uint64_t)i;
         p.reunit = reunit_every > 0 && (p.sweep % (uint64_t)reunit_every) == 0;
         p.seed = seed;
-        if ((rc = DISPATCH(c, run_metropolis_sweep, c, p, c->counts + (size_t)i * kCountSlots))) return rc;
+        if ((rc = DISPATCH(c, run_metropolis_sweep, c, p, sweep_counts(c, i, end)))) return rc;
+        if ((rc = end_sweep(c, i, end))) return rc;
         if (plaq && (rc = sweep_plaquette(c, i, end))) return rc;
     }
     return finish_sweeps(c, end, n_hit, accept, plaq);
@@ -1141,12 +1159,9 @@ int glacx_metropolis_learned(glacx_ctx *c, int n_sweeps, double beta, double eps
     if (n_sweeps < 0 || n_hit < 1 || !(eps > 0.0 && eps < 1.0))
         return fail(c, GLACX_E_ARG, "metropolis_learned: need n_sweeps >= 0, n_hit >= 1, 0 < eps < 1");
     if (n_sweeps == 0) return GLACX_OK;
-    const size_t slots = (size_t)n_sweeps * kCountSlots;
-    int rc = ensure(c, &c->counts, &c->counts_len, slots + n_sweeps);
-    if (rc) return rc;
-    HIP_TRY(c, hipMemsetAsync(c->counts, 0, sizeof(unsigned long long) * slots, c->stream));
     SweepEnd end;
-    if ((rc = begin_sweeps(c, n_sweeps, plaq != nullptr, &end))) return rc;
+    int rc = begin_sweeps(c, n_sweeps, plaq != nullptr, &end);
+    if (rc) return rc;
     for (int i = 0; i < n_sweeps; i++) {
         MetroParams p;
         p.beta = beta;
@@ -1155,7 +1170,8 @@ int glacx_metropolis_learned(glacx_ctx *c, int n_sweeps, double beta, double eps
         p.sweep = sweep_offset + (uint64_t)i;
         p.reunit = reunit_every > 0 && (p.sweep % (uint64_t)reunit_every) == 0;
         p.seed = seed;
-        if ((rc = DISPATCH(c, run_metropolis_learned_sweep, c, p, c->counts + (size_t)i * kCountSlots))) return rc;
+        if ((rc = DISPATCH(c, run_metropolis_learned_sweep, c, p, sweep_counts(c, i, end)))) return rc;
+        if ((rc = end_sweep(c, i, end))) return rc;
         if (plaq && (rc = sweep_plaquette(c, i, end))) return rc;
     }
     return finish_sweeps(c, end, n_hit, accept, plaq);

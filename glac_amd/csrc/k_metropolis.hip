@@ -318,19 +318,22 @@ __global__ __launch_bounds__(64 * (STAPLERS + PROPOSERS), STAPLERS > 1 ? 4 : 2) 
     add_count(count, blockIdx.x, valid ? accepted : 0);
 }
 
-__global__ __launch_bounds__(64) void count_sum_kernel(const unsigned long long *__restrict__ slots,
+__global__ __launch_bounds__(64) void count_sum_kernel(unsigned long long *__restrict__ slots,
                                                        unsigned long long *__restrict__ counts)
 {
-    const unsigned long long *p = slots + (size_t)blockIdx.x * kCountSlots;
+    unsigned long long *p = slots + (size_t)blockIdx.x * kCountSlots;
     unsigned long long n = 0;
 #pragma unroll
-    for (int k = threadIdx.x; k < kCountSlots; k += 64) n += p[k];
+    for (int k = threadIdx.x; k < kCountSlots; k += 64) {
+        n += p[k];
+        p[k] = 0;
+    }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
     if (threadIdx.x == 0) counts[blockIdx.x] = n;
 }
 
-void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, hipStream_t s)
+void launch_count_sum(unsigned long long *slots, unsigned long long *counts, int sweeps, hipStream_t s)
 {
     count_sum_kernel<<<sweeps, 64, 0, s>>>(slots, counts);
 }

@@ -100,7 +100,7 @@ bool flow_measure_fusable(const Geom &g);
 // Accepted hits of a sweep are counted in kCountSlots slots, block b's in slot
 // b % kCountSlots: on one address the blocks of a small lattice, which end
 // together, queue for 5 of their 18 us (512 blocks).  launch_count_sum adds up
-// `sweeps` sweeps' slots.
+// `sweeps` sweeps' slots and leaves them cleared.
 constexpr int kCountSlots = 256;
 __device__ __forceinline__ int count_slot(unsigned block) { return (int)(block & (kCountSlots - 1)); }
 // The wavefront's accepted hits into its slot.
@@ -110,7 +110,7 @@ __device__ __forceinline__ void add_count(unsigned long long *count, unsigned wa
     for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
     if ((threadIdx.x & 63) == 0) atomicAdd(count + count_slot(wavefront), (unsigned long long)n);
 }
-void launch_count_sum(const unsigned long long *slots, unsigned long long *counts, int sweeps, hipStream_t s);
+void launch_count_sum(unsigned long long *slots, unsigned long long *counts, int sweeps, hipStream_t s);
 
 // One checkerboard sub-sweep (mu, parity), in place; accepted hits are added
 // to the sweep's slots at `count`.
