@@ -10,7 +10,8 @@
 // page faults do (15 ms down), eight gain nothing.  The line lies at 16 MiB:
 // 24 MB still go faster (up 0.71 -> 0.68 ms, down 1.35 -> 0.73), 4.7 MB go up no
 // faster (0.21 and 0.23 ms) and would not earn back the pinned memory's
-// allocation (0.75 ms, once per context).
+// allocation (0.75 ms, once per context).  Arrays that the runtime knows (pinned
+// or managed ones) it copies by itself at the link's rate.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -47,17 +48,24 @@ public:
     {
         size_t total = 0;
         for (const HostSpan &s : spans) total += s.bytes;
+        std::vector<HostSpan> direct, sliced;
+        for (const HostSpan &s : spans) (total >= kLeast && ordinary(s.host) ? sliced : direct).push_back(s);
+        total = 0;
+        for (const HostSpan &s : sliced) total += s.bytes;
         if (total < kLeast || !acquire()) {
-            for (const HostSpan &s : spans) {
-                const hipError_t e = up ? hipMemcpyAsync(s.dev, s.host, s.bytes, hipMemcpyHostToDevice, stream)
-                                        : hipMemcpyAsync(s.host, s.dev, s.bytes, hipMemcpyDeviceToHost, stream);
-                if (e != hipSuccess) return e;
-            }
-            return up ? hipSuccess : hipStreamSynchronize(stream);
+            direct.insert(direct.end(), sliced.begin(), sliced.end());
+            sliced.clear();
         }
+        for (const HostSpan &s : direct) {
+            const hipError_t e = up ? hipMemcpyAsync(s.dev, s.host, s.bytes, hipMemcpyHostToDevice, stream)
+                                    : hipMemcpyAsync(s.host, s.dev, s.bytes, hipMemcpyDeviceToHost, stream);
+            if (e != hipSuccess) return e;
+        }
+        if (sliced.empty()) return up ? hipSuccess : hipStreamSynchronize(stream);
         std::vector<HostSpan> slices;
-        for (const HostSpan &s : spans)
-            for (size_t o = 0; o < s.bytes; o += kSlice) slices.push_back({s.host + o, s.dev + o, std::min(kSlice, s.bytes - o)});
+        for (const HostSpan &s : sliced)
+            for (size_t o = 0; o < s.bytes; o += kSlice)
+                slices.push_back({s.host + o, s.dev + o, std::min(kSlice, s.bytes - o)});
         std::atomic<size_t> next{0};
         std::atomic<int> status{hipSuccess};
         auto work = [&](int w) {
@@ -80,6 +88,15 @@ public:
     }
 
 private:
+    // Memory that the runtime knows nothing of: from malloc, the stack, a mapped file.
+    static bool ordinary(const void *p)
+    {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+        (void)hipGetLastError();
+        return true;
+    }
+
     char *slice(int w, int k) { return pinned_ + (size_t)(2 * w + k) * kSlice; }
     hipEvent_t event(int w, int k) { return events_[2 * w + k]; }
 
