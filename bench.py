@@ -98,7 +98,12 @@ def sweep_kernel(rows):
 
 def stage0_kernel(rows):
     """The FP32 flow's measuring stage, likewise."""
-    return rf"flow_stage_kernel<float, {rows}, 0, true>|flow_measure_wide_kernel<float, {rows}>"
+    return rf"flow_stage_kernel<float, {rows}, 0, true(, \w+)*>|flow_measure_wide_kernel<float, {rows}>"
+
+
+def plain_stage_kernel(rows, stage):
+    """A plain FP32 flow stage, whatever it streams."""
+    return rf"flow_stage_kernel<float, {rows}, {stage}, false(, \w+)*>"
 
 
 def valu_issue_frac(prof, launch_ms):
@@ -346,7 +351,7 @@ def main():
     metro_bytes = metropolis_bytes_per_launch(V, True, rows)
     metro_ms = m_ms / max(m_launches, 1)
     metro_gbs = metro_bytes / (metro_ms * 1e-3) / 1e9
-    prof_stage = profiled(n, [f"flow_stage_kernel<float, {rows}, {k}, false>" for k in plain_stages])
+    prof_stage = profiled(n, [plain_stage_kernel(rows, k) for k in plain_stages])
     prof_stage0 = profiled(n, [stage0_kernel(rows)])
     prof_metro = profiled(n, [sweep_kernel(rows)])
 

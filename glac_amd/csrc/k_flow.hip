@@ -66,61 +66,57 @@ template <class T> using FlowLds = LdsMats<T, 8>;
 //                 16^3 x 48        216  264     101.7   100.2   109.3
 //                 24^3 x 48        729  891     390.2   380.1   370.1
 enum StreamBits : unsigned { kStreamAcc = 1, kStreamLinks = 2 };
-// One direction's accumulator as a buffer of 8 V reals.  Buffer accesses carry the
-// policy as an operand; of plain ones in the two arms of a branch the compiler makes
-// one, without it.
-template <class T> __device__ __forceinline__ __amdgpu_buffer_rsrc_t acc_view(const T *acc, const Geom &g, int mu)
-{
-    return __builtin_amdgcn_make_buffer_rsrc((void *)(acc + (size_t)mu * 8 * g.v), (short)0,
-                                             (int)(8u * (unsigned)g.v * (unsigned)sizeof(T)), kBufferFlags);
-}
+// The kernels take the bits as a template parameter: tested at run time they cost
+// a stage of a small lattice 0.1 to 0.2 us (8^4 compressed 7.93 us without, 8.11 with).
 using AccVec = unsigned __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ AccVec acc_get(__amdgpu_buffer_rsrc_t r, const Geom &g, int idx, int plane, bool stream)
+template <bool STREAM, class V> __device__ __forceinline__ V acc_get(const V *p)
 {
-    const unsigned off = (unsigned)idx * 16u, at = (unsigned)plane * 16u * (unsigned)g.v;
-    return stream ? __builtin_amdgcn_raw_buffer_load_b128(r, off, at, store_policy<true>())
-                  : __builtin_amdgcn_raw_buffer_load_b128(r, off, at, store_policy<false>());
-}
-__device__ __forceinline__ void acc_put(__amdgpu_buffer_rsrc_t r, const Geom &g, int idx, int plane, bool stream, AccVec v)
-{
-    const unsigned off = (unsigned)idx * 16u, at = (unsigned)plane * 16u * (unsigned)g.v;
-    if (stream)
-        __builtin_amdgcn_raw_buffer_store_b128(v, r, off, at, store_policy<true>());
+    if constexpr (STREAM)
+        return __builtin_bit_cast(V, __builtin_nontemporal_load(reinterpret_cast<const AccVec *>(p)));
     else
-        __builtin_amdgcn_raw_buffer_store_b128(v, r, off, at, store_policy<false>());
+        return *p;
 }
-__device__ __forceinline__ void acc_store(float *acc, const Geom &g, int mu, int idx, const su3alg<float> &z, bool stream)
+template <bool STREAM, class V> __device__ __forceinline__ void acc_put(V *p, const V &v)
 {
-    const auto r = acc_view(acc, g, mu);
-    acc_put(r, g, idx, 0, stream, __builtin_bit_cast(AccVec, make_float4(z.a0, z.a1, z.p[0], z.p[1])));
-    acc_put(r, g, idx, 1, stream, __builtin_bit_cast(AccVec, make_float4(z.p[2], z.p[3], z.p[4], z.p[5])));
+    if constexpr (STREAM)
+        __builtin_nontemporal_store(__builtin_bit_cast(AccVec, v), reinterpret_cast<AccVec *>(p));
+    else
+        *p = v;
 }
-__device__ __forceinline__ su3alg<float> acc_load(const float *acc, const Geom &g, int mu, int idx, bool stream)
+template <bool STREAM>
+__device__ __forceinline__ void acc_store(float *acc, const Geom &g, int mu, int idx, const su3alg<float> &z)
 {
-    const auto r = acc_view(acc, g, mu);
-    const float4 u = __builtin_bit_cast(float4, acc_get(r, g, idx, 0, stream));
-    const float4 v = __builtin_bit_cast(float4, acc_get(r, g, idx, 1, stream));
+    float4 *q = reinterpret_cast<float4 *>(acc) + (size_t)mu * 2 * g.v + idx;
+    acc_put<STREAM>(q, make_float4(z.a0, z.a1, z.p[0], z.p[1]));
+    acc_put<STREAM>(q + g.v, make_float4(z.p[2], z.p[3], z.p[4], z.p[5]));
+}
+template <bool STREAM>
+__device__ __forceinline__ su3alg<float> acc_load(const float *acc, const Geom &g, int mu, int idx)
+{
+    const float4 *q = reinterpret_cast<const float4 *>(acc) + (size_t)mu * 2 * g.v + idx;
+    const float4 u = acc_get<STREAM>(q), v = acc_get<STREAM>(q + g.v);
     su3alg<float> z;
     z.a0 = u.x, z.a1 = u.y, z.p[0] = u.z, z.p[1] = u.w, z.p[2] = v.x, z.p[3] = v.y, z.p[4] = v.z, z.p[5] = v.w;
     return z;
 }
-__device__ __forceinline__ void acc_store(double *acc, const Geom &g, int mu, int idx, const su3alg<double> &z, bool stream)
+template <bool STREAM>
+__device__ __forceinline__ void acc_store(double *acc, const Geom &g, int mu, int idx, const su3alg<double> &z)
 {
-    const auto r = acc_view(acc, g, mu);
-    acc_put(r, g, idx, 0, stream, __builtin_bit_cast(AccVec, make_double2(z.a0, z.a1)));
+    double2 *q = reinterpret_cast<double2 *>(acc) + (size_t)mu * 4 * g.v + idx;
+    acc_put<STREAM>(q, make_double2(z.a0, z.a1));
 #pragma unroll
-    for (int k = 0; k < 3; k++)
-        acc_put(r, g, idx, k + 1, stream, __builtin_bit_cast(AccVec, make_double2(z.p[2 * k], z.p[2 * k + 1])));
+    for (int k = 0; k < 3; k++) acc_put<STREAM>(q + (size_t)(k + 1) * g.v, make_double2(z.p[2 * k], z.p[2 * k + 1]));
 }
-__device__ __forceinline__ su3alg<double> acc_load(const double *acc, const Geom &g, int mu, int idx, bool stream)
+template <bool STREAM>
+__device__ __forceinline__ su3alg<double> acc_load(const double *acc, const Geom &g, int mu, int idx)
 {
-    const auto r = acc_view(acc, g, mu);
+    const double2 *q = reinterpret_cast<const double2 *>(acc) + (size_t)mu * 4 * g.v + idx;
     su3alg<double> z;
-    const double2 u = __builtin_bit_cast(double2, acc_get(r, g, idx, 0, stream));
+    const double2 u = acc_get<STREAM>(q);
     z.a0 = u.x, z.a1 = u.y;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        const double2 v = __builtin_bit_cast(double2, acc_get(r, g, idx, k + 1, stream));
+        const double2 v = acc_get<STREAM>(q + (size_t)(k + 1) * g.v);
         z.p[2 * k] = v.x, z.p[2 * k + 1] = v.y;
     }
     return z;
@@ -194,14 +190,14 @@ template <class T> __device__ __forceinline__ FlowMeasLds<T> &flow_meas_lds()
 
 // The end of a stage for one link: RK3 combination of the force z with the
 // accumulator, exp, product with the link u, and in FP32 the projection.
-template <class T, int R, int STAGE>
+template <class T, int R, int STAGE, unsigned STREAM>
 __device__ __forceinline__ void finish_link(typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc, const Geom &g,
                                             int mu, int idx, const M3<T> &u, const su3alg<T> &z, const su3alg<T> &cacc,
-                                            T cz, T ca, unsigned stream)
+                                            T cz, T ca)
 {
     su3alg<T> y;
     if constexpr (STAGE == 0) {
-        acc_store(acc, g, mu, idx, z, stream & kStreamAcc);
+        acc_store<(STREAM & kStreamAcc) != 0>(acc, g, mu, idx, z);
         y.a0 = cz * z.a0;
         y.a1 = cz * z.a1;
 #pragma unroll
@@ -211,7 +207,7 @@ __device__ __forceinline__ void finish_link(typename vec2<T>::type *__restrict__
         y.a1 = cz * z.a1 - ca * cacc.a1;
 #pragma unroll
         for (int k = 0; k < 6; k++) y.p[k] = cz * z.p[k] - ca * cacc.p[k];
-        if (STAGE == 1) acc_store(acc, g, mu, idx, y, stream & kStreamAcc);
+        if (STAGE == 1) acc_store<(STREAM & kStreamAcc) != 0>(acc, g, mu, idx, y);
     }
     M3<T> w = zero3<T>();
     mm<false, false, false, R>(w, exp_su3(y), u);  // two rows suffice when two are stored
@@ -233,10 +229,7 @@ __device__ __forceinline__ void finish_link(typename vec2<T>::type *__restrict__
             orthonormalize_rows<true>(d);
         w = convert<T>(d);
     }
-    if (stream & kStreamLinks)
-        store_link<T, R, true>(dir_view<T>(wout, g, mu), idx, w);
-    else
-        store_link<T, R, false>(dir_view<T>(wout, g, mu), idx, w);
+    store_link<T, R, (STREAM & kStreamLinks) != 0>(dir_view<T>(wout, g, mu), idx, w);
 }
 
 // Z = -1/2 T(U A), the form force_from_omega evaluates
@@ -281,12 +274,10 @@ __device__ __forceinline__ void measure_block(const Geom &g, int hb, int mu, T p
 #ifndef GLACX_FP64_FLOW_WAVES
 #define GLACX_FP64_FLOW_WAVES 2
 #endif
-
-template <class T, int R, int STAGE, bool MEAS>
-__global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP64_FLOW_WAVES) void flow_stage_kernel(const typename vec2<T>::type *__restrict__ win,
-                                                            typename vec2<T>::type *__restrict__ wout,
-                                                            T *__restrict__ acc, Geom g, T cz, T ca, unsigned stream,
-                                                            double *__restrict__ meas)
+template <class T, int R, int STAGE, bool MEAS, unsigned STREAM>
+__global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP64_FLOW_WAVES) void flow_stage_kernel(
+    const typename vec2<T>::type *__restrict__ win, typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc, Geom g,
+    T cz, T ca, double *__restrict__ meas)
 {
     static_assert(!MEAS || (STAGE == 0 && sizeof(T) == 4), "the measurement is fused into stage 0 only, FP64 has its own");
     __shared__ FlowLds<T> sh;
@@ -302,7 +293,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
     // passes under the staple loop instead of stalling the step after it; FP64 has
     // no registers left for it (with it in place early, 504 for 391 us)
     su3alg<T> cacc;
-    if constexpr (STAGE != 0 && sizeof(T) == 4) cacc = acc_load(acc, g, mu, idx, stream & kStreamAcc);
+    if constexpr (STAGE != 0 && sizeof(T) == 4) cacc = acc_load<(STREAM & kStreamAcc) != 0>(acc, g, mu, idx);
     const DirView<T> vmu = dir_view<T>(win, g, mu);
     // the site's neighbours x + mu and x - mu, shared with the other
     // wavefronts, whose staples step the same way in direction mu
@@ -332,11 +323,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
         const int p = (lane >> 5) ^ (same_parity ? 0 : 1), r = at - (p ? base1 : base0);
         return (unsigned)r < 32u ? p * 32 + r : -1;
     };
-    auto gather = [&](const DirView<T> &d, int at, int slot) -> M3<T> {
-        if constexpr (kNear)
-            return load_link_at(d, slot >= 0 ? kNoLink : tile_off(at));
-        else
-            return load_link<T, R>(d, at);
+    auto gather = [&](const auto &d, int at, int slot) {
+        return load_link_at(d, slot >= 0 ? kNoLink : tile_off(at));
     };
     auto take_near = [&](M3<T> &m, bool xy, int d, int slot) {
         if (near && xy) {
@@ -474,7 +462,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
                 mm<false, false, false, 2>(q, load_rows01<T, R>(vmu, imn), load_link<T, R>(vnu, ipmmn));
                 rebuild_third_row(q);
                 mm<true, false, true>(a, q, back_link(nu));
-            } else if constexpr (sizeof(T) == 8) {
+            } else if constexpr (kNear) {
                 // two waves per SIMD leave registers for all four gathers of the
                 // term in flight at once (24^3 x 48 479 -> 454 us)
                 const int sm = near_slot(mu < 2, ipm, false), sp = near_slot(nu < 2, ipn, false),
@@ -515,7 +503,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
             }
         }
     }
-    if constexpr (STAGE != 0 && sizeof(T) == 8) cacc = acc_load(acc, g, mu, idx, stream & kStreamAcc);
+    if constexpr (STAGE != 0 && sizeof(T) == 8) cacc = acc_load<(STREAM & kStreamAcc) != 0>(acc, g, mu, idx);
     if (valid) {
         const M3<T> u = lds_get(sh, mu, lane);
         su3alg<T> z;
@@ -524,7 +512,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
         } else {
             z = force_from_omega(mul(u, a));
         }
-        finish_link<T, R, STAGE>(wout, acc, g, mu, idx, u, z, cacc, cz, ca, stream);
+        finish_link<T, R, STAGE, STREAM>(wout, acc, g, mu, idx, u, z, cacc, cz, ca);
     }
     if constexpr (MEAS) {
         // every lane is a real site here (the launch requires whole chunks)
@@ -560,10 +548,10 @@ struct Measure64Lds {
     };
 };
 
+template <unsigned STREAM>
 __global__ __launch_bounds__(kBlock, 2) void flow_measure64_kernel(const double2 *__restrict__ win,
                                                                    double2 *__restrict__ wout, double *__restrict__ acc,
-                                                                   Geom g, double cz, unsigned stream,
-                                                                   double *__restrict__ meas)
+                                                                   Geom g, double cz, double *__restrict__ meas)
 {
     using T = double;
     constexpr int R = 3;
@@ -636,7 +624,7 @@ __global__ __launch_bounds__(kBlock, 2) void flow_measure64_kernel(const double2
         form(tz);
     }
     const su3alg<T> z = force_from_ta2(tz);
-    finish_link<T, R, 0>(wout, acc, g, mu, idx, lds_get(lds.sh, mu, lane), z, z, cz, 0.0, stream);
+    finish_link<T, R, 0, STREAM>(wout, acc, g, mu, idx, lds_get(lds.sh, mu, lane), z, z, cz, 0.0);
     __syncthreads();  // the shared links are done with
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -828,7 +816,8 @@ __global__ __launch_bounds__(3 * kBlock, 3) void flow_measure_wide_kernel(const 
         z = force_from_omega(mul(u, a));
     else
         z = force_from_ta2(tz);
-    finish_link<T, R, 0>(wout, acc, g, mu, idx, u, z, z, cz, T(0), kStreamAcc | kStreamLinks);  // fields below 32 MiB
+    // streaming both: the fields are below 18 MiB
+    finish_link<T, R, 0, kStreamAcc | kStreamLinks>(wout, acc, g, mu, idx, u, z, z, cz, T(0));
     T fa[8], fb[8];
     if (mu < 3) {
 #pragma unroll
@@ -851,44 +840,56 @@ __global__ __launch_bounds__(3 * kBlock, 3) void flow_measure_wide_kernel(const 
 // every lattice with bz Ny Nx / 2 divisible by 32.
 bool flow_measure_fusable(const Geom &g) { return g.run % (kFlowSites / 2) == 0; }
 
-template <class T, int R>
-void launch_flow_stage(const void *win, void *wout, void *acc, const Geom &g, int stage, double eps, double *meas,
-                       hipStream_t s)
+template <class T, int R, unsigned STREAM>
+static void launch_stage(const void *win, void *wout, void *acc, const Geom &g, int stage, double eps, double *meas,
+                         hipStream_t s)
 {
     using V2 = typename vec2<T>::type;
     const unsigned blocks = (unsigned)((g.vh + kFlowSites / 2 - 1) / (kFlowSites / 2));
     const V2 *in = (const V2 *)win;
     V2 *out = (V2 *)wout;
     T *a = (T *)acc;
-    const size_t fields = (size_t)2 * 4 * g.v * 6 * R * sizeof(T), accumulator = (size_t)32 * g.v * sizeof(T);
-    constexpr size_t kInfinityCache = (size_t)256 << 20;
-    const unsigned stream = fields < ((size_t)32 << 20) ? kStreamAcc | kStreamLinks
-                                                        : (fields + accumulator >= kInfinityCache ? kStreamAcc : 0u) |
-                                                              (fields > kInfinityCache ? kStreamLinks : 0u);
     switch (stage) {
     case 0:
         if (meas) {
             if (blocks <= kWideBlocks)
                 flow_measure_wide_kernel<T, R><<<blocks, 3 * kBlock, 0, s>>>(in, out, a, g, T(0.25 * eps), meas);
             else if constexpr (sizeof(T) == 8)
-                flow_measure64_kernel<<<blocks, kBlock, 0, s>>>(in, out, a, g, T(0.25 * eps), stream, meas);
+                flow_measure64_kernel<STREAM><<<blocks, kBlock, 0, s>>>(in, out, a, g, T(0.25 * eps), meas);
             else
-                flow_stage_kernel<T, R, 0, true>
-                    <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), stream, meas);
+                flow_stage_kernel<T, R, 0, true, STREAM>
+                    <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), meas);
             break;
         }
-        flow_stage_kernel<T, R, 0, false>
-            <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), stream, nullptr);
+        flow_stage_kernel<T, R, 0, false, STREAM>
+            <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), nullptr);
         break;
     case 1:
-        flow_stage_kernel<T, R, 1, false><<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(
-            in, out, a, g, T(8.0 / 9.0 * eps), T(17.0 / 36.0 * eps), stream, nullptr);
+        flow_stage_kernel<T, R, 1, false, STREAM><<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(
+            in, out, a, g, T(8.0 / 9.0 * eps), T(17.0 / 36.0 * eps), nullptr);
         break;
     default:
-        flow_stage_kernel<T, R, 2, false>
-            <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.75 * eps), T(1), stream, nullptr);
+        flow_stage_kernel<T, R, 2, false, STREAM>
+            <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.75 * eps), T(1), nullptr);
         break;
     }
+}
+
+template <class T, int R>
+void launch_flow_stage(const void *win, void *wout, void *acc, const Geom &g, int stage, double eps, double *meas,
+                       hipStream_t s)
+{
+    // the table at StreamBits
+    const size_t fields = (size_t)2 * 4 * g.v * 6 * R * sizeof(T), accumulator = (size_t)32 * g.v * sizeof(T);
+    constexpr size_t kInfinityCache = (size_t)256 << 20;
+    constexpr size_t kL2 = (size_t)32 << 20;
+    constexpr unsigned kBoth = kStreamAcc | kStreamLinks;
+    if (fields < kL2 || fields > kInfinityCache)
+        launch_stage<T, R, kBoth>(win, wout, acc, g, stage, eps, meas, s);
+    else if (fields + accumulator >= kInfinityCache)
+        launch_stage<T, R, kStreamAcc>(win, wout, acc, g, stage, eps, meas, s);
+    else
+        launch_stage<T, R, 0>(win, wout, acc, g, stage, eps, meas, s);
 }
 
 template void launch_flow_stage<float, 3>(const void *, void *, void *, const Geom &, int, double, double *,

@@ -27,6 +27,7 @@ def test_sweep_kernel(tmp_path, monkeypatch, name, found):
 
 
 @pytest.mark.parametrize("name, found", [("flow_stage_kernel<float, 2, 0, true>", True),
+                                         ("flow_stage_kernel<float, 2, 0, true, 3u, false>", True),
                                          ("flow_measure_wide_kernel<float, 2>", True),
                                          ("flow_stage_kernel<float, 2, 0, false>", False),
                                          ("flow_measure_wide_kernel<double, 3>", False)])
@@ -41,5 +42,6 @@ def test_measuring_stage(tmp_path, monkeypatch, name, found):
 def test_committed_counters():
     n = (32, 32, 32, 32)
     assert bench.profiled(n, [bench.sweep_kernel(2)])["waves"] == 8192
-    assert bench.profiled(n, [f"flow_stage_kernel<float, 2, {k}, false>" for k in (1, 2)])["waves"] == 65536
-    assert bench.profiled(n, ["flow_stage_kernel<float, 3, 1, false>"]) is None
+    assert bench.profiled(n, [bench.plain_stage_kernel(2, k) for k in (1, 2)])["waves"] == 65536
+    assert bench.profiled(n, [bench.stage0_kernel(2)])["waves"] == 65536
+    assert bench.profiled(n, [bench.plain_stage_kernel(3, 1)]) is None
