@@ -274,7 +274,17 @@ __device__ __forceinline__ void measure_block(const Geom &g, int hb, int mu, T p
 #ifndef GLACX_FP64_FLOW_WAVES
 #define GLACX_FP64_FLOW_WAVES 2
 #endif
-template <class T, int R, int STAGE, bool MEAS, unsigned STREAM>
+// FP64 plain stages of at most kFewBlocks blocks gather a term's links in two pairs and
+// all from memory: their wavefronts have at most two SIMD-mates, and what they wait
+// for is the first pair, behind which the other loads and the look for near links
+// only queue.  Larger launches are bound by requests (see near_slot) and have all four
+// in flight.  Microseconds of a stage by blocks, few and many:
+//     blocks      1      64     324     480     768     850    1024    1296    1980
+//     few        8.3   11.2    17.3    18.9    26.6    33.2    33.6    46.6    66.3
+//     many       9.3   11.4    18.6    19.4    27.2    33.2    33.6    45.6    62.7
+constexpr int kFewBlocks = 768;
+
+template <class T, int R, int STAGE, bool MEAS, unsigned STREAM, bool FEW = false>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP64_FLOW_WAVES) void flow_stage_kernel(
     const typename vec2<T>::type *__restrict__ win, typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc, Geom g,
     T cz, T ca, double *__restrict__ meas)
@@ -315,7 +325,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
     // can have on their way at a time (load the links and multiply nothing, and
     // they take as long); this saves a fifth of the requests: 24^3 x 48 415 -> 391
     // and 387 -> 360 us.  The measuring stage has no registers for it (596 -> 645).
-    constexpr bool kNear = sizeof(T) == 8 && !MEAS;
+    constexpr bool kNear = sizeof(T) == 8 && !MEAS && !FEW;
     const bool near = kNear && (g.bh & 31) == 0;
     const int base0 = kNear ? parity_index(g, 0, hb * (kFlowSites / 2)) : 0, base1 = base0 + g.bh;
     auto near_slot = [&](bool xy, int at, bool same_parity) -> int {
@@ -840,7 +850,7 @@ __global__ __launch_bounds__(3 * kBlock, 3) void flow_measure_wide_kernel(const 
 // every lattice with bz Ny Nx / 2 divisible by 32.
 bool flow_measure_fusable(const Geom &g) { return g.run % (kFlowSites / 2) == 0; }
 
-template <class T, int R, unsigned STREAM>
+template <class T, int R, unsigned STREAM, bool FEW>
 static void launch_stage(const void *win, void *wout, void *acc, const Geom &g, int stage, double eps, double *meas,
                          hipStream_t s)
 {
@@ -861,15 +871,15 @@ static void launch_stage(const void *win, void *wout, void *acc, const Geom &g, 
                     <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), meas);
             break;
         }
-        flow_stage_kernel<T, R, 0, false, STREAM>
+        flow_stage_kernel<T, R, 0, false, STREAM, FEW>
             <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.25 * eps), T(0), nullptr);
         break;
     case 1:
-        flow_stage_kernel<T, R, 1, false, STREAM><<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(
+        flow_stage_kernel<T, R, 1, false, STREAM, FEW><<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(
             in, out, a, g, T(8.0 / 9.0 * eps), T(17.0 / 36.0 * eps), nullptr);
         break;
     default:
-        flow_stage_kernel<T, R, 2, false, STREAM>
+        flow_stage_kernel<T, R, 2, false, STREAM, FEW>
             <<<blocks, kBlock, GLACX_FLOW_LDS_BYTES, s>>>(in, out, a, g, T(0.75 * eps), T(1), nullptr);
         break;
     }
@@ -884,12 +894,24 @@ void launch_flow_stage(const void *win, void *wout, void *acc, const Geom &g, in
     constexpr size_t kInfinityCache = (size_t)256 << 20;
     constexpr size_t kL2 = (size_t)32 << 20;
     constexpr unsigned kBoth = kStreamAcc | kStreamLinks;
-    if (fields < kL2 || fields > kInfinityCache)
-        launch_stage<T, R, kBoth>(win, wout, acc, g, stage, eps, meas, s);
+    if constexpr (sizeof(T) == 8) {
+        if (g.vh <= kFewBlocks * (kFlowSites / 2)) {  // the table at kFewBlocks
+            if (fields < kL2)
+                launch_stage<T, R, kBoth, true>(win, wout, acc, g, stage, eps, meas, s);
+            else
+                launch_stage<T, R, 0, true>(win, wout, acc, g, stage, eps, meas, s);
+            return;
+        }
+    } else if (fields < kL2) {
+        launch_stage<T, R, kBoth, false>(win, wout, acc, g, stage, eps, meas, s);
+        return;
+    }
+    if (fields > kInfinityCache)
+        launch_stage<T, R, kBoth, false>(win, wout, acc, g, stage, eps, meas, s);
     else if (fields + accumulator >= kInfinityCache)
-        launch_stage<T, R, kStreamAcc>(win, wout, acc, g, stage, eps, meas, s);
+        launch_stage<T, R, kStreamAcc, false>(win, wout, acc, g, stage, eps, meas, s);
     else
-        launch_stage<T, R, 0>(win, wout, acc, g, stage, eps, meas, s);
+        launch_stage<T, R, 0, false>(win, wout, acc, g, stage, eps, meas, s);
 }
 
 template void launch_flow_stage<float, 3>(const void *, void *, void *, const Geom &, int, double, double *,
