@@ -48,21 +48,33 @@ template <class T> using FlowLds = LdsMats<T, 8>;
 // Cache's 256 MiB hold what the next stage reads, that throws away what it would
 // find there.  So the accumulator is streamed once the two fields and it take
 // 256 MiB, the links once the two fields alone exceed that.  Both are also while
-// the two fields fit in the eight L2s (32 MiB), where a launch otherwise ends with
-// writing out what they hold: twenty steps of 12 x 10 x 14 x 18 FP32 994 us for
-// 1054, forty of 8^3 x 16 FP64 1550 for 1584; 16^4 FP64 (72 MiB) is the other way,
-// 39.6 us a stage for 36.5.  Microseconds of a plain stage, with nothing, the
-// accumulator, and both streamed:
+// fields and accumulator fit in the eight L2s (32 MiB) or nearly, where a launch
+// otherwise ends with writing out what they hold: two fields below 28 MiB in
+// FP32; below 16 in FP64, whose gathers find less in a cache that streams.
+// Microseconds of a plain stage, with nothing, the accumulator, and both streamed:
 //     MiB of two fields, with accumulator    nothing     acc    both
-//     compressed  16^2 x 32 x 48   144  192      81.0    84.8    87.7
+//     compressed  10 x 16^2 x 12    11   15      10.9            10.4
+//                 16^3 x 12         18   24      14.0            13.3
+//                 16^4              24   32      17.5            17.3
+//                 16^2 x 18^2       30   41      22.3            22.9
+//                 16^3 x 24         36   48      23.2            24.3
+//                 16^2 x 32 x 48   144  192      81.0    84.8    87.7
 //                 32^3 x 16        192  256     115.8   114.1   117.5
 //                 24^3 x 48        243  324     163.8   145.5   160.1
 //                 32^3 x 24        288  384     189.0   183.9   179.6
 //                 48^3 x 96       3888 5184      2633    2593    2555
-//     FP32        24^4             182  223      89.6    96.3   109.1
+//     FP32        12x10x14x18       17   20      12.9            11.8
+//                 16^3 x 12         27   33      16.7            16.2
+//                 14x18x22x10       30   37      21.0            21.2
+//                 16^2 x 18^2       46   56      26.8            28.8
+//                 24^4             182  223      89.6    96.3   109.1
 //                 32^3 x 16        288  352     168.1   160.9   162.9
 //                 32^4             576  704       344     323     315
-//     FP64        16^3 x 32        144  176      65.9    70.6    75.4
+//     FP64        8^3 x 16           9   11      11.7            11.5
+//                 10 x 12^2 x 10    16   19      12.8            12.8
+//                 12^4              23   28      17.3            18.0
+//                 16^4              72   88      33.6            37.6
+//                 16^3 x 32        144  176      65.9    70.6    75.4
 //                 16^3 x 48        216  264     101.7   100.2   109.3
 //                 24^3 x 48        729  891     390.2   380.1   370.1
 enum StreamBits : unsigned { kStreamAcc = 1, kStreamLinks = 2 };
@@ -892,7 +904,7 @@ void launch_flow_stage(const void *win, void *wout, void *acc, const Geom &g, in
     // the table at StreamBits
     const size_t fields = (size_t)2 * 4 * g.v * 6 * R * sizeof(T), accumulator = (size_t)32 * g.v * sizeof(T);
     constexpr size_t kInfinityCache = (size_t)256 << 20;
-    constexpr size_t kL2 = (size_t)32 << 20;
+    constexpr size_t kL2 = (size_t)(sizeof(T) == 8 ? 16 : 28) << 20;
     constexpr unsigned kBoth = kStreamAcc | kStreamLinks;
     if constexpr (sizeof(T) == 8) {
         if (g.vh <= kFewBlocks * (kFlowSites / 2)) {  // the table at kFewBlocks
