@@ -150,10 +150,11 @@ int ensure_stage(glacx_ctx *c)
 // other, or back (null arrays are passed over).
 int copy_host(glacx_ctx *c, double *dev, const double *const *host, int arrays, size_t n, bool up)
 {
-    std::vector<HostSpan> spans;
+    HostSpan spans[Transfer::kMostSpans];
+    int m = 0;
     for (int k = 0; k < arrays; k++)
-        if (host[k]) spans.push_back({(char *)host[k], (char *)(dev + (size_t)k * n), n * sizeof(double)});
-    HIP_TRY(c, c->transfer.run(spans, up, c->device, c->stream));
+        if (host[k]) spans[m++] = {(char *)host[k], (char *)(dev + (size_t)k * n), n * sizeof(double)};
+    HIP_TRY(c, c->transfer.run(spans, m, up, c->device, c->stream));
     return GLACX_OK;
 }
 

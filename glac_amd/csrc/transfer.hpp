@@ -20,7 +20,6 @@
 #include <cstddef>
 #include <cstring>
 #include <thread>
-#include <vector>
 
 namespace glacx {
 
@@ -34,43 +33,40 @@ struct HostSpan {
 class Transfer {
 public:
     static constexpr size_t kSlice = (size_t)4 << 20, kLeast = (size_t)16 << 20;
-    static constexpr int kThreads = 4;
+    static constexpr int kThreads = 4, kMostSpans = 4;
 
     Transfer() = default;
     Transfer(const Transfer &) = delete;
     Transfer &operator=(const Transfer &) = delete;
     ~Transfer() { release(); }
 
-    // Copies every span on `stream`, to the device (`up`) or to the host, behind
-    // the work already there.  A copy to the host is complete on return; one to
-    // the device may be used by what is launched on the stream afterwards.
-    hipError_t run(const std::vector<HostSpan> &spans, bool up, int device, hipStream_t stream)
+    // Copies `n` spans (kMostSpans at most) on `stream`, to the device (`up`) or to
+    // the host, behind the work already there.  A copy to the host is complete on
+    // return; one to the device may be used by what is launched on the stream
+    // afterwards.  Allocates no host memory that could fail: the C entries above it
+    // have nothing to catch an exception with.
+    hipError_t run(const HostSpan *spans, int n, bool up, int device, hipStream_t stream) noexcept
     {
         size_t total = 0;
-        for (const HostSpan &s : spans) total += s.bytes;
-        std::vector<HostSpan> direct, sliced;
-        for (const HostSpan &s : spans) (total >= kLeast && ordinary(s.host) ? sliced : direct).push_back(s);
-        total = 0;
-        for (const HostSpan &s : sliced) total += s.bytes;
-        if (total < kLeast || !acquire()) {
-            direct.insert(direct.end(), sliced.begin(), sliced.end());
-            sliced.clear();
-        }
-        for (const HostSpan &s : direct) {
+        for (int k = 0; k < n; k++) total += spans[k].bytes;
+        Slices sliced;
+        if (total >= kLeast)
+            for (int k = 0; k < n; k++)
+                if (ordinary(spans[k].host)) sliced.add(spans[k]);
+        if (sliced.bytes < kLeast || !acquire()) sliced = Slices();
+        for (int k = 0; k < n; k++) {
+            const HostSpan &s = spans[k];
+            if (sliced.holds(s)) continue;
             const hipError_t e = up ? hipMemcpyAsync(s.dev, s.host, s.bytes, hipMemcpyHostToDevice, stream)
                                     : hipMemcpyAsync(s.host, s.dev, s.bytes, hipMemcpyDeviceToHost, stream);
             if (e != hipSuccess) return e;
         }
-        if (sliced.empty()) return up ? hipSuccess : hipStreamSynchronize(stream);
-        std::vector<HostSpan> slices;
-        for (const HostSpan &s : sliced)
-            for (size_t o = 0; o < s.bytes; o += kSlice)
-                slices.push_back({s.host + o, s.dev + o, std::min(kSlice, s.bytes - o)});
+        if (sliced.n == 0) return up ? hipSuccess : hipStreamSynchronize(stream);
         std::atomic<size_t> next{0};
         std::atomic<int> status{hipSuccess};
         auto work = [&](int w) {
             int e = hipSetDevice(device);
-            if (e == hipSuccess) e = up ? send(slices, next, status, w, stream) : receive(slices, next, status, w, stream);
+            if (e == hipSuccess) e = up ? send(sliced, next, status, w, stream) : receive(sliced, next, status, w, stream);
             if (e != hipSuccess) status = e;
         };
         std::thread helpers[kThreads - 1];
@@ -88,6 +84,35 @@ public:
     }
 
 private:
+    // Spans cut into slices, each span from its start.
+    struct Slices {
+        HostSpan span[kMostSpans];
+        int n = 0;
+        size_t bytes = 0, count = 0;
+
+        static size_t of(const HostSpan &s) { return (s.bytes + kSlice - 1) / kSlice; }
+        void add(const HostSpan &s)
+        {
+            span[n++] = s;
+            bytes += s.bytes;
+            count += of(s);
+        }
+        bool holds(const HostSpan &s) const
+        {
+            for (int k = 0; k < n; k++)
+                if (span[k].dev == s.dev) return true;
+            return false;
+        }
+        size_t size() const { return count; }
+        HostSpan operator[](size_t i) const
+        {
+            int k = 0;
+            for (; i >= of(span[k]); k++) i -= of(span[k]);
+            const size_t o = i * kSlice;
+            return {span[k].host + o, span[k].dev + o, std::min(kSlice, span[k].bytes - o)};
+        }
+    };
+
     // Memory that the runtime knows nothing of: from malloc, the stack, a mapped file.
     static bool ordinary(const void *p)
     {
@@ -100,7 +125,7 @@ private:
     char *slice(int w, int k) { return pinned_ + (size_t)(2 * w + k) * kSlice; }
     hipEvent_t event(int w, int k) { return events_[2 * w + k]; }
 
-    int send(const std::vector<HostSpan> &slices, std::atomic<size_t> &next, std::atomic<int> &status, int w,
+    int send(const Slices &slices, std::atomic<size_t> &next, std::atomic<int> &status, int w,
              hipStream_t stream)
     {
         bool busy[2] = {false, false};
@@ -109,29 +134,29 @@ private:
             if (i >= slices.size() || status != hipSuccess) return hipSuccess;
             hipError_t e = busy[k] ? hipEventSynchronize(event(w, k)) : hipSuccess;
             if (e != hipSuccess) return e;
-            std::memcpy(slice(w, k), slices[i].host, slices[i].bytes);
-            if ((e = hipMemcpyAsync(slices[i].dev, slice(w, k), slices[i].bytes, hipMemcpyHostToDevice, stream)) != hipSuccess)
-                return e;
+            const HostSpan s = slices[i];
+            std::memcpy(slice(w, k), s.host, s.bytes);
+            if ((e = hipMemcpyAsync(s.dev, slice(w, k), s.bytes, hipMemcpyHostToDevice, stream)) != hipSuccess) return e;
             if ((e = hipEventRecord(event(w, k), stream)) != hipSuccess) return e;
             busy[k] = true;
         }
     }
 
-    int receive(const std::vector<HostSpan> &slices, std::atomic<size_t> &next, std::atomic<int> &status, int w,
+    int receive(const Slices &slices, std::atomic<size_t> &next, std::atomic<int> &status, int w,
                 hipStream_t stream)
     {
         size_t held[2];
         auto issue = [&](int k) -> hipError_t {
             const size_t i = held[k] = next++;
             if (i >= slices.size()) return hipSuccess;
-            const hipError_t e =
-                hipMemcpyAsync(slice(w, k), slices[i].dev, slices[i].bytes, hipMemcpyDeviceToHost, stream);
+            const HostSpan s = slices[i];
+            const hipError_t e = hipMemcpyAsync(slice(w, k), s.dev, s.bytes, hipMemcpyDeviceToHost, stream);
             return e != hipSuccess ? e : hipEventRecord(event(w, k), stream);
         };
         hipError_t e = issue(0);
         if (e == hipSuccess) e = issue(1);
         for (int k = 0; e == hipSuccess && held[k] < slices.size() && status == hipSuccess; k ^= 1) {
-            const HostSpan &s = slices[held[k]];
+            const HostSpan s = slices[held[k]];
             if ((e = hipEventSynchronize(event(w, k))) != hipSuccess) break;
             std::memcpy(s.host, slice(w, k), s.bytes);
             e = issue(k);

@@ -1,6 +1,7 @@
 """Host arrays of 16 MiB and more travel through pinned slices, unless the runtime knows their memory (pinned,
 managed): that it copies by itself, at the link's full rate.  Checked on the CPU against a host stand-in of the
-runtime calls, up and down, with arrays of each kind, of two kinds in one call, and without slices."""
+runtime calls, up and down, with arrays of each kind, of two kinds in one call, without slices, and with every host
+allocation failing."""
 import os
 import shutil
 import subprocess
@@ -18,4 +19,4 @@ def test_routes(tmp_path):
                     os.path.join(TESTS, "transfer_check.cpp"), "-o", exe], check=True, capture_output=True)
     out = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stdout + out.stderr
-    assert out.stdout.count("ok ") == 16
+    assert out.stdout.count("ok ") == 32

@@ -1,13 +1,26 @@
 // Host-side check of the copies of glac_amd/csrc/transfer.hpp, built by tests/test_transfer_route.py against
 // tests/host_hip: which arrays travel through the pinned slices and which the runtime copies by itself, and that
-// the bytes arrive.  Prints "ok <case>" per case, exits non-zero on the first violation.
+// the bytes arrive, also when no memory is left on the host (a C entry cannot pass an exception on).  Prints "ok <case>"
+// per case, exits non-zero on the first violation.
 #include <cstdio>
 #include <cstdlib>
+#include <new>
 #include <vector>
 
 #include "../glac_amd/csrc/transfer.hpp"
 
 using namespace glacx;
+
+// While `no_memory` is set every allocation fails.
+static bool no_memory = false;
+void *operator new(std::size_t n)
+{
+    void *p = no_memory ? nullptr : std::malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, std::size_t) noexcept { std::free(p); }
 
 #define REQUIRE(cond)                                                          \
     do {                                                                       \
@@ -28,7 +41,7 @@ struct Case {
     unsigned sliced;               // bit k: array k goes through the slices
 };
 
-static void check(const Case &c, bool up)
+static void check(const Case &c, bool up, bool starved)
 {
     const char *name = c.name;
     std::vector<char> host[kArrays], dev((size_t)kArrays * c.bytes);
@@ -52,7 +65,16 @@ static void check(const Case &c, bool up)
     }
     {
         Transfer t;
-        REQUIRE(t.run(spans, up, 0, nullptr) == hipSuccess);
+        no_memory = starved;
+        bool thrown = false;
+        hipError_t e = hipSuccess;
+        try {
+            e = t.run(spans.data(), (int)spans.size(), up, 0, nullptr);
+        } catch (...) {
+            thrown = true;
+        }
+        no_memory = false;
+        REQUIRE(!thrown && e == hipSuccess);
         for (int k = 0; k < kArrays; k++) {
             size_t direct = 0;
             for (int i = 0; i < rt.n; i++) {
@@ -65,7 +87,7 @@ static void check(const Case &c, bool up)
         REQUIRE(hipGetLastError() == hipSuccess);
     }
     for (int k = 0; k < kArrays; k++) REQUIRE(std::memcmp(host[k].data(), dev.data() + k * c.bytes, c.bytes) == 0);
-    std::printf("ok %s %s\n", name, up ? "up" : "down");
+    std::printf("ok %s %s%s\n", name, up ? "up" : "down", starved ? " starved" : "");
 }
 
 int main()
@@ -82,6 +104,7 @@ int main()
         {"mixed", large, 0x5, hipMemoryTypeHost, false, false, 0xA},
     };
     for (const Case &c : cases)
-        for (const bool up : {true, false}) check(c, up);
+        for (const bool up : {true, false})
+            for (const bool starved : {false, true}) check(c, up, starved);
     return 0;
 }
