@@ -45,13 +45,11 @@ template <class T, int R> __device__ __forceinline__ M3<T> reunitarized(const M3
 // fourth pays.  Microseconds per sub-sweep by blocks per CU, three | four (four
 // with compressed links take 116 registers, which they get with no bound on
 // WAVES; bounded they are scheduled into 104 and 2 % slower):
-//     blocks per CU      4     5     6     8    10    12    16    20    40    81
-//     compressed FP32   43    49    56    70    84   103   143   178   347   693
-//                       46    52    59    73    87   105   142   176   340   678
-//     FP32              51    59    67    86   110   133   180   225   439   862
-//                       58    64    72    92   115   137   179   222   434   848
-// (FP32 with four at up to 12: 118 registers and the block's sum at the end, as
-// they were; now 127 and no sum.)
+//     blocks per CU    4.5   5.1     6     8    10    12    16    20    40    81
+//     compressed FP32 48.1  54.2  55.9  68.9  82.6   102   140   177   350   707
+//                     51.0  56.1  59.6  72.3  86.3   104   141   175   343   692
+//     FP32            56.3  62.5  66.9  85.4   110   134   183   227   445   894
+//                     58.8  65.0  68.8  86.0   109   133   180   224   444   880
 template <class T, int R, int WAVES>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(1, WAVES))) void metropolis_kernel(
     typename vec2<T>::type *__restrict__ f, Geom g, int mu, int parity, MetroParams prm,
@@ -350,7 +348,7 @@ void launch_metropolis(void *f, const Geom &g, int mu, int parity, const MetroPa
             metropolis_small_kernel<T, R, 3, 5><<<groups, 64 * 8, 0, s>>>(links, g, mu, parity, p, count);
         else if (groups <= 768)
             metropolis_small_kernel<T, R, 1, 1><<<groups, 64 * 2, 0, s>>>(links, g, mu, parity, p, count);
-        else if (blocks <= 3072)  // the table at metropolis_kernel
+        else if (blocks <= (R == 2 ? 3072 : 2048))  // the table at metropolis_kernel
             metropolis_kernel<T, R, 3><<<blocks, kBlock, 0, s>>>(links, g, mu, parity, p, count);
         else
             metropolis_kernel<T, R, R == 2 ? 8 : 4><<<blocks, kBlock, 0, s>>>(links, g, mu, parity, p, count);

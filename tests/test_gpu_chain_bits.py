@@ -4,7 +4,8 @@ slices; after one sweep (eight sub-sweeps, each reading links up to one slice aw
 shorter one's ends must be equal.  The pairs lie on the two sides of every line between the kernels:
 
 FP32   256 | 257 groups of 64 links of a direction and parity (3 + 5 | 1 + 1 wavefronts per group), 768 | 769 groups
-       (| one wavefront per group, three per SIMD), 3072 | 3073 blocks of four groups (| more per SIMD)
+       (| one wavefront per group, three per SIMD), 2048 | 2049 blocks of four groups, with two stored rows 3072 | 3073
+       (| more per SIMD)
 FP64   512 | 513 groups
 learned  1536 | 1537 blocks (FP32)"""
 import numpy as np
@@ -52,7 +53,7 @@ def test_small_lattices(space, short, long, prec, hits, reunit):
 
 
 @pytest.mark.parametrize("prec", ["fp32", "fp32c"])
-def test_across_3072_blocks(prec):
+def test_across_2048_and_3072_blocks(prec):
     compare((16, 16, 16), 32, 392, prec, 4)  # 256 | 3136 blocks
 
 
