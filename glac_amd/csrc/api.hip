@@ -231,8 +231,8 @@ template <class T, int R> int run_plaquette_partials(glacx_ctx *c, const void *f
 }
 
 // Measurements whose partials a flow (or a chain, its plaquettes') holds before it
-// sums them: all of them, or as many as `limit` doubles take (kFlowPartials: 32 MiB of a context, which is
-// 64 measurements at 32^4 and six at 48^3 x 96).
+// sums them: all of them, or as many as `limit` doubles take (kFlowPartials: 32 MiB
+// of a context, which is 63 measurements at 32^4 and six at 48^3 x 96).
 constexpr size_t kFlowPartials = (size_t)4 << 20;
 int flow_slots(size_t per, int n_steps, size_t limit)
 {
@@ -284,7 +284,8 @@ int run_flow(glacx_ctx *c, int field, int n_steps, double eps, double *results, 
             std::swap(c->field[field], c->work);
         }
         if (results && (slot == slots - 1 || i == n_steps)) {
-            launch_measure_finish(partials, c->geom, results + row * (size_t)(i - slot), super, slot + 1, row, c->stream);
+            launch_measure_finish(partials, c->geom, results + row * (size_t)(i - slot), super, slot + 1, row,
+                                  c->stream);
             CHECK_LAUNCH(c);
         }
     }
@@ -1110,7 +1111,8 @@ int glacx_train_grad(glacx_ctx *c, const float *samples, int n, const float *z, 
             break;
         }
         launch_train_step(dsmp, (size_t)n, (size_t)n, n, draws, 0, 0, beta, c->params, c->mean_std, dz, c->inter,
-                          c->partials, c->partials + groups, c->grad, c->adam_m, c->adam_v, 0.f, 0, c->params_bf16, c->stream);
+                          c->partials, c->partials + groups, c->grad, c->adam_m, c->adam_v, 0.f, 0, c->params_bf16,
+                          c->stream);
         if (hipGetLastError() != hipSuccess) {
             rc = fail(c, GLACX_E_HIP, "train_grad: launch failed");
             break;

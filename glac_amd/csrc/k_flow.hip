@@ -203,9 +203,9 @@ template <class T> __device__ __forceinline__ FlowMeasLds<T> &flow_meas_lds()
 // The end of a stage for one link: RK3 combination of the force z with the
 // accumulator, exp, product with the link u, and in FP32 the projection.
 template <class T, int R, int STAGE, unsigned STREAM>
-__device__ __forceinline__ void finish_link(typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc, const Geom &g,
-                                            int mu, int idx, const M3<T> &u, const su3alg<T> &z, const su3alg<T> &cacc,
-                                            T cz, T ca)
+__device__ __forceinline__ void finish_link(typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc,
+                                            const Geom &g, int mu, int idx, const M3<T> &u, const su3alg<T> &z,
+                                            const su3alg<T> &cacc, T cz, T ca)
 {
     su3alg<T> y;
     if constexpr (STAGE == 0) {
@@ -298,10 +298,11 @@ constexpr int kFewBlocks = 768;
 
 template <class T, int R, int STAGE, bool MEAS, unsigned STREAM, bool FEW = false>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP64_FLOW_WAVES) void flow_stage_kernel(
-    const typename vec2<T>::type *__restrict__ win, typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc, Geom g,
-    T cz, T ca, double *__restrict__ meas)
+    const typename vec2<T>::type *__restrict__ win, typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc,
+    Geom g, T cz, T ca, double *__restrict__ meas)
 {
-    static_assert(!MEAS || (STAGE == 0 && sizeof(T) == 4), "the measurement is fused into stage 0 only, FP64 has its own");
+    static_assert(!MEAS || (STAGE == 0 && sizeof(T) == 4),
+                  "the measurement is fused into stage 0 only, FP64 has its own");
     __shared__ FlowLds<T> sh;
     const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // one direction per wavefront
     const int lane = threadIdx.x & 63;
@@ -374,7 +375,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 ? (MEAS ? 3 : 4) : GLACX_FP6
             // that the upper links both of them gather come from L1 the second time
             // (24^3 x 48 440 -> 435 us).  FP32 sums the terms in another order, which
             // its results show in their last digits.
-            const int nu = MEAS ? (int)((kPhaseNu >> (4 * e)) & 0xF) : (sizeof(T) == 8 ? mu ^ (k + 1) : (mu + k + 1) & 3);
+            const int nu = MEAS ? (int)((kPhaseNu >> (4 * e)) & 0xF)
+                                : (sizeof(T) == 8 ? mu ^ (k + 1) : (mu + k + 1) & 3);
             const DirView<T> vnu = dir_view<T>(win, g, nu);
             const int ipn = nbr[0][nu][lane], imn = nbr[1][nu][lane];
             const int ipmmn = site_step(g, xpm, nu, -1).idx;
@@ -714,10 +716,9 @@ template <class T, class V2> __device__ __forceinline__ M3<T> wide_get(const V2 
 }
 
 template <class T, int R>
-__global__ __launch_bounds__(3 * kBlock, 3) void flow_measure_wide_kernel(const typename vec2<T>::type *__restrict__ win,
-                                                                        typename vec2<T>::type *__restrict__ wout,
-                                                                        T *__restrict__ acc, Geom g, T cz,
-                                                                        double *__restrict__ meas)
+__global__ __launch_bounds__(3 * kBlock, 3) void flow_measure_wide_kernel(
+    const typename vec2<T>::type *__restrict__ win, typename vec2<T>::type *__restrict__ wout, T *__restrict__ acc,
+    Geom g, T cz, double *__restrict__ meas)
 {
     __shared__ __align__(16) WideLds<T, R> lds;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), mu = wave & 3, k = wave >> 2;

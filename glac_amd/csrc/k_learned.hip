@@ -457,8 +457,8 @@ __global__ __launch_bounds__(64) void update_kernel(const float *__restrict__ in
 #pragma unroll
         for (int k = 0; k < kSet; k++) {
             const size_t g = min(g0 + k, groups - 1);
-            const __amdgpu_buffer_rsrc_t r =
-                __builtin_amdgcn_make_buffer_rsrc((void *)(inter + g * kCols * kTrainSites), (short)0, kStep, kBufferFlags);
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                (void *)(inter + g * kCols * kTrainSites), (short)0, kStep, kBufferFlags);
             a[which][k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, oa, 0, 0));
             b[which][k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, ob, 0, 0));
         }
@@ -516,7 +516,8 @@ __global__ __launch_bounds__(kBlock) void to_bf16_kernel(const float *__restrict
 //                     62.0   69.9   70.6   79.5   99.4   145   196
 //                     62.2   71.7   73.2   81.5   99.3   142   190
 template <class T, int R, int WAVES>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? WAVES : 1, sizeof(T) == 4 ? WAVES : 2)))
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? WAVES : 1, sizeof(T) == 4 ? WAVES : 2)))
 void metropolis_learned_kernel(typename vec2<T>::type *__restrict__ f, Geom g, int mu, int parity, MetroParams prm,
                                const unsigned short *__restrict__ wbf16, const float *__restrict__ mean_std,
                                unsigned long long *__restrict__ count)
@@ -676,7 +677,8 @@ void launch_metropolis_learned(void *f, const Geom &g, int mu, int parity, const
     auto *links = (typename vec2<T>::type *)f;
     if constexpr (sizeof(T) == 4) {
         if (blocks <= 6 * 256) {  // the table at metropolis_learned_kernel; 256 CUs
-            metropolis_learned_kernel<T, R, 3><<<blocks, kBlock, 0, s>>>(links, g, mu, parity, p, wbf16, mean_std, count);
+            metropolis_learned_kernel<T, R, 3>
+                <<<blocks, kBlock, 0, s>>>(links, g, mu, parity, p, wbf16, mean_std, count);
             return;
         }
     }

@@ -300,8 +300,8 @@ __device__ __forceinline__ void finish_row(const double *__restrict__ slice, con
 // Few chunks: one block per measurement, a wavefront per time slice.
 constexpr int kRowWaves = 16, kRowSlices = 512;  // a context's largest extent is 512
 constexpr int kRowChunks = 2048;
-__global__ __launch_bounds__(64 * kRowWaves) void measure_row_kernel(const double *__restrict__ partials, Geom g, int cps,
-                                                                     int super, size_t stride, size_t pitch,
+__global__ __launch_bounds__(64 * kRowWaves) void measure_row_kernel(const double *__restrict__ partials, Geom g,
+                                                                     int cps, int super, size_t stride, size_t pitch,
                                                                      double *__restrict__ out)
 {
     __shared__ double slice[kMeasAcc * kRowSlices];
@@ -346,8 +346,9 @@ __global__ __launch_bounds__(kBlock) void measure_slice_kernel(double *__restric
 }
 
 // ... then one wavefront per measurement.
-__global__ __launch_bounds__(64) void measure_finish_kernel(const double *__restrict__ partials, Geom g, int cps, int super,
-                                                            size_t stride, size_t pitch, double *__restrict__ out)
+__global__ __launch_bounds__(64) void measure_finish_kernel(const double *__restrict__ partials, Geom g, int cps,
+                                                            int super, size_t stride, size_t pitch,
+                                                            double *__restrict__ out)
 {
     finish_row(partials + blockIdx.x * stride + (size_t)kMeasAcc * g.n[3] * cps, g, super, threadIdx.x,
                out + blockIdx.x * pitch);
@@ -425,8 +426,8 @@ __global__ __launch_bounds__(kMeasSites *kMeasWaves) void plaquette_kernel(const
 }
 
 constexpr int kFinishBlock = 1024;
-__global__ __launch_bounds__(kFinishBlock) void plaquette_finish_kernel(const double *__restrict__ partials, int n, Geom g,
-                                                                        double *__restrict__ out)
+__global__ __launch_bounds__(kFinishBlock) void plaquette_finish_kernel(const double *__restrict__ partials, int n,
+                                                                        Geom g, double *__restrict__ out)
 {
     double acc[1] = {0.0};
 #pragma unroll 8

@@ -171,8 +171,9 @@ __device__ __forceinline__ StapleTerm<T, R> staple_term(const typename vec2<T>::
 }
 // a += the two terms, as staple() adds them
 template <class T, int R>
-__device__ __forceinline__ void add_term(M3<T> &a, const StapleTerm<T, R> &t, const typename vec2<T>::type *__restrict__ f,
-                                         const Geom &g, const Site &x, int nu)
+__device__ __forceinline__ void add_term(M3<T> &a, const StapleTerm<T, R> &t,
+                                         const typename vec2<T>::type *__restrict__ f, const Geom &g, const Site &x,
+                                         int nu)
 {
     if constexpr (R == 2) {
         add_to(a, t.up);

@@ -75,8 +75,7 @@ constexpr int kMeasAcc = 4;
 // `rows` measurements (measure_partials_count(g) doubles of partials each, side
 // by side) into rows of out, `pitch` doubles apart: {plaq, E_raw, Q, Q(t)...},
 // or with `super` (GLAC's SuperSampler) {plaq, E_raw, Q, W, Q(t)..., W(t)...}.
-// mode: 0 plain,
-// 1 SuperSampler (Weinberg), 2 plain plus per-site densities into
+// mode: 0 plain, 1 SuperSampler (Weinberg), 2 plain plus per-site densities into
 // density[0..V) (charge) and density[V..2V) (action), GLAC site order.
 int measure_partials_count(const Geom &g);
 template <class T, int R>
@@ -89,17 +88,17 @@ template <class T, int R> void launch_plaquette(const void *f, const Geom &g, do
 void launch_plaquette_finish(const double *partials, int nparts, const Geom &g, double *out, int rows, hipStream_t s);
 
 // One RK3 stage (0, 1, 2): win -> wout, accumulator read/written in acc.
-// With `meas` (stage 0 only, FP32 links, flow_measure_fusable(g)) the stage
-// also writes the clover-measurement partials of win into meas, in the layout
-// launch_measure_finish reads.
+// With `meas` (stage 0 only, flow_measure_fusable(g)) the stage also writes the
+// clover-measurement partials of win into meas, in the layout launch_measure_finish
+// reads.
 template <class T, int R>
 void launch_flow_stage(const void *win, void *wout, void *acc, const Geom &g, int stage, double eps, double *meas,
                        hipStream_t s);
 bool flow_measure_fusable(const Geom &g);
 
-// Accepted hits of a sweep are counted in kCountSlots slots, block b's in slot
-// b % kCountSlots: on one address the blocks of a small lattice, which end
-// together, queue for 5 of their 18 us (512 blocks).  launch_count_sum adds up
+// Accepted hits of a sweep are counted in kCountSlots slots, wavefront w's (or block
+// w's, in small lattices) in slot w % kCountSlots: on one address the blocks of a small
+// lattice, which end together, queue for 5 of their 18 us (512 blocks).  launch_count_sum adds up
 // `sweeps` sweeps' slots and leaves them cleared.
 constexpr int kCountSlots = 256;
 __device__ __forceinline__ int count_slot(unsigned block) { return (int)(block & (kCountSlots - 1)); }

@@ -387,12 +387,15 @@ template <bool STREAM> constexpr int store_policy() { return STREAM ? 2 : 0; }
 template <bool STREAM> __device__ __forceinline__ void buf_store(const DirView<float> &d, unsigned off, int k, float2 z)
 {
     using U2 = unsigned int __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, z), d.r, off, k * d.plane_bytes, store_policy<STREAM>());
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, z), d.r, off, k * d.plane_bytes,
+                                          store_policy<STREAM>());
 }
-template <bool STREAM> __device__ __forceinline__ void buf_store(const DirView<double> &d, unsigned off, int k, double2 z)
+template <bool STREAM>
+__device__ __forceinline__ void buf_store(const DirView<double> &d, unsigned off, int k, double2 z)
 {
     using U4 = unsigned int __attribute__((ext_vector_type(4)));
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, z), d.r, off + k * kTileRun, 0, store_policy<STREAM>());
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, z), d.r, off + k * kTileRun, 0,
+                                           store_policy<STREAM>());
 }
 
 // Third row of an SU(3) matrix from its first two.

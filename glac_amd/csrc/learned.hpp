@@ -188,16 +188,18 @@ __device__ __forceinline__ bool mlp_forward_mfma(const MlpImage &im, const float
         }
 #pragma unroll
         for (int m = 0; m < 2; m++) {
-            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w2[16 * m + row][mlp_col(row, 4 * grp)]), a1[0],
-                                                                lds_bias(&im.b2[16 * m + 4 * grp]), 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w2[16 * m + row][mlp_col(row, 16 + 4 * grp)]), a1[1], d, 0, 0, 0);
+            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w2[16 * m + row][mlp_col(row, 4 * grp)]),
+                                                                a1[0], lds_bias(&im.b2[16 * m + 4 * grp]), 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w2[16 * m + row][mlp_col(row, 16 + 4 * grp)]),
+                                                          a1[1], d, 0, 0, 0);
             a2[m] = lrelu_bf16(d);
         }
 #pragma unroll
         for (int m = 0; m < 3; m++) {
-            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w3[16 * m + row][mlp_col(row, 4 * grp)]), a2[0],
-                                                                lds_bias(&im.b3[16 * m + 4 * grp]), 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w3[16 * m + row][mlp_col(row, 16 + 4 * grp)]), a2[1], d, 0, 0, 0);
+            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w3[16 * m + row][mlp_col(row, 4 * grp)]),
+                                                                a2[0], lds_bias(&im.b3[16 * m + 4 * grp]), 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds_frag(&im.w3[16 * m + row][mlp_col(row, 16 + 4 * grp)]),
+                                                          a2[1], d, 0, 0, 0);
             const int r0 = 16 * m + 4 * grp;
             if (m < 2) {
                 *reinterpret_cast<f32x4 *>(obuf + mlp_out(16 * nt + row, r0)) = d;

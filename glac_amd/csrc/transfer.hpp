@@ -66,7 +66,8 @@ public:
         std::atomic<int> status{hipSuccess};
         auto work = [&](int w) {
             int e = hipSetDevice(device);
-            if (e == hipSuccess) e = up ? send(sliced, next, status, w, stream) : receive(sliced, next, status, w, stream);
+            if (e == hipSuccess)
+                e = up ? send(sliced, next, status, w, stream) : receive(sliced, next, status, w, stream);
             if (e != hipSuccess) status = e;
         };
         std::thread helpers[kThreads - 1];
@@ -136,7 +137,8 @@ private:
             if (e != hipSuccess) return e;
             const HostSpan s = slices[i];
             std::memcpy(slice(w, k), s.host, s.bytes);
-            if ((e = hipMemcpyAsync(s.dev, slice(w, k), s.bytes, hipMemcpyHostToDevice, stream)) != hipSuccess) return e;
+            e = hipMemcpyAsync(s.dev, slice(w, k), s.bytes, hipMemcpyHostToDevice, stream);
+            if (e != hipSuccess) return e;
             if ((e = hipEventRecord(event(w, k), stream)) != hipSuccess) return e;
             busy[k] = true;
         }

@@ -40,7 +40,10 @@ enum glacx_precision {
     GLACX_FP32_COMPRESSED = 2 /* as GLACX_FP32_LINKS, but only the first two rows
                                  of each link are stored; the third is rebuilt
                                  as conj(row0 x row1).  SU(3) links only:
-                                 uploads and loads of other links fail */
+                                 uploads and loads of links that deviate by
+                                 1e-6 or more fail.  What is not a number
+                                 deviates by nothing: a link with NaN entries
+                                 is taken, and spreads */
 };
 
 enum glacx_field { GLACX_FIELD_MAIN = 0, GLACX_FIELD_FLOW = 1 };
@@ -61,7 +64,7 @@ enum glacx_kernel {
     GLACX_K_PLAQUETTE = 3,
     GLACX_K_METROPOLIS_LEARNED = 4,
     GLACX_K_TRAIN = 5,
-    GLACX_K_FLOW_STAGE_MEASURE = 6, /* stage 0 with the clover observables fused (FP32 flow with measurement) */
+    GLACX_K_FLOW_STAGE_MEASURE = 6, /* stage 0 with the clover observables fused (flow with measurement) */
     GLACX_K_COUNT = 7
 };
 

@@ -8,7 +8,12 @@
 
 enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2 };
 enum hipMemcpyKind { hipMemcpyHostToDevice = 1, hipMemcpyDeviceToHost = 2 };
-enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1, hipMemoryTypeDevice = 2, hipMemoryTypeManaged = 3 };
+enum hipMemoryType {
+    hipMemoryTypeUnregistered = 0,
+    hipMemoryTypeHost = 1,
+    hipMemoryTypeDevice = 2,
+    hipMemoryTypeManaged = 3
+};
 struct hipPointerAttribute_t {
     hipMemoryType type;
 };

@@ -13,7 +13,8 @@ N = (8, 8, 8, 8)
 FIGURES = {"waves": 1.0, "valu_per_wave": 2.0, "traffic_bytes": 3.0}
 
 
-@pytest.mark.parametrize("name, found", [("metropolis_kernel<float, 2, 3>", True), ("metropolis_kernel<float, 2, 8>", True),
+@pytest.mark.parametrize("name, found", [("metropolis_kernel<float, 2, 3>", True),
+                                         ("metropolis_kernel<float, 2, 8>", True),
                                          ("metropolis_small_kernel<float, 2, 3, 5>", True),
                                          ("metropolis_kernel<float, 3, 4>", False),
                                          ("metropolis_kernel<double, 3, 2>", False),

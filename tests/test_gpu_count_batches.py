@@ -16,7 +16,7 @@ def chain(L, proposal, sweeps, offset=0):
 
 
 @pytest.mark.parametrize("proposal", ["rst", "learned"])
-@pytest.mark.parametrize("sweeps", [1023, 1024, 1025, 2049, 5000])  # 4097 and more: sums in device memory
+@pytest.mark.parametrize("sweeps", [1024, 1025, 5000])  # 4097 and more: sums in device memory
 def test_counts_of_a_call_that_goes_round(sweeps, proposal):
     print(f"\n[gpu case] count batches, {sweeps} {proposal} sweeps", flush=True)
     with glacx.Lattice(N, glacx.FP64) as L:

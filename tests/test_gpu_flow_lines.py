@@ -15,8 +15,9 @@ glacx = pytest.importorskip("glac_amd")
 FEW = [(10, 12, 12, 10), (12, 12, 12, 10), (16, 16, 16, 12)]  # 15.8 and 19.0 MiB; 768 blocks
 MANY = [(6, 12, 32, 22),                                      # 792 blocks
         (2, 16, 40, 40), (64, 2, 20, 20), (6, 4, 46, 48), (24, 24, 8, 12), (12, 10, 22, 20), (10, 6, 30, 28)]
-CASES = ([(n, "FP64") for n in FEW + MANY] + [((16, 16, 14, 14), "FP32_LINKS"), ((16, 16, 14, 16), "FP32_LINKS"),
-                                              ((16, 16, 16, 18), "FP32_COMPRESSED"), ((16, 16, 18, 18), "FP32_COMPRESSED")])
+CASES = [(n, "FP64") for n in FEW + MANY]
+CASES += [((16, 16, 14, 14), "FP32_LINKS"), ((16, 16, 14, 16), "FP32_LINKS")]                # 27.6 and 31.5 MiB
+CASES += [((16, 16, 16, 18), "FP32_COMPRESSED"), ((16, 16, 18, 18), "FP32_COMPRESSED")]      # 27.0 and 30.4 MiB
 
 
 @pytest.mark.parametrize("n, prec", CASES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v)

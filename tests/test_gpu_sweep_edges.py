@@ -26,7 +26,8 @@ def tail_links(n, rest):
     of z and t holds the last entries, in (t, z, y, x / 2) order."""
     nx, ny, nz, nt = n
     bz, bt = (4 if nz % 4 == 0 else 2), (4 if nt % 4 == 0 else 2)
-    t, z, y, x = np.meshgrid(np.arange(nt - bt, nt), np.arange(nz - bz, nz), np.arange(ny), np.arange(nx), indexing="ij")
+    t, z, y, x = np.meshgrid(np.arange(nt - bt, nt), np.arange(nz - bz, nz), np.arange(ny), np.arange(nx),
+                             indexing="ij")
     site = (x + nx * (y + ny * (z + nz * t))).ravel()
     parity = ((x + y + z + t) & 1).ravel()
     mask = np.zeros(int(np.prod(n)), bool)

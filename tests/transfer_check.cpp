@@ -1,7 +1,7 @@
 // Host-side check of the copies of glac_amd/csrc/transfer.hpp, built by tests/test_transfer_route.py against
 // tests/host_hip: which arrays travel through the pinned slices and which the runtime copies by itself, and that
-// the bytes arrive, also when no memory is left on the host (a C entry cannot pass an exception on).  Prints "ok <case>"
-// per case, exits non-zero on the first violation.
+// the bytes arrive, also when no memory is left on the host (a C entry cannot pass an exception on).  Prints
+// "ok <case>" per case, exits non-zero on the first violation.
 #include <cstdio>
 #include <cstdlib>
 #include <new>
