@@ -503,8 +503,8 @@ __global__ __launch_bounds__(kBlock) void to_bf16_kernel(const float *__restrict
 }
 
 // ---- sampling with the learned proposal ----------------------------------------
-// What bounds it: the vector ALU (7500 instructions a wavefront, three quarters
-// of the time) and, beside it, LDS.  Against outputs and weights in plain rows
+// What bounds it: the vector ALU (7400 instructions a wavefront, at 32^4 nearly all
+// the time) and, beside it, LDS.  Against outputs and weights in plain rows
 // (a sixth of the time went to bank conflicts) and a parameter at a time into
 // LDS before the staple's loads: 24^3x48 79.5 -> 76.5 us a sub-sweep, 32^4 102 ->
 // 99, 32^3x8 43 -> 38.5.
