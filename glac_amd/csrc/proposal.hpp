@@ -42,15 +42,18 @@ __device__ __forceinline__ void su2_near_unity(const T r0, const T r1, const T r
     b = {x2, x1};
 }
 
-// The product v, whose sign is its user's business: put into the multiply, as the
-// compiler does otherwise, the signs cost the compressed sweep 2 to 4 % (32^4
-// 69.2 | 68.9 us with three wavefronts per SIMD, 74.1 | 72.3 with four; 32^3 x 64
-// 143.8 | 141.3; three stored rows 32^3 x 28 75.9 | 73.9).
-template <class T> __device__ __forceinline__ T held(T v)
+// a b - c d with c d rounded first, as a product and a fused multiply-add: the
+// compiler may not fuse what product() forms, so only a b is left to fuse.  Written as
+// fma(a, b, -(c d)) the sign goes into the multiply, which costs the compressed sweep
+// 2 to 4 % (32^4 69.2 | 68.9 us with three wavefronts per SIMD, 74.1 | 72.3 with four;
+// 32^3 x 64 143.8 | 141.3; three stored rows 32^3 x 28 75.9 | 73.9), and a product made
+// opaque by an empty asm up to 2 % with many hits (32^3 x 52, 23 hits, 198.8 | 195.0).
+template <class T> __device__ __forceinline__ T product(T a, T b)
 {
-    asm("" : "+v"(v));
-    return v;
+#pragma clang fp contract(off)
+    return a * b;
 }
+template <class T> __device__ __forceinline__ T cross(T a, T b, T c, T d) { return a * b - product(c, d); }
 
 // X = R S T with r in block (0,1), s in block (0,2), t in block (1,2), each
 // [[a, b], [-conj(b), conj(a)]] there.  Which product of a pair is rounded before
@@ -60,22 +63,22 @@ template <class T>
 __device__ __forceinline__ M3<T> rst_product(cpx<T> ra, cpx<T> rb, cpx<T> sa, cpx<T> sb, cpx<T> ta, cpx<T> tb)
 {
     // R_00 S_01 and R_10 S_01
-    const T pr = fma(ra.r, sb.r, -held(ra.i * sb.i)), pi = fma(ra.r, sb.i, ra.i * sb.r);
-    const T qr = fma(-rb.r, sb.r, -held(rb.i * sb.i)), qi = fma(rb.i, sb.r, -held(rb.r * sb.i));
+    const T pr = cross(ra.r, sb.r, ra.i, sb.i), pi = fma(ra.r, sb.i, ra.i * sb.r);
+    const T qr = cross(-rb.r, sb.r, rb.i, sb.i), qi = cross(rb.i, sb.r, rb.r, sb.i);
     M3<T> x;
-    x.e[0][0] = {fma(ra.r, sa.r, -held(ra.i * sa.i)), fma(ra.i, sa.r, ra.r * sa.i)};
-    x.e[0][1] = {fma(rb.r, ta.r, -held(rb.i * ta.i)) + fma(-tb.r, pr, -held(tb.i * pi)),
-                 fma(rb.i, ta.r, rb.r * ta.i) + fma(tb.i, pr, -held(tb.r * pi))};
-    x.e[0][2] = {fma(rb.r, tb.r, -held(rb.i * tb.i)) + fma(pr, ta.r, ta.i * pi),
-                 fma(rb.r, tb.i, rb.i * tb.r) + fma(pi, ta.r, -held(ta.i * pr))};
-    x.e[1][0] = {fma(-rb.r, sa.r, -held(rb.i * sa.i)), fma(rb.i, sa.r, -held(rb.r * sa.i))};
-    x.e[1][1] = {fma(ra.r, ta.r, ra.i * ta.i) + fma(-tb.r, qr, -held(tb.i * qi)),
-                 fma(ra.r, ta.i, -held(ra.i * ta.r)) + fma(tb.i, qr, -held(tb.r * qi))};
+    x.e[0][0] = {cross(ra.r, sa.r, ra.i, sa.i), fma(ra.i, sa.r, ra.r * sa.i)};
+    x.e[0][1] = {cross(rb.r, ta.r, rb.i, ta.i) + cross(-tb.r, pr, tb.i, pi),
+                 fma(rb.i, ta.r, rb.r * ta.i) + cross(tb.i, pr, tb.r, pi)};
+    x.e[0][2] = {cross(rb.r, tb.r, rb.i, tb.i) + fma(pr, ta.r, ta.i * pi),
+                 fma(rb.r, tb.i, rb.i * tb.r) + cross(pi, ta.r, ta.i, pr)};
+    x.e[1][0] = {cross(-rb.r, sa.r, rb.i, sa.i), cross(rb.i, sa.r, rb.r, sa.i)};
+    x.e[1][1] = {fma(ra.r, ta.r, ra.i * ta.i) + cross(-tb.r, qr, tb.i, qi),
+                 cross(ra.r, ta.i, ra.i, ta.r) + cross(tb.i, qr, tb.r, qi)};
     x.e[1][2] = {fma(ra.r, tb.r, ra.i * tb.i) + fma(qr, ta.r, ta.i * qi),
-                 fma(ra.r, tb.i, -held(ra.i * tb.r)) + fma(qi, ta.r, -held(ta.i * qr))};
+                 cross(ra.r, tb.i, ra.i, tb.r) + cross(qi, ta.r, ta.i, qr)};
     x.e[2][0] = {-sb.r, sb.i};
-    x.e[2][1] = {fma(sa.i, tb.i, -held(sa.r * tb.r)), fma(sa.r, tb.i, sa.i * tb.r)};
-    x.e[2][2] = {fma(sa.r, ta.r, -held(sa.i * ta.i)), fma(-sa.i, ta.r, -held(sa.r * ta.i))};
+    x.e[2][1] = {cross(sa.i, tb.i, sa.r, tb.r), fma(sa.r, tb.i, sa.i * tb.r)};
+    x.e[2][2] = {cross(sa.r, ta.r, sa.i, ta.i), cross(-sa.i, ta.r, sa.r, ta.i)};
     return x;
 }
 
